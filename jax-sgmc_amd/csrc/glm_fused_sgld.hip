@@ -1,0 +1,6 @@
+// The fused GLM step in mode SGMC_MODE_SGLD, every D class.
+#include "glm_fused.h"
+
+namespace sgmc {
+template void launch_fused<SGMC_MODE_SGLD>(int, int, hipStream_t, const FusedArgs&);
+}  // namespace sgmc
