@@ -401,6 +401,36 @@ int sgmc_resgld_swap(const sgmc_glm_chain* chains, int nchains, const sgmc_swap_
                      int npairs, float F, int swap_every, const int32_t* save_slot,
                      int table_len, const int32_t* iter, void* stream);
 
+/* ------------------------------------------------- launches of many tables ----
+ * One chain table's part of sgmc_glm_fused_run: the arguments of sgmc_glm_fused_step
+ * (advance_iter = 1), of sgmc_resgld_swap (pairs NULL without an exchange), and a HOST
+ * list of nops operations (kind, count), run in order on `stream`. */
+#define SGMC_OP_ITERATIONS 0 /* count iterations, one sgmc_glm_fused_step per evaluation */
+#define SGMC_OP_LOOP 1       /* count iterations in one sgmc_glm_fused_loop */
+#define SGMC_OP_SWAP 2       /* count launches of sgmc_resgld_swap */
+typedef struct sgmc_glm_run {
+  const sgmc_glm_chain* chains;
+  const int32_t* block_chain;
+  const float* inv_mass;
+  const float* sqrt_mass;
+  const float* eps_table;
+  const int32_t* save_slot;
+  int32_t* iter;
+  unsigned* done;
+  void* stream;
+  const sgmc_swap_pair* pairs;
+  const int32_t* ops;
+  int32_t nops;
+  int32_t nchains, nblocks, uniform_dclass, family, has_prior, mode, steps, table_len;
+  int32_t npairs, swap_every;
+  float sigma, prior_scale, pot_temperature, friction, alpha, lmbd, F;
+} sgmc_glm_run;
+/* Issues the operations of nruns tables (a HOST array), the tables taken in turn launch
+ * by launch, so that tables on different streams start together instead of one after the
+ * other's last launch is issued. Every table is checked before the first launch. No
+ * reference counterpart (solver.py:162-171 runs chains one by one). */
+int sgmc_glm_fused_run(const sgmc_glm_run* runs, int nruns);
+
 /* ------------------------------------------------------------ MLP (MFMA) ----
  * Bayesian MLP classifier x -> relu(x W1 + b1) -> relu(. W2 + b2) -> . W3 + b3 with a
  * 10-class softmax cross-entropy likelihood: the potential and its gradient

@@ -34,6 +34,9 @@ MODE_SGHMC = 2
 MODE_AMAGOLD = 3
 MODE_OBABO = 4
 MODE_SGGMC = 5
+OP_ITERATIONS = 0
+OP_LOOP = 1
+OP_SWAP = 2
 
 
 class GlmChain(ctypes.Structure):
@@ -46,6 +49,21 @@ class GlmChain(ctypes.Structure):
       ("n", c_int32), ("block_begin", c_int32), ("nblocks", c_int32), ("dclass", c_int32),
       ("temperature", c_float), ("energy", c_void_p), ("theta_old", c_void_p),
       ("mom_old", c_void_p),
+  ]
+
+
+class GlmRun(ctypes.Structure):
+  """Mirror of ``sgmc_glm_run`` (include/sgmc.h)."""
+  _fields_ = [
+      ("chains", c_void_p), ("block_chain", c_void_p), ("inv_mass", c_void_p),
+      ("sqrt_mass", c_void_p), ("eps_table", c_void_p), ("save_slot", c_void_p),
+      ("iter", c_void_p), ("done", c_void_p), ("stream", c_void_p),
+      ("pairs", c_void_p), ("ops", c_void_p), ("nops", c_int32), ("nchains", c_int32),
+      ("nblocks", c_int32), ("uniform_dclass", c_int32), ("family", c_int32),
+      ("has_prior", c_int32), ("mode", c_int32), ("steps", c_int32), ("table_len", c_int32),
+      ("npairs", c_int32), ("swap_every", c_int32), ("sigma", c_float),
+      ("prior_scale", c_float), ("pot_temperature", c_float), ("friction", c_float),
+      ("alpha", c_float), ("lmbd", c_float), ("F", c_float),
   ]
 
 
@@ -152,6 +170,7 @@ _SIGNATURES = {
                                     c_int, c_float, c_float, c_int, c_int, c_int, c_float,
                                     c_float, c_float, c_void_p, c_void_p, c_void_p, c_int,
                                     c_void_p, c_void_p, c_void_p, c_int, c_void_p]),
+    "sgmc_glm_fused_run": (c_int, [c_void_p, c_int]),
     "sgmc_resgld_swap": (c_int, [c_void_p, c_int, c_void_p, c_int, c_float, c_int, c_void_p,
                                  c_int, c_void_p, c_void_p]),
     "sgmc_mlp_full_potential": (c_int, [c_void_p, c_void_p, c_void_p]),

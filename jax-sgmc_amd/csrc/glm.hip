@@ -12,7 +12,9 @@
 // with the Gaussian prior log p = sum_j (log(2 pi s_p^2) + w_j^2 / s_p^2) / (-2).
 #include <math.h>
 
+#include <algorithm>
 #include <mutex>
+#include <vector>
 
 #include "glm_fused.h"
 
@@ -299,6 +301,89 @@ int scratch_of_current_device(void* stream, float** out) {
   return SGMC_OK;
 }
 
+// ---- launches of one chain table ----
+bool known_mode(int mode) { return mode >= SGMC_MODE_SGLD && mode <= SGMC_MODE_SGGMC; }
+
+// Launches of one iteration: OBABO modes take two per leapfrog step.
+int launches_of(const sgmc_glm_run& r) {
+  return (r.mode == SGMC_MODE_OBABO || r.mode == SGMC_MODE_SGGMC) ? 2 * r.steps : r.steps;
+}
+
+// Modes that run many iterations in one launch: no Metropolis-Hastings test in between.
+bool loop_mode(int mode) {
+  return mode == SGMC_MODE_SGLD || mode == SGMC_MODE_SGLD_RMS || mode == SGMC_MODE_SGHMC ||
+         mode == SGMC_MODE_OBABO;
+}
+
+int check_run(const char* who, const sgmc_glm_run& r) {
+  SGMC_REQUIRE(r.chains && r.eps_table && r.iter && r.done, SGMC_E_ARG, "%s: null pointer", who);
+  SGMC_REQUIRE(r.block_chain || (r.nchains > 0 && r.nblocks % r.nchains == 0), SGMC_E_ARG,
+               "%s: without a block map nblocks must be a multiple of nchains", who);
+  SGMC_REQUIRE(r.nchains >= 1 && r.nblocks >= r.nchains && r.table_len >= 1, SGMC_E_ARG,
+               "%s: bad sizes", who);
+  SGMC_REQUIRE(r.family == SGMC_LIK_LINEAR_GAUSSIAN || r.family == SGMC_LIK_LOGISTIC, SGMC_E_ARG,
+               "%s: unknown family %d", who, r.family);
+  SGMC_REQUIRE(known_mode(r.mode), SGMC_E_ARG, "%s: unknown mode %d", who, r.mode);
+  SGMC_REQUIRE(r.steps >= 1, SGMC_E_ARG, "%s: steps %d", who, r.steps);
+  SGMC_REQUIRE(r.pot_temperature != 0.0f, SGMC_E_ARG, "%s: temperature is zero", who);
+  return SGMC_OK;
+}
+
+// The kernel arguments of a table's first launch of an iteration.
+FusedArgs run_args(const sgmc_glm_run& r) {
+  FusedArgs a;
+  a.chains = r.chains;
+  a.block_chain = r.block_chain;
+  a.blocks_per_chain = r.block_chain ? 0 : r.nblocks / r.nchains;
+  a.eps_table = r.eps_table;
+  a.save_slot = r.save_slot;
+  a.iter = r.iter;
+  a.done = r.done;
+  a.inv_mass = r.inv_mass;
+  a.sqrt_mass = r.sqrt_mass;
+  a.table_len = r.table_len;
+  a.nchains = r.nchains;
+  a.step = 0;
+  a.steps = r.steps;
+  a.friction = r.friction;
+  a.four_friction = (float)(4.0 * (double)r.friction);
+  a.alpha = r.alpha;
+  a.lmbd = r.lmbd;
+  a.L = make_lik(r.family, r.sigma);
+  a.pr = make_prior(r.has_prior, r.prior_scale);
+  a.pot_temperature = r.pot_temperature;
+  a.advance = 1;
+  a.iter_offset = 0;
+  return a;
+}
+
+void launch_step(const sgmc_glm_run& r, const FusedArgs& a) {
+  const int dc = r.uniform_dclass, nb = r.nblocks;
+  hipStream_t s = as_stream(r.stream);
+  switch (r.mode) {
+    case SGMC_MODE_SGLD: launch_fused<SGMC_MODE_SGLD>(dc, nb, s, a); break;
+    case SGMC_MODE_SGLD_RMS: launch_fused<SGMC_MODE_SGLD_RMS>(dc, nb, s, a); break;
+    case SGMC_MODE_SGHMC: launch_fused<SGMC_MODE_SGHMC>(dc, nb, s, a); break;
+    case SGMC_MODE_AMAGOLD: launch_fused<SGMC_MODE_AMAGOLD>(dc, nb, s, a); break;
+    case SGMC_MODE_OBABO: launch_fused<SGMC_MODE_OBABO>(dc, nb, s, a); break;
+    default: launch_fused<SGMC_MODE_SGGMC>(dc, nb, s, a); break;
+  }
+}
+
+// `iterations` iterations of a table of one-block chains in one launch. Modes without
+// leapfrog steps take one evaluation per iteration whatever `steps` says.
+void launch_loop_mode(const sgmc_glm_run& r, int iterations, FusedArgs a) {
+  if (r.mode != SGMC_MODE_SGHMC && r.mode != SGMC_MODE_OBABO) a.steps = 1;
+  const int dc = r.uniform_dclass, n = r.nchains;
+  hipStream_t s = as_stream(r.stream);
+  switch (r.mode) {
+    case SGMC_MODE_SGLD: launch_loop<SGMC_MODE_SGLD>(dc, n, iterations, s, a); break;
+    case SGMC_MODE_SGLD_RMS: launch_loop<SGMC_MODE_SGLD_RMS>(dc, n, iterations, s, a); break;
+    case SGMC_MODE_SGHMC: launch_loop<SGMC_MODE_SGHMC>(dc, n, iterations, s, a); break;
+    default: launch_loop<SGMC_MODE_OBABO>(dc, n, iterations, s, a); break;
+  }
+}
+
 }  // namespace
 
 extern "C" {
@@ -474,59 +559,110 @@ int sgmc_glm_fused_step(const sgmc_glm_chain* chains, int nchains, const int32_t
                         const float* sqrt_mass, const float* eps_table, int table_len,
                         const int32_t* save_slot, int32_t* iter, unsigned* done,
                         int advance_iter, void* stream) {
-  SGMC_REQUIRE(chains && eps_table && iter && done, SGMC_E_ARG,
-               "sgmc_glm_fused_step: null pointer");
-  SGMC_REQUIRE(block_chain || (nchains > 0 && nblocks % nchains == 0), SGMC_E_ARG,
-               "sgmc_glm_fused_step: without a block map nblocks must be a multiple of "
-               "nchains");
-  SGMC_REQUIRE(nchains >= 1 && nblocks >= nchains && table_len >= 1, SGMC_E_ARG,
-               "sgmc_glm_fused_step: bad sizes");
-  SGMC_REQUIRE(family == SGMC_LIK_LINEAR_GAUSSIAN || family == SGMC_LIK_LOGISTIC, SGMC_E_ARG,
-               "sgmc_glm_fused_step: unknown family %d", family);
-  SGMC_REQUIRE(mode == SGMC_MODE_SGLD || mode == SGMC_MODE_SGLD_RMS ||
-               mode == SGMC_MODE_SGHMC || mode == SGMC_MODE_AMAGOLD ||
-               mode == SGMC_MODE_OBABO || mode == SGMC_MODE_SGGMC,
-               SGMC_E_ARG, "sgmc_glm_fused_step: unknown mode %d", mode);
-  const int launches =
-      (mode == SGMC_MODE_OBABO || mode == SGMC_MODE_SGGMC) ? 2 * steps : steps;
-  SGMC_REQUIRE(steps >= 1 && step >= 0 && step < launches, SGMC_E_ARG,
-               "sgmc_glm_fused_step: launch %d of %d", step, launches);
-  SGMC_REQUIRE(pot_temperature != 0.0f, SGMC_E_ARG, "sgmc_glm_fused_step: temperature is zero");
-  FusedArgs a;
-  a.chains = chains;
-  a.block_chain = block_chain;
-  a.blocks_per_chain = block_chain ? 0 : nblocks / nchains;
-  a.eps_table = eps_table;
-  a.save_slot = save_slot;
-  a.iter = iter;
-  a.done = done;
-  a.inv_mass = inv_mass;
-  a.sqrt_mass = sqrt_mass;
-  a.table_len = table_len;
-  a.nchains = nchains;
+  sgmc_glm_run r = {};
+  r.chains = chains;
+  r.block_chain = block_chain;
+  r.inv_mass = inv_mass;
+  r.sqrt_mass = sqrt_mass;
+  r.eps_table = eps_table;
+  r.save_slot = save_slot;
+  r.iter = iter;
+  r.done = done;
+  r.stream = stream;
+  r.nchains = nchains;
+  r.nblocks = nblocks;
+  r.uniform_dclass = uniform_dclass;
+  r.family = family;
+  r.has_prior = has_prior;
+  r.mode = mode;
+  r.steps = steps;
+  r.table_len = table_len;
+  r.sigma = sigma;
+  r.prior_scale = prior_scale;
+  r.pot_temperature = pot_temperature;
+  r.friction = friction;
+  r.alpha = alpha;
+  r.lmbd = lmbd;
+  const int rc = check_run("sgmc_glm_fused_step", r);
+  if (rc != SGMC_OK) return rc;
+  SGMC_REQUIRE(step >= 0 && step < launches_of(r), SGMC_E_ARG,
+               "sgmc_glm_fused_step: launch %d of %d", step, launches_of(r));
+  FusedArgs a = run_args(r);
   a.step = step;
-  a.steps = steps;
-  a.friction = friction;
-  a.four_friction = (float)(4.0 * (double)friction);
-  a.alpha = alpha;
-  a.lmbd = lmbd;
-  a.L = make_lik(family, sigma);
-  a.pr = make_prior(has_prior, prior_scale);
-  a.pot_temperature = pot_temperature;
   a.advance = advance_iter ? 1 : 0;
-  a.iter_offset = 0;
-  hipStream_t s = as_stream(stream);
-  switch (mode) {
-    case SGMC_MODE_SGLD: launch_fused<SGMC_MODE_SGLD>(uniform_dclass, nblocks, s, a); break;
-    case SGMC_MODE_SGLD_RMS:
-      launch_fused<SGMC_MODE_SGLD_RMS>(uniform_dclass, nblocks, s, a);
-      break;
-    case SGMC_MODE_SGHMC: launch_fused<SGMC_MODE_SGHMC>(uniform_dclass, nblocks, s, a); break;
-    case SGMC_MODE_AMAGOLD: launch_fused<SGMC_MODE_AMAGOLD>(uniform_dclass, nblocks, s, a); break;
-    case SGMC_MODE_OBABO: launch_fused<SGMC_MODE_OBABO>(uniform_dclass, nblocks, s, a); break;
-    default: launch_fused<SGMC_MODE_SGGMC>(uniform_dclass, nblocks, s, a); break;
-  }
+  launch_step(r, a);
   return check_launch("sgmc_glm_fused_step");
+}
+
+int sgmc_glm_fused_run(const sgmc_glm_run* runs, int nruns) {
+  SGMC_REQUIRE(runs && nruns >= 1, SGMC_E_ARG, "sgmc_glm_fused_run: no tables");
+  for (int k = 0; k < nruns; ++k) {
+    const sgmc_glm_run& r = runs[k];
+    const int rc = check_run("sgmc_glm_fused_run", r);
+    if (rc != SGMC_OK) return rc;
+    SGMC_REQUIRE(r.nops >= 0 && (r.ops || r.nops == 0), SGMC_E_ARG,
+                 "sgmc_glm_fused_run: no operations");
+    for (int i = 0; i < r.nops; ++i) {
+      const int op = r.ops[2 * i];
+      SGMC_REQUIRE(op >= SGMC_OP_ITERATIONS && op <= SGMC_OP_SWAP && r.ops[2 * i + 1] >= 0,
+                   SGMC_E_ARG, "sgmc_glm_fused_run: operation (%d, %d)", op, r.ops[2 * i + 1]);
+      SGMC_REQUIRE(op != SGMC_OP_LOOP || (loop_mode(r.mode) && r.nblocks == r.nchains),
+                   SGMC_E_ARG, "sgmc_glm_fused_run: a loop launch of mode %d, %d blocks for %d "
+                   "chains", r.mode, r.nblocks, r.nchains);
+      SGMC_REQUIRE(op != SGMC_OP_SWAP || (r.pairs && r.npairs >= 1 && r.nchains >= 2 &&
+                                          r.swap_every >= 1),
+                   SGMC_E_ARG, "sgmc_glm_fused_run: a swap launch without pairs");
+    }
+  }
+  // one launch per table and turn
+  struct Cursor {
+    int op = 0;
+    int64_t at = 0;  // launches of the operation issued so far
+  };
+  std::vector<Cursor> cur(nruns);
+  for (bool any = true; any;) {
+    any = false;
+    for (int k = 0; k < nruns; ++k) {
+      const sgmc_glm_run& r = runs[k];
+      Cursor& c = cur[k];
+      while (c.op < r.nops) {
+        const int count = r.ops[2 * c.op + 1];
+        const int64_t total = r.ops[2 * c.op] == SGMC_OP_ITERATIONS
+                                  ? (int64_t)count * launches_of(r)
+                                  : r.ops[2 * c.op] == SGMC_OP_LOOP ? (count > 0) : count;
+        if (c.at < total) break;
+        ++c.op;
+        c.at = 0;
+      }
+      if (c.op == r.nops) continue;
+      any = true;
+      int rc;
+      switch (r.ops[2 * c.op]) {
+        case SGMC_OP_ITERATIONS: {
+          FusedArgs a = run_args(r);
+          a.step = (int)(c.at % launches_of(r));
+          launch_step(r, a);
+          rc = check_launch("sgmc_glm_fused_run");
+          break;
+        }
+        case SGMC_OP_LOOP: {
+          FusedArgs a = run_args(r);
+          a.blocks_per_chain = 1;
+          a.block_chain = nullptr;
+          a.advance = -1;
+          launch_loop_mode(r, r.ops[2 * c.op + 1], a);
+          rc = check_launch("sgmc_glm_fused_run");
+          break;
+        }
+        default:
+          rc = sgmc_resgld_swap(r.chains, r.nchains, r.pairs, r.npairs, r.F, r.swap_every,
+                                r.save_slot, r.table_len, r.iter, r.stream);
+      }
+      if (rc != SGMC_OK) return rc;
+      ++c.at;
+    }
+  }
+  return SGMC_OK;
 }
 
 int sgmc_glm_fused_loop(const sgmc_glm_chain* chains, int nchains, int uniform_dclass,
@@ -541,49 +677,36 @@ int sgmc_glm_fused_loop(const sgmc_glm_chain* chains, int nchains, int uniform_d
                "sgmc_glm_fused_loop: bad sizes");
   SGMC_REQUIRE(family == SGMC_LIK_LINEAR_GAUSSIAN || family == SGMC_LIK_LOGISTIC, SGMC_E_ARG,
                "sgmc_glm_fused_loop: unknown family %d", family);
-  SGMC_REQUIRE(mode == SGMC_MODE_SGLD || mode == SGMC_MODE_SGLD_RMS ||
-                   mode == SGMC_MODE_SGHMC || mode == SGMC_MODE_OBABO,
-               SGMC_E_ARG, "sgmc_glm_fused_loop: mode %d needs a test between iterations",
+  SGMC_REQUIRE(loop_mode(mode), SGMC_E_ARG, "sgmc_glm_fused_loop: mode %d needs a test between iterations",
                mode);
   SGMC_REQUIRE(steps >= 1, SGMC_E_ARG, "sgmc_glm_fused_loop: steps %d", steps);
   SGMC_REQUIRE(pot_temperature != 0.0f, SGMC_E_ARG, "sgmc_glm_fused_loop: temperature is zero");
   if (iterations == 0) return SGMC_OK;
-  FusedArgs a;
-  a.chains = chains;
-  a.block_chain = nullptr;
-  a.blocks_per_chain = 1;
-  a.eps_table = eps_table;
-  a.save_slot = save_slot;
-  a.iter = iter;
-  a.done = done;
-  a.inv_mass = inv_mass;
-  a.sqrt_mass = sqrt_mass;
-  a.table_len = table_len;
-  a.nchains = nchains;
-  a.step = 0;
-  a.steps = (mode == SGMC_MODE_SGHMC || mode == SGMC_MODE_OBABO) ? steps : 1;
-  a.friction = friction;
-  a.four_friction = (float)(4.0 * (double)friction);
-  a.alpha = alpha;
-  a.lmbd = lmbd;
-  a.L = make_lik(family, sigma);
-  a.pr = make_prior(has_prior, prior_scale);
-  a.pot_temperature = pot_temperature;
+  sgmc_glm_run r = {};
+  r.chains = chains;
+  r.inv_mass = inv_mass;
+  r.sqrt_mass = sqrt_mass;
+  r.eps_table = eps_table;
+  r.save_slot = save_slot;
+  r.iter = iter;
+  r.done = done;
+  r.stream = stream;
+  r.nchains = r.nblocks = nchains;
+  r.uniform_dclass = uniform_dclass;
+  r.family = family;
+  r.has_prior = has_prior;
+  r.mode = mode;
+  r.steps = steps;
+  r.table_len = table_len;
+  r.sigma = sigma;
+  r.prior_scale = prior_scale;
+  r.pot_temperature = pot_temperature;
+  r.friction = friction;
+  r.alpha = alpha;
+  r.lmbd = lmbd;
+  FusedArgs a = run_args(r);
   a.advance = -1;
-  a.iter_offset = 0;
-  hipStream_t s = as_stream(stream);
-  switch (mode) {
-    case SGMC_MODE_SGLD:
-      launch_loop<SGMC_MODE_SGLD>(uniform_dclass, nchains, iterations, s, a);
-      break;
-    case SGMC_MODE_SGLD_RMS:
-      launch_loop<SGMC_MODE_SGLD_RMS>(uniform_dclass, nchains, iterations, s, a);
-      break;
-    case SGMC_MODE_SGHMC:
-      launch_loop<SGMC_MODE_SGHMC>(uniform_dclass, nchains, iterations, s, a);
-      break;
-    default: launch_loop<SGMC_MODE_OBABO>(uniform_dclass, nchains, iterations, s, a); break;
-  }
+  launch_loop_mode(r, iterations, a);
   return check_launch("sgmc_glm_fused_loop");
 }
 
