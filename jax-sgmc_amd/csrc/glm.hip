@@ -48,7 +48,6 @@ __global__ void __launch_bounds__(kNT) glm_potential_kernel(PotArgs a) {
   __shared__ float lds_lik[kLdsRows];
   __shared__ int flag;
   float4 th[CPL];
-  load_theta<LPR, CPL>(a.theta, a.D, th);
   float4 acc[CPL];
 #pragma unroll
   for (int k = 0; k < CPL; ++k) acc[k] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -57,7 +56,8 @@ __global__ void __launch_bounds__(kNT) glm_potential_kernel(PotArgs a) {
   wave_rows(a.n, gridDim.x, blockIdx.x, r0, r1, b0, b1);
   RowSource src{a.idx, 0, Key{0, 0}, Key{0, 0}, 0, 0, 0, 0, a.idx ? a.N : (int64_t)a.n};
   accumulate_rows<LPR, CPL>(to_global(a.X), a.ldx, to_global(a.y), a.D4, src, r0, r1, th, a.L,
-                            acc, lik_acc, lds_lik, b0);
+                            acc, lik_acc, lds_lik, b0,
+                            [&] { load_theta<LPR, CPL>(to_global(a.theta), a.D, th); });
   // Block record: column sums, the block's lik sum and its lik sum of squared deviations
   // about the block mean; per-row likelihoods go straight to out_lik.
   const int stride = 4 * a.D4 + 2;
@@ -146,7 +146,7 @@ __global__ void __launch_bounds__(kNT) glm_full_kernel(FullArgs a) {
   __shared__ double lds_d[kWaves];
   __shared__ int flag;
   float4 th[CPL];
-  load_theta<LPR, CPL>(a.theta, a.D, th);
+  load_theta<LPR, CPL>(to_global(a.theta), a.D, th);
   constexpr int RPW = kWave / LPR;
   const int lane = threadIdx.x & (kWave - 1);
   const int seg = lane / LPR;

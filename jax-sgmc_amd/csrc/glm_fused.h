@@ -34,19 +34,59 @@ struct FusedArgs {
   float pot_temperature;
 };
 
-// Normal for element i of a single-leaf tree of size S under random_tree(sub):
-// the leaf key is split(sub, 1)[0].
-__device__ __forceinline__ float leaf_normal(Key leafkey, uint32_t S, uint32_t i) {
-  return bits_to_normal(bits_word(leafkey, S, i));
+// LDS of one fused block.
+template <int MODE>
+struct FusedLds {
+  __attribute__((aligned(16))) float cols[kWaves * kMaxD];  // the wavefronts' column sums
+  float small[4 * kWaves];                                   // reduction slots
+  float lik[kLdsRows];
+  float p[MODE == SGMC_MODE_SGHMC ? kMaxD : 1];              // resampled momentum
+  int flag;
+};
+
+// Sums over the block of wave sums that every wavefront has put in slot[0 .. kWaves) before
+// a barrier.
+__device__ __forceinline__ float slot_sum(const float* slot) {
+  float t = 0.0f;
+#pragma unroll
+  for (int i = 0; i < kWaves; ++i) t += slot[i];
+  return t;
+}
+__device__ __forceinline__ void put_slot(float* slot, float v) {
+  v = wave_sum(v);
+  if ((threadIdx.x & (kWave - 1)) == 0) slot[threadIdx.x / kWave] = v;
 }
 
-// MODE: the table's SGMC_MODE_*, fixed at compile time (the other modes' branches are
-// folded away).
+// One evaluation of chain ch by its block bchain: draw, gather, likelihood, reduction, and
+// in the chain's last block to arrive the update. MODE: the table's SGMC_MODE_*, fixed at
+// compile time (the other modes' branches are folded away).
+//
+// A launch of small chains is a chain of latencies: descriptor, keys, index draw, rows,
+// reduction, records, arrival, update. Everything that does not depend on the row sums is
+// therefore done while something else is awaited: the key splits run as one Threefry block
+// on two lanes each (split2_uniform), the step's noise, the resampled momentum and the
+// evaluation point are formed behind the first rows' loads, the update's state is loaded
+// with the arrival (every block loads it, 2 to 4 D floats; only the last uses it), the
+// iteration counter is advanced beside the update, and the reductions share barriers.
+// Per launch, from HIP graphs: 16 rms_prop chains (D = 100, n = 1000, 16 blocks each) 17.7 ->
+// 15.7 us, 64 SGHMC chains (D = 12, n = 300) 13.1 -> 9.6, 4 OBABO chains (D = 300, n = 512,
+// 16 blocks) 14.3 -> 11.3, one SGLD chain of 64 blocks (D = 300, n = 4096) 19.5 -> 14.8, 64
+// SGHMC chains (D = 512, n = 4096, 4 blocks) 95.7 -> 93. What is left of a small chain's 9 us
+// is the launch itself (2.5 us) and five dependent memory round trips.
 template <int LPR, int CPL, int MODE>
 __device__ __forceinline__ void fused_body(const FusedArgs& a, const sgmc_glm_chain& ch,
-                                           int bchain, float* lds_cols, float* lds_small,
-                                           float* lds_lik, int* flag) {
-  constexpr int mode = MODE;
+                                           int bchain, FusedLds<MODE>& lds) {
+  constexpr bool hmc = MODE == SGMC_MODE_SGHMC;
+  constexpr bool amg = MODE == SGMC_MODE_AMAGOLD;
+  constexpr bool ob_mh = MODE == SGMC_MODE_SGGMC;
+  constexpr bool ob = MODE == SGMC_MODE_OBABO || ob_mh;
+  constexpr bool rms = MODE == SGMC_MODE_SGLD_RMS;
+  constexpr bool has_mom = hmc || amg || ob;
+  constexpr bool shift = hmc || amg;  // evaluation point theta + scale M^-1 p
+  // noise pairs (j, j + m) of one thread
+  constexpr int NP = 4 * LPR * CPL > 2 * kNT ? 2 : 1;
+  const Key key0 = load_key(ch.key);
+  const Key dkey0 = load_key(ch.dkey);
   const int it = max(0, min(a.iter[0] + a.iter_offset, a.table_len - 1));
   const float eps = a.eps_table[it];
   const int D = ch.D;
@@ -59,13 +99,6 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const sgmc_glm_ch
   gfloat* g_samples = to_global(ch.samples);
   gcfloat* g_inv_mass = to_global(a.inv_mass);
   gcfloat* g_sqrt_mass = to_global(a.sqrt_mass);
-  const Key key0 = load_key(ch.key);
-  const bool hmc = mode == SGMC_MODE_SGHMC;
-  const bool amg = mode == SGMC_MODE_AMAGOLD;
-  const bool ob_mh = mode == SGMC_MODE_SGGMC;
-  const bool ob = mode == SGMC_MODE_OBABO || ob_mh;
-  const bool has_mom = hmc || amg || ob;
-  const bool shift = hmc || amg;  // evaluation point theta + scale M^-1 p
   const bool resample = hmc && a.step == 0;
   // OBABO: two launches per leapfrog step, the even one O B A, the odd one B O.
   const int sub = a.step & 1;
@@ -74,75 +107,28 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const sgmc_glm_ch
   // AMAGOLD iteration (integrator.py:521-523, 401-408).
   const float half = 0.5f * eps;
   const float pos_scale = (amg && a.step == 0) ? half : eps;
+  const uint32_t S = (uint32_t)D, m = (S + 1) >> 1;
 
-  // Momentum used by this step: resampled p = sqrt_mass * xi at the first step.
-  Key key_noise = key0;  // key split for this step's noise
-  Key resample_leaf{0, 0};
-  if (resample) {
-    Key k1, sub;
-    split2(key0, k1, sub);
-    resample_leaf = split_key(sub, 1, 0);
-    key_noise = k1;
-  }
-
-  // Evaluation point: theta (SGLD) or theta + scale M^-1 p (SGHMC, AMAGOLD).
+  // Loads of the evaluation point theta (SGLD, OBABO) or theta + scale M^-1 p (SGHMC,
+  // AMAGOLD).
+  const int q4 = 4 * ((threadIdx.x & (kWave - 1)) % LPR);
   float4 th[CPL];
-  {
-    const int q = (threadIdx.x & (kWave - 1)) % LPR;
-#pragma unroll
-    for (int k = 0; k < CPL; ++k) {
-      float e[4];
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const int c = 4 * (q + LPR * k) + t;
-        float v = 0.0f;
-        if (c < D) {
-          v = g_theta[c];
-          if (shift) {
-            float p;
-            if (resample) {
-              const float xi = leaf_normal(resample_leaf, (uint32_t)D, (uint32_t)c);
-              p = a.sqrt_mass ? g_sqrt_mass[c] * xi : xi;
-            } else {
-              p = g_mom[c];
-            }
-            const float s = a.inv_mass ? g_inv_mass[c] * p : p;
-            v = v + pos_scale * s;
-          }
-        }
-        e[t] = v;
-      }
-      th[k] = make_float4(e[0], e[1], e[2], e[3]);
-    }
-  }
+  load_theta<LPR, CPL>(g_theta, D, th);
+  float4 pe[CPL];
+  if (shift && !resample) load_theta<LPR, CPL>(g_mom, D, pe);
 
   // Minibatch indices: (dkey', sub) = split(dkey); k1, k2 = split(sub).
   Key dnext, dsub;
-  split2(load_key(ch.dkey), dnext, dsub);
+  split2_uniform(dkey0, dnext, dsub);
   RowSource src;
   src.idx = nullptr;
   src.draw = 1;
-  split2(dsub, src.k1, src.k2);
+  split2_uniform(dsub, src.k1, src.k2);
   src.n = (uint32_t)ch.n;
   src.span = (uint32_t)ch.N;
   src.mult = randint_mult(src.span);
   src.magic = randint_magic(src.span);
   src.rows = ch.N;
-  // Noise key of this step (used by the chain's last block only; derived here, where
-  // it overlaps the wait for the evaluation point, instead of after the arrival).
-  // OBABO: (key', s1, s2) = split(key, 3) at both launches of a leapfrog step; the even
-  // one draws from s1, the odd one from s2 and stores key'.
-  Key knext, leaf;
-  if (ob) {
-    Key k0, s1, s2;
-    split3(key0, k0, s1, s2);
-    leaf = split_key(sub ? s2 : s1, 1, 0);
-    knext = sub ? k0 : key0;
-  } else {
-    Key ksub;
-    split2(key_noise, knext, ksub);
-    leaf = split_key(ksub, 1, 0);
-  }
 
   float4 acc[CPL];
 #pragma unroll
@@ -150,55 +136,223 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const sgmc_glm_ch
   float lik_acc = 0.0f;
   int r0, r1, b0, b1;
   wave_rows(ch.n, ch.nblocks, bchain, r0, r1, b0, b1);
-  accumulate_rows<LPR, CPL>(to_global(ch.X), ch.ldx, to_global(ch.y), D4, src, r0, r1, th, a.L,
-                            acc, lik_acc, lds_lik, b0);
+  // The step's noise: thread t owns the pairs jp = t + kNT h (h < NP, jp < m) of elements
+  // jp and jp + m, which share one Threefry block. xr: the resampled momentum of the same
+  // elements.
+  Key knext;
+  float xi[NP][2], xr[NP][2];
+  accumulate_rows<LPR, CPL>(
+      to_global(ch.X), ch.ldx, to_global(ch.y), D4, src, r0, r1, th, a.L, acc, lik_acc, lds.lik,
+      b0, [&] {
+        // Noise key of this step. OBABO: (key', s1, s2) = split(key, 3) at both launches of
+        // a leapfrog step; the even one draws from s1, the odd one from s2 and stores key'.
+        Key leaf;
+        if (ob) {
+          Key k0, s1, s2;
+          split3(key0, k0, s1, s2);
+          leaf = split_key(sub ? s2 : s1, 1, 0);
+          knext = sub ? k0 : key0;
+        } else {
+          Key key_noise = key0, ksub;
+          if (resample) {
+            // momentum of this iteration: p = sqrt_mass * xi, drawn before the step's noise
+            split2_uniform(key0, key_noise, ksub);
+            const Key rleaf = split_key(ksub, 1, 0);
+#pragma unroll
+            for (int h = 0; h < NP; ++h) {
+              const uint32_t jp = threadIdx.x + kNT * h;
+              if (jp < m) {
+                uint32_t w0, w1;
+                bits_pair(rleaf, S, jp, w0, w1);
+                xr[h][0] = bits_to_normal(w0);
+                lds.p[jp] = a.sqrt_mass ? g_sqrt_mass[jp] * xr[h][0] : xr[h][0];
+                if (jp + m < S) {
+                  xr[h][1] = bits_to_normal(w1);
+                  lds.p[jp + m] = a.sqrt_mass ? g_sqrt_mass[jp + m] * xr[h][1] : xr[h][1];
+                }
+              }
+            }
+          }
+          split2_uniform(key_noise, knext, ksub);
+          leaf = split_key(ksub, 1, 0);
+        }
+#pragma unroll
+        for (int h = 0; h < NP; ++h) {
+          const uint32_t jp = threadIdx.x + kNT * h;
+          xi[h][0] = xi[h][1] = 0.0f;
+          if (jp < m) {
+            uint32_t w0, w1;
+            bits_pair(leaf, S, jp, w0, w1);
+            xi[h][0] = bits_to_normal(w0);
+            xi[h][1] = bits_to_normal(w1);
+          }
+        }
+        if (resample) {
+          lds_sync();
+#pragma unroll
+          for (int k = 0; k < CPL; ++k) {
+            float e[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+              const int c = q4 + 4 * LPR * k + t;
+              e[t] = c < D ? lds.p[c] : 0.0f;
+            }
+            pe[k] = make_float4(e[0], e[1], e[2], e[3]);
+          }
+        }
+        if (shift) {
+#pragma unroll
+          for (int k = 0; k < CPL; ++k) {
+            const float p[4] = {pe[k].x, pe[k].y, pe[k].z, pe[k].w};
+            float v[4] = {th[k].x, th[k].y, th[k].z, th[k].w};
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+              const int c = q4 + 4 * LPR * k + t;
+              if (c < D) {
+                const float s = a.inv_mass ? g_inv_mass[c] * p[t] : p[t];
+                v[t] = v[t] + pos_scale * s;
+              }
+            }
+            th[k] = make_float4(v[0], v[1], v[2], v[3]);
+          }
+        }
+      });
   // Block record: column sums, then the block's lik sum and its lik sum of squared
-  // deviations about the block mean (combined into var(lik) by the last block).
+  // deviations about the block mean (combined into var(lik) by the last block). A chain of
+  // one block keeps its record in LDS.
+  // The two column sums of a noise pair lie side by side in the record and are written
+  // and read by one 8-byte access each (two 4-byte ones where the caller's record buffer
+  // is not 8-byte aligned).
   const int stride = 4 * D4 + 2;
+  const bool single = ch.nblocks == 1;
+  const bool wide = ((uintptr_t)ch.partial & 7) == 0;
   gfloat* mine = g_partial + (int64_t)bchain * stride;
-  const float ls = block_reduce_write<LPR, CPL>(acc, lik_acc, D4, mine, lds_cols, lds_small);
+  const float ls = block_reduce<LPR, CPL>(acc, lik_acc, D4, lds.cols, lds.small);
+  float s[NP][2];
+#pragma unroll
+  for (int h = 0; h < NP; ++h) {
+    const uint32_t jp = threadIdx.x + kNT * h;
+    s[h][0] = s[h][1] = 0.0f;
+    if (jp < m) {
+      s[h][0] = col_sum(lds.cols, D4, jp);
+      if (jp + m < S) s[h][1] = col_sum(lds.cols, D4, jp + m);
+      if (!single) {
+        if (wide) {
+          publish2(mine + 2 * jp, s[h][0], s[h][1]);
+        } else {
+          publish(mine + 2 * jp, s[h][0]);
+          publish(mine + 2 * jp + 1, s[h][1]);
+        }
+      }
+    }
+  }
   const int cnt = b1 - b0;
-  float m2 = 0.0f;
+  float* slot1 = lds.small + kWaves;
   if (ch.var) {
     const float mb = cnt > 0 ? ls / (float)cnt : 0.0f;
     float s2 = 0.0f;
     for (int j = threadIdx.x; j < cnt; j += kNT) {
-      const float d = lds_lik[j] - mb;
+      const float d = lds.lik[j] - mb;
       s2 += d * d;
     }
-    m2 = block_sum<kNT>(s2, lds_small);
+    put_slot(slot1, s2);
   }
-  if (threadIdx.x == 0) {
+  if (ch.lik)
+    for (int j = threadIdx.x; j < cnt; j += kNT) g_lik[b0 + j] = lds.lik[j];
+  lds_sync();
+  const float m2 = ch.var ? slot_sum(slot1) : 0.0f;
+  if (!single && threadIdx.x == 0) {
     publish(mine + 4 * D4, ls);
     publish(mine + 4 * D4 + 1, m2);
   }
-  if (ch.lik)
-    for (int j = threadIdx.x; j < cnt; j += kNT) g_lik[b0 + j] = lds_lik[j];
-  // A chain of one block needs no arrival counter: a barrier makes its records
-  // visible to its own threads.
-  if (ch.nblocks == 1) {
-    __syncthreads();
-  } else if (!arrive_last(ch.counter, ch.nblocks, flag)) {
-    return;
+  // The state of the owned elements (the chain's other blocks only read it).
+  float wv[NP][2], pv[NP][2], imv[NP][2], smv[NP][2], vv[NP][2];
+#pragma unroll
+  for (int h = 0; h < NP; ++h) {
+    const uint32_t jp = threadIdx.x + kNT * h;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const uint32_t j = e && jp + m < S ? jp + m : jp;
+      const bool in = jp < m;
+      wv[h][e] = in ? g_theta[j] : 0.0f;
+      pv[h][e] = (in && has_mom && !resample) ? g_mom[j] : 0.0f;
+      imv[h][e] = (in && has_mom && a.inv_mass) ? g_inv_mass[j] : 1.0f;
+      smv[h][e] = (in && (resample || amg || ob) && a.sqrt_mass) ? g_sqrt_mass[j] : 1.0f;
+      vv[h][e] = (in && rms) ? g_v[j] : 0.0f;
+    }
   }
+  if (!single && !arrive_last(ch.counter, ch.nblocks, &lds.flag)) return;
 
   // ---- last block of this chain: potential, gradient and the state update ----
-  // Loads first: each of the first nb threads takes its block's (lik sum, M2) record
-  // now; the reductions that need them wait until after the parameter update, whose
-  // own loads (column sums, theta, momentum) do not depend on them, so the whole
-  // finalizer pays one memory round trip instead of one per phase.
+  const bool last_step = !has_mom || a.step == launches - 1;
+  // Every block of this chain has read the iteration counter. The last chain of the launch
+  // to get here advances it (read by the next launch), on a wavefront that does not wait
+  // for it.
+  if (a.advance >= 0 && threadIdx.x == kNT - kWave) {
+    const unsigned prev = atomicAdd(a.done, 1u);
+    if (prev == (unsigned)a.nchains - 1) {
+      atomicExch(a.done, 0u);
+      if (last_step && a.advance) atomicAdd(a.iter, 1);
+    }
+  }
   const int nb = ch.nblocks;
   const float c = (float)(-ch.N) / (float)ch.n;
   const int per_block = (ch.n + nb - 1) / nb;
   float rec_ls = 0.0f, rec_m2 = 0.0f;
-  if (threadIdx.x < nb) {
+  if (single) {
+    if (threadIdx.x == 0) {
+      rec_ls = ls;
+      rec_m2 = m2;
+    }
+  } else if (threadIdx.x < nb) {
     rec_ls = consume(g_partial + (int64_t)threadIdx.x * stride + 4 * D4);
     if (ch.var) rec_m2 = consume(g_partial + (int64_t)threadIdx.x * stride + 4 * D4 + 1);
   }
+  // Column sums over the records, in block order; with more records than one round of
+  // loads takes and threads to spare (m <= kNT / 2), in `parts` runs of blocks whose sums
+  // are then added in order.
+  constexpr bool kParts = 4 * LPR * CPL <= kNT;  // m <= kNT / 2
+  if (single) {
+    // the sum over one record starts from +0
+#pragma unroll
+    for (int h = 0; h < NP; ++h) {
+      s[h][0] = 0.0f + s[h][0];
+      s[h][1] = 0.0f + s[h][1];
+    }
+  } else if (kParts && wide && nb > 16) {
+    const int mp = m <= kNT / 4 ? kNT / 4 : kNT / 2;
+    const int parts = kNT / mp, part = threadIdx.x / mp, jl = threadIdx.x % mp;
+    const int per = (nb + parts - 1) / parts;
+    float p0 = 0.0f, p1 = 0.0f;
+    if (jl < (int)m)
+      sum_pairs<16>(g_partial + 2 * jl, stride, part * per, min(nb, part * per + per), p0, p1);
+    lds.cols[2 * threadIdx.x] = p0;
+    lds.cols[2 * threadIdx.x + 1] = p1;
+    lds_sync();
+    s[0][0] = s[0][1] = 0.0f;
+    if (threadIdx.x < mp)
+      for (int k = 0; k < parts; ++k) {
+        s[0][0] += lds.cols[2 * (k * mp + threadIdx.x)];
+        s[0][1] += lds.cols[2 * (k * mp + threadIdx.x) + 1];
+      }
+  } else {
+#pragma unroll
+    for (int h = 0; h < NP; ++h) {
+      const uint32_t jp = threadIdx.x + kNT * h;
+      if (jp >= m) break;
+      gcfloat* p = g_partial + 2 * jp;
+      // (the row buffers of CPL > 1 leave the registers for 32 records at their occupancy)
+      if (wide) sum_pairs<(CPL > 1 ? 32 : 16)>(p, stride, 0, nb, s[h][0], s[h][1]);
+      else sum_strided2(p, p + 1, stride, nb, s[h][0], s[h][1]);
+    }
+  }
+  float sl = rec_ls;
+  for (int b = threadIdx.x + kNT; b < nb; b += kNT)
+    sl += consume(g_partial + (int64_t)b * stride + 4 * D4);
+  put_slot(lds.small, sl);
 
   // AMAGOLD and SGGMC samples are saved after the Metropolis-Hastings test, not here.
   const int slot = (a.save_slot && !amg && !ob_mh) ? a.save_slot[it] : -1;
-  const bool last_step = !has_mom || a.step == launches - 1;
   const float Tn = ch.temperature;
   // obabo O-step coefficients (integrator.py:192-200): sqrt(exp(-f eps)) and
   // sqrt((1 - exp(-f eps)) T), float32.
@@ -208,7 +362,6 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const sgmc_glm_ch
     ob_noise = sqrtf((1.0f - perm) * Tn);
     ob_decay = sqrtf(perm);
   }
-  const bool rms = mode == SGMC_MODE_SGLD_RMS;
   // reversible_leapfrog momentum coefficients (integrator.py:420-437), float32.
   const float ef = eps * a.friction;
   const float am_decay = 1.0f - ef;
@@ -219,45 +372,24 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const sgmc_glm_ch
   float edot = 0.0f;
 
   float lp = 0.0f;
-  const uint32_t S = (uint32_t)D;
-  const uint32_t m = (S + 1) >> 1;
-  for (uint32_t jp = threadIdx.x; jp < m; jp += kNT) {
-    // Element jp and its partner jp + m share one Threefry block of the noise draw.
-    uint32_t w0, w1;
-    bits_pair(leaf, S, jp, w0, w1);
-    const bool two = jp + m < S;
-    const uint32_t jj[2] = {jp, two ? jp + m : jp};
-    // every load of both columns is issued before the arithmetic
-    float s[2];
-    sum_strided2(g_partial + jj[0], g_partial + jj[1], stride, nb, s[0], s[1]);
-    float wv[2], pv[2], imv[2], smv[2], vv[2];
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const uint32_t j = jj[h];
-      wv[h] = g_theta[j];
-      pv[h] = (has_mom && !resample) ? g_mom[j] : 0.0f;
-      imv[h] = (has_mom && a.inv_mass) ? g_inv_mass[j] : 1.0f;
-      smv[h] = ((resample || amg || ob) && a.sqrt_mass) ? g_sqrt_mass[j] : 1.0f;
-      vv[h] = rms ? g_v[j] : 0.0f;
-    }
+  for (int h = 0; h < NP; ++h) {
+    const uint32_t jp = threadIdx.x + kNT * h;
+    if (jp >= m) break;
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      if (h && !two) break;
-      const uint32_t j = jj[h];
-      const float xi = bits_to_normal(h ? w1 : w0);
-      float wj = wv[h];
+    for (int e = 0; e < 2; ++e) {
+      if (e && jp + m >= S) break;
+      const uint32_t j = e ? jp + m : jp;
+      const float x = xi[h][e];
+      float wj = wv[h][e];
       float p = 0.0f, sm = 0.0f;
       if (has_mom) {
-        if (resample) {
-          const float xr = leaf_normal(resample_leaf, S, j);
-          p = a.sqrt_mass ? smv[h] * xr : xr;
-        } else {
-          p = pv[h];
-        }
-        sm = a.inv_mass ? imv[h] * p : p;
+        if (resample) p = a.sqrt_mass ? smv[h][e] * xr[h][e] : xr[h][e];
+        else p = pv[h][e];
+        sm = a.inv_mass ? imv[h][e] * p : p;
         if (shift) wj = wj + pos_scale * sm;  // evaluation point
       }
-      float g = c * s[h];
+      float g = c * s[h][e];
       if (a.pr.has_prior) {
         g = g + wj * a.pr.inv_var;
         lp += (a.pr.log_norm + (wj * wj) * a.pr.inv_var) / -2.0f;
@@ -266,9 +398,9 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const sgmc_glm_ch
       float wn;
       if (!has_mom) {
         const float sg = (-eps) * g;
-        const float sn = sqrtf((2.0f * Tn) * eps) * xi;
+        const float sn = sqrtf((2.0f * Tn) * eps) * x;
         if (rms) {
-          const float vn = a.alpha * vv[h] + (1.0f - a.alpha) * (g * g);
+          const float vn = a.alpha * vv[h][e] + (1.0f - a.alpha) * (g * g);
           g_v[j] = vn;
           const float G = 1.0f / (a.lmbd + sqrtf(vn));
           wn = wj + ((0.0f + G * sg) + sqrtf(G) * sn);
@@ -279,53 +411,49 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const sgmc_glm_ch
         const float C = a.friction;
         float pn = p + ((-eps) * C) * sm;
         pn = pn + (-eps) * g;
-        pn = pn + C * (sqrtf(2.0f * eps) * xi);
+        pn = pn + C * (sqrtf(2.0f * eps) * x);
         g_mom[j] = pn;
         wn = wj;
       } else if (ob) {
         if (sub == 0) {
           // O: p1 = decay p + noise (M^{1/2} xi); B: p2 = (-eps/2) g + p1;
           // A: theta += eps M^-1 p2 (integrator.py:214-238).
-          const float p1 = ob_decay * p + ob_noise * (smv[h] * xi);
-          edot += p1 * (imv[h] * p1);
+          const float p1 = ob_decay * p + ob_noise * (smv[h][e] * x);
+          edot += p1 * (imv[h][e] * p1);
           const float p2 = (-half) * g + p1;
           if (ob_mh && a.step == 0) {
-            g_theta_old[j] = wv[h];
+            g_theta_old[j] = wv[h][e];
             g_mom_old[j] = p;
           }
           g_mom[j] = p2;
-          wn = wj + eps * (imv[h] * p2);
+          wn = wj + eps * (imv[h][e] * p2);
         } else {
           // B: p3 = (-eps/2) g + p2; O with the second noise (integrator.py:244-262).
           const float p3 = (-half) * g + p;
-          edot += p3 * (imv[h] * p3);
-          g_mom[j] = ob_decay * p3 + ob_noise * (smv[h] * xi);
+          edot += p3 * (imv[h][e] * p3);
+          g_mom[j] = ob_decay * p3 + ob_noise * (smv[h][e] * x);
           wn = wj;
         }
       } else {
         // p' = (((1 - eps f) p + (-eps) g) + sqrt(4 f eps) (M^{1/2} xi)) / (1 + eps f);
         // energy term (p + p') . (M^-1 g); final half position step after the last.
-        const float noise = am_noise * (smv[h] * xi);
+        const float noise = am_noise * (smv[h][e] * x);
         const float pn = am_rescale * ((am_decay * p + (-eps) * g) + noise);
-        edot += (p + pn) * (imv[h] * g);
+        edot += (p + pn) * (imv[h][e] * g);
         if (a.step == 0) {
-          g_theta_old[j] = wv[h];
+          g_theta_old[j] = wv[h][e];
           g_mom_old[j] = p;
         }
         g_mom[j] = pn;
-        wn = last_step ? wj + half * (imv[h] * pn) : wj;
+        wn = last_step ? wj + half * (imv[h][e] * pn) : wj;
       }
       g_theta[j] = wn;
       if (slot >= 0 && last_step && ch.samples) g_samples[(int64_t)slot * D + j] = wn;
     }
   }
+  lds_sync();  // the lik sums of the records
+  const float mean = slot_sum(lds.small) / (float)ch.n;
   // var(lik) = (sum_b M2_b + cnt_b (mean_b - mean)^2) / n  (pairwise/Chan combination)
-  float sl = rec_ls;
-  for (int b = threadIdx.x + kNT; b < nb; b += kNT)
-    sl += consume(g_partial + (int64_t)b * stride + 4 * D4);
-  const float sumlik = block_sum<kNT>(sl, lds_small);
-  const float mean = sumlik / (float)ch.n;
-  float var_sum = 0.0f;
   if (ch.var) {
     float t = 0.0f;
     for (int b = threadIdx.x; b < nb; b += kNT) {
@@ -339,11 +467,14 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const sgmc_glm_ch
         t += m2_b + (float)k * (d * d);
       }
     }
-    var_sum = block_sum<kNT>(t, lds_small);
+    put_slot(lds.small + kWaves, t);
   }
-  lp = block_sum<kNT>(lp, lds_small);
-  if (amg || ob) edot = block_sum<kNT>(edot, lds_small);
+  put_slot(lds.small + 2 * kWaves, lp);
+  if (amg || ob) put_slot(lds.small + 3 * kWaves, edot);
+  lds_sync();
   if (threadIdx.x == 0) {
+    lp = slot_sum(lds.small + 2 * kWaves);
+    if (amg || ob) edot = slot_sum(lds.small + 3 * kWaves);
     if (amg) ch.energy[0] = half * edot + (a.step == 0 ? 0.0f : ch.energy[0]);
     if (ob) ch.energy[sub] = ch.energy[sub] + 0.5f * edot;
     const float Uc = ((float)(-ch.N) * mean - lp) / a.pot_temperature;
@@ -353,17 +484,9 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const sgmc_glm_ch
     if (ob_mh && a.step == 0) ch.energy[2] = ch.U[0];
     ch.U[0] = Uk;
     if (slot >= 0 && last_step && ch.samples_U) ch.samples_U[slot] = Uk;
-    if (ch.var) ch.var[0] = var_sum / (float)ch.n;
+    if (ch.var) ch.var[0] = slot_sum(lds.small + kWaves) / (float)ch.n;
     store_key(ch.key, knext);
     store_key(ch.dkey, dnext);
-    // Last chain of the launch advances the iteration counter (read by the next launch).
-    if (a.advance >= 0) {
-      const unsigned prev = atomicAdd(a.done, 1u);
-      if (prev == (unsigned)a.nchains - 1) {
-        atomicExch(a.done, 0u);
-        if (last_step && a.advance) atomicAdd(a.iter, 1);
-      }
-    }
   }
 }
 
@@ -688,34 +811,29 @@ __device__ __forceinline__ void resident_loop(const FusedArgs& a, const sgmc_glm
 // iteration counter by the number of iterations.
 template <int DCLASS, int MODE>
 __global__ void __launch_bounds__(kNT) glm_loop_kernel(FusedArgs a, int iterations) {
-  __shared__ __attribute__((aligned(16))) float lds_cols[kWaves * kMaxD];
-  __shared__ float lds_small[kWaves];
-  __shared__ float lds_lik[kLdsRows];
-  __shared__ float res_th[64];
-  __shared__ float res_eps[kResWindow];
-  __shared__ int res_slot[kResWindow];
-  __shared__ uint32_t res_kp[16];
-  __shared__ float res_xi[128];
-  __shared__ int flag;
+  __shared__ FusedLds<MODE> lds;
   // The grid has one block per chain and every chain one block (sgmc_glm_check_table).
   const int chain = blockIdx.x;
   const sgmc_glm_chain ch = a.chains[chain];
   const int dc = DCLASS >= 0 ? DCLASS : ch.dclass;
   FusedArgs b = a;
   b.advance = -1;
-  constexpr int mode = MODE;
-  const int launches = mode == SGMC_MODE_OBABO ? 2 * a.steps : a.steps;
+  const int launches = MODE == SGMC_MODE_OBABO ? 2 * a.steps : a.steps;
   // SGLD chains of D <= 64 and minibatches of at most 256 rows without per-row
   // likelihood output run resident (block-uniform choice)
   bool resident = false;
-  constexpr bool kResident = DCLASS == 0 || DCLASS == 5 || DCLASS == 1;
-  if constexpr (kResident)
-    resident = (mode == SGMC_MODE_SGLD || mode == SGMC_MODE_SGLD_RMS) && !ch.lik &&
-               ch.n <= kWaves * kWave;
-  if (resident) {
-    if constexpr (kResident)
+  constexpr bool kResident = (DCLASS == 0 || DCLASS == 5 || DCLASS == 1) &&
+                             (MODE == SGMC_MODE_SGLD || MODE == SGMC_MODE_SGLD_RMS);
+  if constexpr (kResident) {
+    __shared__ float res_th[64];
+    __shared__ float res_eps[kResWindow];
+    __shared__ int res_slot[kResWindow];
+    __shared__ uint32_t res_kp[16];
+    __shared__ float res_xi[128];
+    resident = !ch.lik && ch.n <= kWaves * kWave;
+    if (resident)
       resident_loop<DCLASS == 0 ? 4 : DCLASS == 5 ? 8 : 16, MODE>(
-          a, ch, iterations, lds_cols, lds_small, lds_lik, res_th, res_eps, res_slot, res_kp,
+          a, ch, iterations, lds.cols, lds.small, lds.lik, res_th, res_eps, res_slot, res_kp,
           res_xi);
   }
   for (int t = 0; t < (resident ? 0 : iterations); ++t) {
@@ -723,12 +841,12 @@ __global__ void __launch_bounds__(kNT) glm_loop_kernel(FusedArgs a, int iteratio
     for (int st = 0; st < launches; ++st) {
       b.step = st;
       switch (dc) {
-        case 0: fused_body<4, 1, MODE>(b, ch, 0, lds_cols, lds_small, lds_lik, &flag); break;
-        case 1: fused_body<16, 1, MODE>(b, ch, 0, lds_cols, lds_small, lds_lik, &flag); break;
-        case 5: fused_body<8, 1, MODE>(b, ch, 0, lds_cols, lds_small, lds_lik, &flag); break;
-        case 2: fused_body<64, 1, MODE>(b, ch, 0, lds_cols, lds_small, lds_lik, &flag); break;
-        case 3: fused_body<64, 2, MODE>(b, ch, 0, lds_cols, lds_small, lds_lik, &flag); break;
-        default: fused_body<64, 4, MODE>(b, ch, 0, lds_cols, lds_small, lds_lik, &flag); break;
+        case 0: fused_body<4, 1, MODE>(b, ch, 0, lds); break;
+        case 1: fused_body<16, 1, MODE>(b, ch, 0, lds); break;
+        case 5: fused_body<8, 1, MODE>(b, ch, 0, lds); break;
+        case 2: fused_body<64, 1, MODE>(b, ch, 0, lds); break;
+        case 3: fused_body<64, 2, MODE>(b, ch, 0, lds); break;
+        default: fused_body<64, 4, MODE>(b, ch, 0, lds); break;
       }
       __syncthreads();
     }
@@ -744,10 +862,7 @@ __global__ void __launch_bounds__(kNT) glm_loop_kernel(FusedArgs a, int iteratio
 
 template <int DCLASS, int MODE>
 __global__ void __launch_bounds__(kNT) glm_fused_kernel(FusedArgs a) {
-  __shared__ __attribute__((aligned(16))) float lds_cols[kWaves * kMaxD];
-  __shared__ float lds_small[kWaves];
-  __shared__ float lds_lik[kLdsRows];
-  __shared__ int flag;
+  __shared__ FusedLds<MODE> lds;
   // A uniform table maps blocks to chains arithmetically, which saves the dependent
   // load of the map before the chain descriptor can be read.
   // The block map and the chains' block ranges agree (sgmc_glm_check_table checks the
@@ -760,12 +875,12 @@ __global__ void __launch_bounds__(kNT) glm_fused_kernel(FusedArgs a) {
   const int bchain = blockIdx.x - ch.block_begin;
   const int dc = DCLASS >= 0 ? DCLASS : ch.dclass;
   switch (dc) {
-    case 0: fused_body<4, 1, MODE>(a, ch, bchain, lds_cols, lds_small, lds_lik, &flag); break;
-    case 1: fused_body<16, 1, MODE>(a, ch, bchain, lds_cols, lds_small, lds_lik, &flag); break;
-    case 5: fused_body<8, 1, MODE>(a, ch, bchain, lds_cols, lds_small, lds_lik, &flag); break;
-    case 2: fused_body<64, 1, MODE>(a, ch, bchain, lds_cols, lds_small, lds_lik, &flag); break;
-    case 3: fused_body<64, 2, MODE>(a, ch, bchain, lds_cols, lds_small, lds_lik, &flag); break;
-    default: fused_body<64, 4, MODE>(a, ch, bchain, lds_cols, lds_small, lds_lik, &flag); break;
+    case 0: fused_body<4, 1, MODE>(a, ch, bchain, lds); break;
+    case 1: fused_body<16, 1, MODE>(a, ch, bchain, lds); break;
+    case 5: fused_body<8, 1, MODE>(a, ch, bchain, lds); break;
+    case 2: fused_body<64, 1, MODE>(a, ch, bchain, lds); break;
+    case 3: fused_body<64, 2, MODE>(a, ch, bchain, lds); break;
+    default: fused_body<64, 4, MODE>(a, ch, bchain, lds); break;
   }
 }
 

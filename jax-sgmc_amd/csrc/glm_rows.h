@@ -66,7 +66,7 @@ struct RowSource {
 
 // Sum over the LPR lanes of a segment (segments are aligned runs of LPR lanes); every
 // lane of the segment gets the sum. Steps inside a 16-lane row use DPP (quad
-// permutes, half-row and row mirrors), the xor-16 step a ds_swizzle, the last step
+// permutes, half-row and row mirrors), the xor-16 step a lane swap, the last step
 // two readlanes.
 template <int CTRL>
 __device__ __forceinline__ float dpp_add(float v) {
@@ -80,7 +80,7 @@ __device__ __forceinline__ float seg_sum(float v) {
   if (LPR >= 4) v = dpp_add<0x4E>(v);   // quad_perm [2,3,0,1]
   if (LPR >= 8) v = dpp_add<0x141>(v);  // row_half_mirror
   if (LPR >= 16) v = dpp_add<0x140>(v); // row_mirror
-  if (LPR >= 32) v += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), 0x401F));
+  if (LPR >= 32) v = xor16_add(v);
   if (LPR >= 64)
     v = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 0)) +
         __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 32));
@@ -98,10 +98,26 @@ struct Unroll {
 
 // Row ids of one 64-row chunk of a wavefront's range: lane l holds the id of row cb + l
 // (-1 when outside [0, rows) or past the range end). Labels are loaded with the rows'
-// features, so nothing here has to be waited on before the next loads are issued.
+// features, so nothing here has to be waited on before the next loads are issued. At
+// most 32 drawn rows take their two randint words on the two lane halves (lanes 0-31 the
+// words of k1, lanes 32-63 those of k2), one Threefry block of latency instead of two.
+// Every lane of the wavefront calls this.
 __device__ __forceinline__ int chunk_rows(const RowSource& src, int cb, int r1) {
   const int lane = threadIdx.x & (kWave - 1);
   int rid = -1;
+  if (src.draw && r1 - cb <= kWave / 2) {
+    const int rr = lane & (kWave / 2 - 1);
+    const bool low = lane < kWave / 2;
+    const Key kk = {low ? src.k1.k0 : src.k2.k0, low ? src.k1.k1 : src.k2.k1};
+    const uint32_t word = bits_word(kk, src.n, (uint32_t)min(cb + rr, r1 - 1));
+    uint32_t hi;
+    lane_swap32(word, hi);  // the k2 word of row rr
+    if (low && cb + rr < r1) {
+      const int64_t r = (int64_t)(int32_t)randint_offset(word, hi, src.span, src.mult, src.magic);
+      if (r >= 0 && r < src.rows) rid = (int)r;
+    }
+    return rid;
+  }
   if (cb + lane < r1) {
     const int64_t r = src.row(cb + lane);
     if (r >= 0) rid = (int)r;
@@ -251,23 +267,29 @@ __device__ __forceinline__ void process_group(RowGroup<LPR, CPL>& g, int row0, i
 
 // Accumulates sum_j r_j x_j (this lane's chunks) and sum_j lik_j over minibatch rows
 // [r0, r1). Loads run one row group ahead of the arithmetic (two register buffers), and
-// the row ids of the next 64-row chunk are drawn before the current chunk is done.
-template <int LPR, int CPL>
+// the row ids of the next 64-row chunk are drawn before the current chunk is done. mid()
+// runs (on every wavefront, also one without rows) when the first loads are in flight: it
+// sets th, and whatever else does not depend on the rows is hidden behind them.
+template <int LPR, int CPL, class Mid>
 __device__ __forceinline__ void accumulate_rows(gcfloat* __restrict__ X, int64_t ldx,
                                                 gcfloat* __restrict__ y, int D4,
                                                 const RowSource& src, int r0, int r1,
                                                 const float4 (&th)[CPL], const Lik& L,
                                                 float4 (&acc)[CPL], float& lik_acc,
-                                                float* lds_lik, int lds_row0) {
+                                                float* lds_lik, int lds_row0, Mid mid) {
   constexpr int RPW = kWave / LPR;
   constexpr int G = RPW * RowGroup<LPR, CPL>::U;  // rows per group; divides 64
   static_assert(kWave % G == 0, "row groups must tile a 64-row chunk");
-  if (r0 >= r1) return;
+  if (r0 >= r1) {
+    mid();
+    return;
+  }
   int cb = r0;
   int rid = chunk_rows(src, cb, r1);
-  int rid_n = chunk_rows(src, cb + kWave, r1);
   RowGroup<LPR, CPL> ga, gb;
   load_group<LPR, CPL>(X, ldx, y, D4, 0, rid, ga);
+  int rid_n = cb + kWave < r1 ? chunk_rows(src, cb + kWave, r1) : -1;
+  mid();
   int gl = 0;  // group offset inside the current chunk
   // The prefetch is issued on every path (rows past the range carry id -1 and load the
   // clamped row 0), so the number of loads in flight is the same on every path and the
@@ -283,7 +305,7 @@ __device__ __forceinline__ void accumulate_rows(gcfloat* __restrict__ X, int64_t
       cb += kWave;
       nl = 0;
       rid = rid_n;
-      rid_n = chunk_rows(src, cb + kWave, r1);
+      rid_n = cb + kWave < r1 ? chunk_rows(src, cb + kWave, r1) : -1;
     }
     gl = nl;
     nl = gl + G;
@@ -296,32 +318,41 @@ __device__ __forceinline__ void accumulate_rows(gcfloat* __restrict__ X, int64_t
       cb += kWave;
       nl = 0;
       rid = rid_n;
-      rid_n = chunk_rows(src, cb + kWave, r1);
+      rid_n = cb + kWave < r1 ? chunk_rows(src, cb + kWave, r1) : -1;
     }
     gl = nl;
   }
 }
 
-// Reduces acc over the segments of each wavefront and over the block's wavefronts;
-// hands column sum c (0 <= c < 4 D4) to put(c, s) and returns the block's lik sum.
-template <int LPR, int CPL, bool LDS_SYNC = false, class Put>
+// v + (v of lane l ^ M).
+template <int M>
+__device__ __forceinline__ float xor_add(float v) {
+  if (M == 32) return xor32_add(v);
+  if (M == 16) return xor16_add(v);
+  if (M == 8) return ror_add<8>(v);
+  return v + __shfl_xor(v, M, kWave);
+}
+template <int M>
+__device__ __forceinline__ void xor_add4(float4& a) {
+  a = make_float4(xor_add<M>(a.x), xor_add<M>(a.y), xor_add<M>(a.z), xor_add<M>(a.w));
+}
+
+// Reduces acc over the segments of each wavefront and leaves the wavefronts' sums in
+// lds_cols ([kWaves][4 D4]) and their lik sums in lds_small; returns the block's lik sum.
+// One barrier: lds_cols and lds_small must not be in use by a slower wavefront.
+template <int LPR, int CPL>
 __device__ __forceinline__ float block_reduce(float4 (&acc)[CPL], float lik_acc, int D4,
-                                              float* lds_cols, float* lds_small, Put put) {
+                                              float* lds_cols, float* lds_small) {
   const int lane = threadIdx.x & (kWave - 1);
   const int w = threadIdx.x / kWave;
   const int q = lane % LPR;
 #pragma unroll
   for (int k = 0; k < CPL; ++k) {
-#pragma unroll
-    for (int m = LPR; m < kWave; m <<= 1) {
-      acc[k].x += __shfl_xor(acc[k].x, m, kWave);
-      acc[k].y += __shfl_xor(acc[k].y, m, kWave);
-      acc[k].z += __shfl_xor(acc[k].z, m, kWave);
-      acc[k].w += __shfl_xor(acc[k].w, m, kWave);
-    }
+    if (LPR <= 4) xor_add4<4>(acc[k]);
+    if (LPR <= 8) xor_add4<8>(acc[k]);
+    if (LPR <= 16) xor_add4<16>(acc[k]);
+    if (LPR <= 32) xor_add4<32>(acc[k]);
   }
-  if (LDS_SYNC) lds_sync();
-  else __syncthreads();
   if (lane < LPR) {
 #pragma unroll
     for (int k = 0; k < CPL; ++k) {
@@ -329,14 +360,21 @@ __device__ __forceinline__ float block_reduce(float4 (&acc)[CPL], float lik_acc,
       if (c4 < D4) reinterpret_cast<float4*>(lds_cols + w * 4 * D4)[c4] = acc[k];
     }
   }
-  const float lsum = block_sum<kNT, LDS_SYNC>(lik_acc, lds_small);  // contains barriers
-  for (int c = threadIdx.x; c < 4 * D4; c += kNT) {
-    float s = 0.0f;
+  lik_acc = wave_sum(lik_acc);
+  if (lane == 0) lds_small[w] = lik_acc;
+  __syncthreads();
+  float lsum = 0.0f;
 #pragma unroll
-    for (int ww = 0; ww < kWaves; ++ww) s += lds_cols[ww * 4 * D4 + c];
-    put(c, s);
-  }
+  for (int i = 0; i < kWaves; ++i) lsum += lds_small[i];
   return lsum;
+}
+
+// Column sum c over the wavefronts.
+__device__ __forceinline__ float col_sum(const float* lds_cols, int D4, int c) {
+  float s = 0.0f;
+#pragma unroll
+  for (int ww = 0; ww < kWaves; ++ww) s += lds_cols[ww * 4 * D4 + c];
+  return s;
 }
 
 // block_reduce with the column sums published to out[0..4*D4) for the chain's last block.
@@ -344,8 +382,9 @@ template <int LPR, int CPL>
 __device__ __forceinline__ float block_reduce_write(float4 (&acc)[CPL], float lik_acc, int D4,
                                                     gfloat* __restrict__ out, float* lds_cols,
                                                     float* lds_small) {
-  return block_reduce<LPR, CPL>(acc, lik_acc, D4, lds_cols, lds_small,
-                                [&](int c, float s) { publish(out + c, s); });
+  const float lsum = block_reduce<LPR, CPL>(acc, lik_acc, D4, lds_cols, lds_small);
+  for (int c = threadIdx.x; c < 4 * D4; c += kNT) publish(out + c, col_sum(lds_cols, D4, c));
+  return lsum;
 }
 
 // Splits rows [0, n) of a minibatch among the blocks of a chain and then among the
@@ -362,7 +401,7 @@ __device__ __forceinline__ void wave_rows(int n, int nblocks, int b, int& r0, in
 }
 
 template <int LPR, int CPL>
-__device__ __forceinline__ void load_theta(const float* __restrict__ w, int D, float4 (&th)[CPL]) {
+__device__ __forceinline__ void load_theta(gcfloat* w, int D, float4 (&th)[CPL]) {
   const int q = (threadIdx.x & (kWave - 1)) % LPR;
 #pragma unroll
   for (int k = 0; k < CPL; ++k) {

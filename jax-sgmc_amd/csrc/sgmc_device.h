@@ -330,16 +330,69 @@ __device__ __forceinline__ void store_key(uint32_t* p, Key k) {
 
 // ---- wavefront / block reductions ---------------------------------------------
 
+// v + (v of lane l ^ 32), v + (v of lane l ^ 16) by the lane-swap instructions.
+__device__ __forceinline__ uint32_t lane_swap32(uint32_t v, uint32_t& other) {
+  const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  other = r[1];
+  return r[0];
+}
+__device__ __forceinline__ uint32_t lane_swap16(uint32_t v, uint32_t& other) {
+  const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  other = r[1];
+  return r[0];
+}
+__device__ __forceinline__ float xor32_add(float v) {
+  uint32_t b;
+  const uint32_t a = lane_swap32(__float_as_uint(v), b);
+  return __uint_as_float(a) + __uint_as_float(b);
+}
+__device__ __forceinline__ float xor16_add(float v) {
+  uint32_t b;
+  const uint32_t a = lane_swap16(__float_as_uint(v), b);
+  return __uint_as_float(a) + __uint_as_float(b);
+}
+// v rotated by N lanes inside each row of 16 (the same lane as l ^ 8 for N = 8).
+template <int N>
+__device__ __forceinline__ uint32_t row_ror(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x120 + N, 0xF, 0xF, false);
+}
+template <int N>
+__device__ __forceinline__ float ror_add(float v) {
+  return v + __uint_as_float(row_ror<N>(__float_as_uint(v)));
+}
+__device__ __forceinline__ double make_d(uint32_t lo, uint32_t hi) {
+  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+template <int N>
+__device__ __forceinline__ double ror_add_d(double v) {
+  const uint64_t u = (uint64_t)__double_as_longlong(v);
+  return v + make_d(row_ror<N>((uint32_t)u), row_ror<N>((uint32_t)(u >> 32)));
+}
+
+// Wavefront sums, every lane gets the total. The additions are those of an xor butterfly
+// over 32, 16, 8, 4, 2, 1 (the same bits): after the xor-32, 16 and 8 steps the values
+// repeat every 8 lanes, so a rotation by 4 inside a row of 16 fetches the xor-4 partner's
+// value, and so on. Lane swaps and DPP adds, no LDS permutes (one of the latter costs
+// about 100 cycles of latency on the path of every reduction).
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
-  return v;
+  v = xor16_add(xor32_add(v));
+  return ror_add<1>(ror_add<2>(ror_add<4>(ror_add<8>(v))));
 }
 
 __device__ __forceinline__ double wave_sum_d(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
-  return v;
+  {
+    const uint64_t u = (uint64_t)__double_as_longlong(v);
+    uint32_t lb, hb;
+    const uint32_t la = lane_swap32((uint32_t)u, lb), ha = lane_swap32((uint32_t)(u >> 32), hb);
+    v = make_d(la, ha) + make_d(lb, hb);
+  }
+  {
+    const uint64_t u = (uint64_t)__double_as_longlong(v);
+    uint32_t lb, hb;
+    const uint32_t la = lane_swap16((uint32_t)u, lb), ha = lane_swap16((uint32_t)(u >> 32), hb);
+    v = make_d(la, ha) + make_d(lb, hb);
+  }
+  return ror_add_d<1>(ror_add_d<2>(ror_add_d<4>(ror_add_d<8>(v))));
 }
 
 // Sum over a block of NT threads (NT a multiple of 64); every thread gets the total.
@@ -401,6 +454,51 @@ __device__ __forceinline__ double consume(const double* p) {
   return __hip_atomic_load(to_global(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Two adjacent floats (p 8-byte aligned) published in one store, consumed in one load.
+__device__ __forceinline__ void publish2(SGMC_GLOBAL float* p, float a, float b) {
+  __hip_atomic_store((SGMC_GLOBAL uint64_t*)p,
+                     ((uint64_t)__float_as_uint(b) << 32) | __float_as_uint(a), __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint64_t consume2(const SGMC_GLOBAL float* p) {
+  return __hip_atomic_load((const SGMC_GLOBAL uint64_t*)p, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Adds records b .. b + K - 1 (those below b1) to a0, a1 in order. All K loads go out before
+// the first add, without branches in between (records past b1 - 1 reload that one and are
+// not added).
+template <int K>
+__device__ __forceinline__ void add_pairs(const SGMC_GLOBAL float* p, int64_t stride, int b,
+                                          int b1, float& a0, float& a1) {
+  uint64_t x[K];
+#pragma unroll
+  for (int t = 0; t < K; ++t) x[t] = consume2(p + (int64_t)min(b + t, b1 - 1) * stride);
+#pragma unroll
+  for (int t = 0; t < K; ++t) {
+    const bool in = b + t < b1;
+    a0 += in ? __uint_as_float((uint32_t)x[t]) : 0.0f;
+    a1 += in ? __uint_as_float((uint32_t)(x[t] >> 32)) : 0.0f;
+  }
+}
+
+// s0 = sum over b in [b0, b1) of p[b * stride], s1 of p[b * stride + 1], each added in
+// block order from +0, from published records 8-byte aligned. Up to MOST (16 or 32, two
+// registers each) records are in flight at a time: with eight, a chain of 64 blocks paid
+// eight memory round trips here.
+template <int MOST>
+__device__ __forceinline__ void sum_pairs(const SGMC_GLOBAL float* p, int64_t stride, int b0,
+                                          int b1, float& s0, float& s1) {
+  float a0 = 0.0f, a1 = 0.0f;
+  int b = b0;
+  for (; b1 - b > 16; b += MOST) add_pairs<MOST>(p, stride, b, b1, a0, a1);
+  if (b1 - b > 8) add_pairs<16>(p, stride, b, b1, a0, a1);
+  else if (b1 - b > 4) add_pairs<8>(p, stride, b, b1, a0, a1);
+  else if (b1 - b > 0) add_pairs<4>(p, stride, b, b1, a0, a1);
+  s0 = a0;
+  s1 = a1;
+}
+
 // s0 = sum over b in [0, nb) of p0[b * stride], s1 likewise for p1, each added in block
 // order, from published records. The loads go out eight records at a time (missing
 // records read as +0, which leaves the sums unchanged), so one memory latency covers
@@ -440,9 +538,10 @@ __device__ __forceinline__ bool arrive_last(unsigned* counter, unsigned expected
   __syncthreads();
   if (threadIdx.x == 0) {
     const unsigned prev =
-        __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_fetch_add(to_global(counter), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const bool last = (prev == expected - 1);
-    if (last) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (last)
+      __hip_atomic_store(to_global(counter), 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     *lds_flag = last ? 1 : 0;
   }
   __syncthreads();
