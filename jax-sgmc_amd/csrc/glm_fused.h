@@ -844,6 +844,7 @@ __global__ void __launch_bounds__(kNT) glm_loop_kernel(FusedArgs a, int iteratio
         case 0: fused_body<4, 1, MODE>(b, ch, 0, lds); break;
         case 1: fused_body<16, 1, MODE>(b, ch, 0, lds); break;
         case 5: fused_body<8, 1, MODE>(b, ch, 0, lds); break;
+        case 6: fused_body<32, 1, MODE>(b, ch, 0, lds); break;
         case 2: fused_body<64, 1, MODE>(b, ch, 0, lds); break;
         case 3: fused_body<64, 2, MODE>(b, ch, 0, lds); break;
         default: fused_body<64, 4, MODE>(b, ch, 0, lds); break;
@@ -878,6 +879,7 @@ __global__ void __launch_bounds__(kNT) glm_fused_kernel(FusedArgs a) {
     case 0: fused_body<4, 1, MODE>(a, ch, bchain, lds); break;
     case 1: fused_body<16, 1, MODE>(a, ch, bchain, lds); break;
     case 5: fused_body<8, 1, MODE>(a, ch, bchain, lds); break;
+    case 6: fused_body<32, 1, MODE>(a, ch, bchain, lds); break;
     case 2: fused_body<64, 1, MODE>(a, ch, bchain, lds); break;
     case 3: fused_body<64, 2, MODE>(a, ch, bchain, lds); break;
     default: fused_body<64, 4, MODE>(a, ch, bchain, lds); break;
@@ -899,6 +901,7 @@ void launch_fused(int dclass, int nblocks, hipStream_t s, const FusedArgs& a) {
     case 3: hipLaunchKernelGGL((glm_fused_kernel<3, MODE>), grid, block, 0, s, a); break;
     case 4: hipLaunchKernelGGL((glm_fused_kernel<4, MODE>), grid, block, 0, s, a); break;
     case 5: hipLaunchKernelGGL((glm_fused_kernel<5, MODE>), grid, block, 0, s, a); break;
+    case 6: hipLaunchKernelGGL((glm_fused_kernel<6, MODE>), grid, block, 0, s, a); break;
     default: hipLaunchKernelGGL((glm_fused_kernel<-1, MODE>), grid, block, 0, s, a); break;
   }
 }
@@ -913,6 +916,7 @@ void launch_loop(int dclass, int nchains, int iterations, hipStream_t s, const F
     case 3: hipLaunchKernelGGL((glm_loop_kernel<3, MODE>), grid, block, 0, s, a, iterations); break;
     case 4: hipLaunchKernelGGL((glm_loop_kernel<4, MODE>), grid, block, 0, s, a, iterations); break;
     case 5: hipLaunchKernelGGL((glm_loop_kernel<5, MODE>), grid, block, 0, s, a, iterations); break;
+    case 6: hipLaunchKernelGGL((glm_loop_kernel<6, MODE>), grid, block, 0, s, a, iterations); break;
     default:
       hipLaunchKernelGGL((glm_loop_kernel<-1, MODE>), grid, block, 0, s, a, iterations);
       break;
