@@ -33,6 +33,8 @@ _OBABO = (_lib.MODE_OBABO, _lib.MODE_SGGMC)
 # floats of per-chain energy bookkeeping: AMAGOLD's energy; OBABO's kinetic energies at
 # the start and the end; SGGMC's as OBABO plus the minibatch potential of the start
 _ENERGY = {_lib.MODE_AMAGOLD: 1, _lib.MODE_OBABO: 2, _lib.MODE_SGGMC: 3}
+# modes without a test between iterations, which a loop launch can run
+_LOOPS = (_lib.MODE_SGLD, _lib.MODE_SGLD_RMS, _lib.MODE_SGHMC, _lib.MODE_OBABO)
 _KEEPS_START = (_lib.MODE_AMAGOLD, _lib.MODE_SGGMC)
 FAMILIES = {"linear_gaussian": _lib.LIK_LINEAR_GAUSSIAN, "logistic": _lib.LIK_LOGISTIC}
 NT = 256
@@ -54,6 +56,49 @@ def blocks_for(n, D, target_bytes):
   return max(1, -(-n // LDS_ROWS), min(nb, (n + 31) // 32))
 
 
+# Rows below which a further block of a chain only adds a record for the last block to
+# sum: one row group of each of the block's four wavefronts (256, 128 and 64 rows at
+# D <= 16, 32 and 64), and 32 rows above (two groups of the wavefronts' 4 or 8 rows).
+def _min_block_rows(D):
+  return 256 if D <= 16 else 128 if D <= 32 else 64 if D <= 64 else 32
+
+
+def default_blocks(n, D, loops, cus):
+  """Grid blocks of every chain of a table when no bytes-per-block target is given.
+
+  n, D: minibatch sizes and row lengths of the chains; loops: whether the table's sampler
+  can run iterations in one launch (one block per chain); cus: compute units.
+
+  - A chain whose minibatch is under 96 KiB gets one block where iterations can run in a
+    loop launch: D = 32, n = 512 takes 8.2 us per iteration there and 8.9 as launches of
+    four blocks, D = 100, n = 128 takes 7.9 and 9.2; D = 64, n = 512 (128 KiB) 11.3
+    against 9.4, D = 256, n = 128 (128 KiB) 10.9 against 9.4. Without a loop launch the
+    line is 40 KiB (D = 32, n = 256, 32 KiB: 8.6 with one block, 8.8 with two;
+    D = 100, n = 128, 51 KiB: 10.6 and 9.2).
+  - Otherwise the table gets one block per compute unit, shared out by the chains' bytes:
+    64 SGHMC chains (D = 512, n = 4096) take 93 us at 256 blocks, 102 at 192, 102 at 384
+    and 121 at 4096 (64 KiB of rows per block); 8 chains (D = 1000, n = 4096) 34.7 at 128
+    or 256 and 50.7 at 64; 16 rms_prop chains (D = 100, n = 1000) 13.7 at 256 and 15.6 at
+    96 blocks.
+  - Row lengths up to 256 (four resident blocks per unit instead of two or three) take two
+    blocks per unit where that still leaves a chain at most eight records: 64 chains of
+    D = 100, n = 2048 take 25.8 us at 256 blocks and 20.1 at 512; 8 chains of D = 256,
+    n = 2048 take 15.2 and 17.8 (64 records to sum per chain).
+  """
+  n, D = np.asarray(n, np.int64), np.asarray(D, np.int64)
+  rows_bytes = n * 4 * ((D + 3) // 4 * 4)
+  share = cus * rows_bytes / max(1, int(rows_bytes.sum()))
+  share = np.where(D <= 256, np.maximum(share, np.minimum(8.0, 2.0 * share)), share)
+  out = []
+  for nc, d, b, s in zip(n, D, rows_bytes, share):
+    least = -(-int(nc) // LDS_ROWS)
+    nb = min(int(round(float(s))), -(-int(nc) // _min_block_rows(int(d))))
+    if b < (96 if loops else 40) * 1024:
+      nb = 1
+    out.append(max(1, least, nb))
+  return out
+
+
 class FusedGLM:
   """Chain table for ``sgmc_glm_fused_step``.
 
@@ -62,6 +107,7 @@ class FusedGLM:
   dkey (two uint32 words each), temperature (SGLD noise temperature, default 1).
   Optional per-chain keys: N (observations, default X.shape[0]) and save (default
   True; False leaves the chain out of the sample buffer).
+  target_bytes: bytes of rows per block; default: the split of default_blocks.
   keep_lik: also keep the per-row likelihoods of the last evaluation in ``lik``.
   mode: "sgld", "sgld_rms" (one launch per iteration), "sghmc", "amagold" (``steps``
   launches), "obabo", "sggmc" (two launches per leapfrog step); "amagold" and "sggmc"
@@ -122,7 +168,8 @@ class FusedGLM:
     dcl = {_lib.query("sgmc_glm_dclass", d) for d in Ds}
     self.uniform_dclass = dcl.pop() if len(dcl) == 1 else -1
     total_bytes = sum(int(c["n"]) * 4 * _align4(int(c["D"])) for c in chains)
-    self.target_bytes = target_bytes or max(64 * 1024, total_bytes // 2048)
+    self._target_bytes = target_bytes or max(64 * 1024, total_bytes // 2048)
+    self._blocks_by_rule = not target_bytes  # until a target is set
     self.keep_lik = bool(keep_lik)
     self.exchange = None
     self.mh = None
@@ -176,8 +223,23 @@ class FusedGLM:
       self.samples = torch.zeros(self.n_slots * P, device=dev)
       self.samples_U = torch.zeros(self.C * self.n_slots, device=dev)
 
+  @property
+  def target_bytes(self):
+    """Bytes of rows per block; setting it replaces the default split at the next
+    _build_table."""
+    return self._target_bytes
+
+  @target_bytes.setter
+  def target_bytes(self, value):
+    self._target_bytes = value
+    self._blocks_by_rule = False
+
   def _build_table(self):
-    nbs = [blocks_for(int(n), int(d), self.target_bytes) for n, d in zip(self.n, self.D)]
+    if self._blocks_by_rule:
+      nbs = default_blocks(self.n, self.D, self.mode in _LOOPS,
+                           torch.cuda.get_device_properties(self.device).multi_processor_count)
+    else:
+      nbs = [blocks_for(int(n), int(d), self.target_bytes) for n, d in zip(self.n, self.D)]
     self.nblocks_chain = np.array(nbs)
     # Grid order: chains with the most bytes per block first, so that the longest
     # blocks start in the first wave of the dispatch (longest-processing-time first).
@@ -260,8 +322,7 @@ class FusedGLM:
     (``sgmc_glm_fused_loop``), cut at the exchange's test iterations."""
     return (bool(np.all(self.nblocks_chain == 1)) and self.mh is None and
             (self.exchange is None or self.exchange.sparse) and
-            self.mode in (_lib.MODE_SGLD, _lib.MODE_SGLD_RMS, _lib.MODE_SGHMC,
-                          _lib.MODE_OBABO))
+            self.mode in _LOOPS)
 
   def _launch_loop(self, iterations):
     _lib.call("sgmc_glm_fused_loop", _lib.ptr(self.table), self.C, self.uniform_dclass,
