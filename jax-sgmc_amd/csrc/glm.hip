@@ -32,14 +32,27 @@ struct PotArgs {
   float* out_lik;
   float* out_var;
   float* partial;      // [nblocks][4*D4 + 2]
-  unsigned* counter;
+  unsigned* counter;   // [kPotCounters]: the launch's, then one per run of blocks
   int64_t ldx;
   int64_t N;
   int n, D, D4;
+  int group;           // blocks per run of a two-level reduction, or 0
   Lik L;
   Prior pr;
   float temperature;
 };
+
+// Arrival counters of a potential launch.
+constexpr int kPotCounters = 64;
+
+// Blocks per run of the two-level reduction (0: one level). One level reads 32 records
+// per memory round trip; beyond that the last block's serial sum outgrows the round trip and
+// arrival that a second level adds (n = 40001, D = 301, 256 blocks: 121 us with one level
+// of eight records per round trip, 20.8 with two).
+static int pot_group(int nblocks) {
+  if (nblocks <= 32) return 0;
+  return std::max(16, (nblocks + kPotCounters - 2) / (kPotCounters - 1));
+}
 
 template <int LPR, int CPL>
 __global__ void __launch_bounds__(kNT) glm_potential_kernel(PotArgs a) {
@@ -59,10 +72,24 @@ __global__ void __launch_bounds__(kNT) glm_potential_kernel(PotArgs a) {
                             acc, lik_acc, lds_lik, b0,
                             [&] { load_theta<LPR, CPL>(to_global(a.theta), a.D, th); });
   // Block record: column sums, the block's lik sum and its lik sum of squared deviations
-  // about the block mean; per-row likelihoods go straight to out_lik.
+  // about the block mean; per-row likelihoods go straight to out_lik. Columns 2j and
+  // 2j + 1 are one 8-byte access (two 4-byte ones where the records are not 8-byte aligned).
   const int stride = 4 * a.D4 + 2;
-  gfloat* mine = to_global(a.partial) + (int64_t)blockIdx.x * stride;
-  const float ls = block_reduce_write<LPR, CPL>(acc, lik_acc, a.D4, mine, lds_cols, lds_small);
+  const int nb = gridDim.x;
+  gfloat* part = to_global(a.partial);
+  gfloat* mine = part + (int64_t)blockIdx.x * stride;
+  const bool wide = ((uintptr_t)a.partial & 7) == 0;
+  auto put2 = [&](gfloat* p, float s0, float s1) {
+    if (wide) {
+      publish2(p, s0, s1);
+    } else {
+      publish(p, s0);
+      publish(p + 1, s1);
+    }
+  };
+  const float ls = block_reduce<LPR, CPL>(acc, lik_acc, a.D4, lds_cols, lds_small);
+  for (int j = threadIdx.x; j < 2 * a.D4; j += kNT)
+    put2(mine + 2 * j, col_sum(lds_cols, a.D4, 2 * j), col_sum(lds_cols, a.D4, 2 * j + 1));
   const int cnt = b1 - b0;
   float m2 = 0.0f;
   if (a.out_var) {
@@ -82,28 +109,51 @@ __global__ void __launch_bounds__(kNT) glm_potential_kernel(PotArgs a) {
     gfloat* lo = to_global(a.out_lik);
     for (int j = threadIdx.x; j < cnt; j += kNT) lo[b0 + j] = lds_lik[j];
   }
-  if (!arrive_last(a.counter, gridDim.x, &flag)) return;
+  // Sums columns 2j, 2j + 1 over records 0 .. count - 1 of a run, `step` records apart.
+  auto sum2 = [&](gcfloat* p, int64_t step, int count, float& s0, float& s1) {
+    if (wide) sum_pairs<32>(p, step, 0, count, s0, s1);
+    else sum_strided2(p, p + 1, step, count, s0, s1);
+  };
+  // Many blocks reduce in two levels: the last block of each run of `group` blocks sums the
+  // run's columns into the run's first record, the last of those sums the runs.
+  const int runs = a.group ? (nb + a.group - 1) / a.group : nb;
+  const int64_t step = a.group ? (int64_t)a.group * stride : stride;
+  if (a.group) {
+    const int run = blockIdx.x / a.group, first = run * a.group;
+    const int members = min(a.group, nb - first);
+    if (!arrive_last(a.counter + 1 + run, members, &flag)) return;
+    gfloat* p = part + (int64_t)first * stride;
+    for (int j = threadIdx.x; j < 2 * a.D4; j += kNT) {
+      float s0, s1;
+      sum2(p + 2 * j, stride, members, s0, s1);
+      put2(p + 2 * j, s0, s1);
+    }
+  }
+  if (!arrive_last(a.counter, runs, &flag)) return;
 
   // Last block: combine the block records, add the prior, scale.
-  gcfloat* part = to_global(a.partial);
-  const int nb = gridDim.x;
   const float c = (float)(-a.N) / (float)a.n;
   float sl = 0.0f;
   for (int b = threadIdx.x; b < nb; b += kNT) sl += consume(part + (int64_t)b * stride + 4 * a.D4);
+  float lp = 0.0f;
+  for (int j2 = threadIdx.x; j2 < 2 * a.D4; j2 += kNT) {
+    float s[2];
+    sum2(part + 2 * j2, step, runs, s[0], s[1]);
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int j = 2 * j2 + e;
+      if (j >= a.D) break;
+      const float wj = a.theta[j];
+      float g = c * s[e];
+      if (a.pr.has_prior) {
+        g = g + wj * a.pr.inv_var;
+        lp += (a.pr.log_norm + (wj * wj) * a.pr.inv_var) / -2.0f;
+      }
+      a.out_grad[j] = g / a.temperature;
+    }
+  }
   const float sumlik = block_sum<kNT>(sl, lds_small);
   const float mean = sumlik / (float)a.n;
-  float lp = 0.0f;
-  for (int j = threadIdx.x; j < a.D; j += kNT) {
-    float s, unused;
-    sum_strided2(part + j, part + j, stride, nb, s, unused);
-    const float wj = a.theta[j];
-    float g = c * s;
-    if (a.pr.has_prior) {
-      g = g + wj * a.pr.inv_var;
-      lp += (a.pr.log_norm + (wj * wj) * a.pr.inv_var) / -2.0f;
-    }
-    a.out_grad[j] = g / a.temperature;
-  }
   lp = block_sum<kNT>(lp, lds_small);
   if (threadIdx.x == 0) a.out_U[0] = ((float)(-a.N) * mean - lp) / a.temperature;
   if (a.out_var) {
@@ -214,7 +264,7 @@ int launch_potential(const char* who, int family, const float* X, int64_t ldx, c
                      const int32_t* idx, int n, int64_t N, int D, const float* theta,
                      float sigma, int has_prior, float prior_scale, float temperature,
                      float* out_U, float* out_grad, float* out_lik, float* out_var,
-                     float* partial, unsigned* counter, int nblocks, void* stream) {
+                     float* partial, unsigned* counter, int group, int nblocks, void* stream) {
   SGMC_REQUIRE(X && y && theta && out_U && out_grad, SGMC_E_ARG, "%s: null pointer", who);
   SGMC_REQUIRE(family == SGMC_LIK_LINEAR_GAUSSIAN || family == SGMC_LIK_LOGISTIC, SGMC_E_ARG,
                "%s: unknown family %d", who, family);
@@ -239,6 +289,7 @@ int launch_potential(const char* who, int family, const float* X, int64_t ldx, c
   a.D4 = (D + 3) / 4;
   a.partial = partial;
   a.counter = counter;
+  a.group = group;
   a.ldx = ldx;
   a.N = N;
   a.n = n;
@@ -267,7 +318,7 @@ int launch_potential(const char* who, int family, const float* X, int64_t ldx, c
 // call leaves it at zero (the potential's last block resets it); the records are
 // written before they are read in every call.
 constexpr int64_t kScratchFloats = 1 << 18;
-constexpr int64_t kScratchCounterFloats = 64;
+constexpr int64_t kScratchCounterFloats = kPotCounters;
 constexpr int64_t kScratchRecordFloats = kScratchFloats - kScratchCounterFloats;
 constexpr int kScratchDevices = 64;
 static __device__ __align__(256) float scratch[kScratchFloats];
@@ -396,14 +447,19 @@ extern "C" {
 int64_t sgmc_glm_workspace_floats(int n, int D, int nblocks) {
   const int D4 = (D + 3) / 4;
   (void)n;
-  return (int64_t)nblocks * (4 * D4 + 2) + 4;
+  return (int64_t)nblocks * (4 * D4 + 2) + kPotCounters;
 }
 
+// One block per compute unit (two at 256 < D <= 512), each with at least one row group of its
+// four wavefronts. n = 40001, D = 301: 19.3 us at 507 blocks, 20.8 at 256; n = 60000,
+// D = 1000: 49.2 and 45.9; n = 20000, D = 100: 13.8 and 12.7; n = 60000, D = 64: 14.2 and
+// 13.2. (256 rows per block, whatever the size: 87.5, 270.7, 38.2 and 63.3 us.)
 int sgmc_glm_blocks(int n, int D) {
-  (void)D;
-  const int rows = 256;
-  int b = (n + rows - 1) / rows;
-  return b < 1 ? 1 : b;
+  const int blocks = D > 256 && D <= 512 ? 512 : 256;
+  const int least = D <= 16 ? 256 : D <= 32 ? 128 : D <= 64 ? 64 : 32;
+  const int rows = std::max(least, (int)(((int64_t)n + blocks - 1) / blocks));
+  const int b = (int)(((int64_t)n + rows - 1) / rows);
+  return std::max(b < 1 ? 1 : b, (int)(((int64_t)n + kLdsRows - 1) / kLdsRows));
 }
 
 int sgmc_glm_potential(int family, const float* X, int64_t ldx, const float* y,
@@ -414,13 +470,15 @@ int sgmc_glm_potential(int family, const float* X, int64_t ldx, const float* y,
   SGMC_REQUIRE(workspace, SGMC_E_ARG, "sgmc_glm_potential: null workspace");
   SGMC_REQUIRE(D >= 1 && D <= kMaxD && nblocks >= 1, SGMC_E_ARG,
                "sgmc_glm_potential: D=%d outside [1, %d] or nblocks=%d", D, kMaxD, nblocks);
-  SGMC_REQUIRE(workspace_floats >= sgmc_glm_workspace_floats(n, D, nblocks), SGMC_E_ARG,
-               "sgmc_glm_potential: workspace too small");
   const int64_t records = (int64_t)nblocks * (4 * ((D + 3) / 4) + 2);
+  SGMC_REQUIRE(workspace_floats >= records + 4, SGMC_E_ARG,
+               "sgmc_glm_potential: workspace too small");
+  // a workspace with room for one counter only reduces in one level
+  const int group = workspace_floats >= records + kPotCounters ? pot_group(nblocks) : 0;
   return launch_potential("sgmc_glm_potential", family, X, ldx, y, idx, n, N, D, theta, sigma,
                           has_prior, prior_scale, temperature, out_U, out_grad, out_lik,
                           out_var, workspace, reinterpret_cast<unsigned*>(workspace + records),
-                          nblocks, stream);
+                          group, nblocks, stream);
 }
 
 int sgmc_glm_potential_noalloc(int family, const float* X, int64_t ldx, const float* y,
@@ -442,7 +500,7 @@ int sgmc_glm_potential_noalloc(int family, const float* X, int64_t ldx, const fl
   return launch_potential("sgmc_glm_potential_noalloc", family, X, ldx, y, idx, n, N, D, theta,
                           sigma, has_prior, prior_scale, temperature, out_U, out_grad, out_lik,
                           out_var, base + kScratchCounterFloats,
-                          reinterpret_cast<unsigned*>(base), nblocks, stream);
+                          reinterpret_cast<unsigned*>(base), pot_group(nblocks), nblocks, stream);
 }
 
 int64_t sgmc_glm_full_workspace_doubles(int64_t N, int rows_per_block) {

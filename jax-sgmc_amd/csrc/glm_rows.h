@@ -377,16 +377,6 @@ __device__ __forceinline__ float col_sum(const float* lds_cols, int D4, int c) {
   return s;
 }
 
-// block_reduce with the column sums published to out[0..4*D4) for the chain's last block.
-template <int LPR, int CPL>
-__device__ __forceinline__ float block_reduce_write(float4 (&acc)[CPL], float lik_acc, int D4,
-                                                    gfloat* __restrict__ out, float* lds_cols,
-                                                    float* lds_small) {
-  const float lsum = block_reduce<LPR, CPL>(acc, lik_acc, D4, lds_cols, lds_small);
-  for (int c = threadIdx.x; c < 4 * D4; c += kNT) publish(out + c, col_sum(lds_cols, D4, c));
-  return lsum;
-}
-
 // Splits rows [0, n) of a minibatch among the blocks of a chain and then among the
 // wavefronts of a block (contiguous ranges).
 __device__ __forceinline__ void wave_rows(int n, int nblocks, int b, int& r0, int& r1,
