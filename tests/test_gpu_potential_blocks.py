@@ -71,3 +71,31 @@ def test_gather_rows(dtype, row, rows):
   L.call("sgmc_gather_rows", L.ptr(src), 1000, L.ptr(idx), L.ptr(out), rows, row * es, row * es,
          L.stream())
   assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("N,D,rows", [
+    (1, 1, 1), (3, 5, 128), (257, 17, 64), (1000, 64, 63), (1000, 96, 1000), (1003, 128, 100),
+    (2047, 129, 2048), (1500, 257, 129), (900, 511, 128), (700, 1000, 77), (530, 1024, 265)])
+@pytest.mark.parametrize("family", ["linear_gaussian", "logistic"])
+def test_full_potential_splits(N, D, rows, family):
+  """Blocks and wavefronts with fewer rows than a row group, with none, and row lengths at
+  the edges of the row classes: 1e-6 relative to the float64 oracle."""
+  print(family, N, D, rows, flush=True)
+  rng = np.random.default_rng(N + D)
+  X = (rng.standard_normal((N, D)) / np.sqrt(D)).astype(np.float32)
+  y = (rng.random(N) < 0.5).astype(np.float32)
+  w = (0.3 * rng.standard_normal(D)).astype(np.float32)
+  ld = (D + 3) // 4 * 4
+  Xp = np.full((N, ld), 9.0, np.float32)  # the padding is not read into the sums
+  Xp[:, :D] = X
+  Xd, yd, wd = (torch.as_tensor(v, device=DEV) for v in (Xp, y, w))
+  ws = torch.zeros(int(L.query("sgmc_glm_full_workspace_doubles", N, rows)), device=DEV,
+                   dtype=torch.float64)
+  out = torch.empty((), dtype=torch.float64, device=DEV)
+  fam = L.LIK_LOGISTIC if family == "logistic" else L.LIK_LINEAR_GAUSSIAN
+  for _ in range(2):
+    L.call("sgmc_glm_full_potential", fam, L.ptr(Xd), ld, L.ptr(yd), N, D, L.ptr(wd), 0.7, 1, 2.0,
+           1.5, L.ptr(out), L.ptr(ws), ws.numel(), rows, L.stream())
+    lik, _ = (om.logistic(w, X, y) if family == "logistic" else om.linear_gaussian(w, X, y, 0.7))
+    want = (-np.sum(lik) - om.gaussian_logprior(w, 2.0)[0]) / 1.5
+    assert abs(out.item() - want) <= 1e-6 * abs(want)
