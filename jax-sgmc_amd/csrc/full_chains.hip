@@ -20,6 +20,8 @@
 //   (blocks in order by the last block to arrive), so the result is deterministic.
 #include <math.h>
 
+#include <type_traits>
+
 #include "glm_common.h"
 #include "sgmc_common.h"
 #include "sgmc_device.h"
@@ -37,9 +39,6 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
-constexpr int kSpAhead = 2;     // 16-column k-blocks of A loads in flight (split kernel)
-constexpr int kSpLdsE = 4096;   // 16-byte Theta operand entries per half (64 KiB each)
-
 struct FcArgs {
   const float* X;
   const float* y;
@@ -50,12 +49,11 @@ struct FcArgs {
   int64_t ldx;
   int64_t ld_theta;
   int64_t N;
-  int64_t tiles;         // ceil(N / 64)
+  int64_t tiles;         // ceil(N / 64), split kernel: ceil(N / kTile)
   int D;
   int D4;                // ceil(D / 4): float4 columns of a row that may be read
   int D8r;               // ceil(D / 8) rounded up to kFcAhead
   int nchains;           // chains of this launch (<= 32 NT)
-  int D16r;              // split kernel: ceil(D / 16) rounded up to kSpAhead
   int x_exp;             // split kernel: X is scaled by 2^x_exp before splitting
   Lik L;
   Prior pr;
@@ -118,6 +116,44 @@ __device__ __forceinline__ float fam_lik(const Lik& L, float z, float y) {
   const float e = __builtin_amdgcn_exp2f(-fabsf(z) * kLog2e);
   const float sp = fmaxf(z, 0.0f) + __builtin_amdgcn_logf(1.0f + e) * kLn2;
   return y * z - sp;
+}
+
+// The last block: sums every chain's block records and forms U. Eight threads per chain
+// (64 chains of 512 threads) take every eighth block and prior term, then the eight sums are
+// added in order.
+__device__ __forceinline__ void finish_chains(const FcArgs& a, double (*red)[kFcChainsMax]) {
+  const int c = threadIdx.x % kFcChainsMax, sub = threadIdx.x / kFcChainsMax;
+  double tot = 0.0, lp = 0.0;
+  if (c < a.nchains) {
+    // sixteen records per memory round trip (missing ones add +0)
+    for (int b0 = sub; b0 < (int)gridDim.x; b0 += 16 * kFcWaves) {
+      double v[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int b = b0 + i * kFcWaves;
+        v[i] = consume(a.partial + (int64_t)min(b, (int)gridDim.x - 1) * kFcChainsMax + c);
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) tot += b0 + i * kFcWaves < (int)gridDim.x ? v[i] : 0.0;
+    }
+    if (a.pr.has_prior) {
+      const double iv = (double)a.pr.inv_var;
+      const double ln = (double)a.pr.log_norm;
+      const float* th = a.thetas + (int64_t)c * a.ld_theta;
+#pragma unroll 8
+      for (int k = sub; k < a.D; k += kFcWaves) {
+        const double wk = (double)th[k];
+        lp += (ln + wk * wk * iv) / -2.0;
+      }
+    }
+  }
+  __syncthreads();
+  red[sub][c] = -tot - lp;
+  __syncthreads();
+  if (threadIdx.x >= a.nchains) return;
+  double u = 0.0;
+  for (int v = 0; v < kFcWaves; ++v) u += red[v][threadIdx.x];
+  a.out_U[threadIdx.x] = u / a.temperature;
 }
 
 template <int NT, int FAM>
@@ -239,21 +275,7 @@ __global__ void __launch_bounds__(kFcThreads) glm_full_chains_kernel(FcArgs a) {
     publish(a.partial + (int64_t)blockIdx.x * kFcChainsMax + threadIdx.x, s);
   }
   if (!arrive_last(a.counter, gridDim.x, &flag)) return;
-  const int c = threadIdx.x;
-  if (c >= a.nchains) return;
-  double tot = 0.0;
-  for (int b = 0; b < (int)gridDim.x; ++b) tot += consume(a.partial + (int64_t)b * kFcChainsMax + c);
-  double lp = 0.0;
-  if (a.pr.has_prior) {
-    const double iv = (double)a.pr.inv_var;
-    const double ln = (double)a.pr.log_norm;
-    const float* th = a.thetas + (int64_t)c * a.ld_theta;
-    for (int k = 0; k < a.D; ++k) {
-      const double wk = (double)th[k];
-      lp += (ln + wk * wk * iv) / -2.0;
-    }
-  }
-  a.out_U[c] = (-tot - lp) / a.temperature;
+  finish_chains(a, lds_red);
 }
 
 // Split-fp16 variant. Each scaled value v = 2^e x (|v| < 2^14) becomes hi = f16(v) and
@@ -263,60 +285,58 @@ __global__ void __launch_bounds__(kFcThreads) glm_full_chains_kernel(FcArgs a) {
 // dropping lo_x lo_t (below 2^-20 of the product). The row dot products are then good
 // to about 1e-6 relative where float32 products give 6e-8, for a fifth of the
 // matrix-core time of v_mfma_f32_32x32x2_f32. X is read as float32 and split in
-// registers (splitting the dataset once into stored halves measured slower: the pass is
-// bound by memory latency, not by the conversions); X is scaled by the caller's 2^x_exp
-// (one exponent for the dataset), Theta per chain by 2^e_c from max |theta_c| over its
-// finite entries; z = acc 2^-(x_exp + e_c) is exact. Layout as in the float32 kernel
-// with 16-column k-blocks: lane l takes x[row + l % 32][16 j + 8 (l / 32) + 0..7] and
-// the Theta entry (j, t, l) holds Theta[32 t + l % 32][16 j + 8 (l / 32) + 0..7] as hi
-// and lo halves.
+// registers; X is scaled by the caller's 2^x_exp (one exponent for the dataset), Theta per
+// chain by 2^e_c from max |theta_c| over its finite entries; z = acc 2^-(x_exp + e_c) is
+// exact.
+//
+// Layout: the columns are shared out over S of a block's eight wavefronts (`per` k-blocks
+// of 16 columns each, at most KB), and S wavefronts together take a tile of 32 rows, 8 / S
+// tiles at a time. Theta's halves for a wavefront's columns stay in its registers for the
+// whole launch: lane l holds Theta[32 t + l % 32][16 j + 8 (l / 32) + 0..7] of k-block j and
+// chain tile t. X is loaded as it lies in memory, 256 bytes of four rows per instruction, and
+// turned into the A operand's order (x[row + l % 32][16 j + 8 (l / 32) + 0..7] on lane l)
+// through the wavefront's own 8 KiB of LDS, chunks swizzled by row against bank conflicts;
+// the loads of the next AHEAD steps are in flight while a tile is multiplied, across the
+// barrier too. (Loading operand order straight from memory touches every cache line with
+// four instructions of 32 lines each and stopped at 4.5 TB/s.) With S > 1 the wavefronts'
+// partial z go through the same LDS (double buffered, one barrier per step): wavefront w adds
+// the S partials of accumulator quads w, w + S, ... in order and applies the likelihood to
+// them. With Theta's operands in LDS instead (128 KiB, one block per unit, each
+// wavefront its own rows in operand order): N = 1e6, D = 512, 64 chains 521 -> 432 us, 20
+// chains 507 -> 347 (5.9 TB/s of X); N = 400000, D = 1000, 64 chains 1375 -> 615; N = 300007,
+// D = 90, 20 chains 107 -> 36; N = 5000 69 -> 14. At 64 chains the partials' LDS traffic and
+// the likelihoods add to the read; at D = 30 (74 us for 20 of rows) the likelihoods bound it.
+constexpr int kTile = 32;  // rows per tile
+
+// hi = f16(sc v), lo = f16(sc v - hi): sc is a power of two, so both are one rounding of an
+// exact value and one mixed-precision fused multiply-add each.
 __device__ __forceinline__ void split8(v4f a, v4f b, float sc, f16x8& hi, f16x8& lo) {
-  const float v[8] = {a.x * sc, a.y * sc, a.z * sc, a.w * sc,
-                      b.x * sc, b.y * sc, b.z * sc, b.w * sc};
+  const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const _Float16 h = (_Float16)v[i];
-    hi[i] = h;
-    lo[i] = (_Float16)(v[i] - (float)h);
-  }
+  for (int i = 0; i < 8; ++i) hi[i] = (_Float16)__builtin_fmaf(v[i], sc, 0.0f);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) lo[i] = (_Float16)__builtin_fmaf(v[i], sc, -(float)hi[i]);
 }
 
-template <int NT>
-__device__ __forceinline__ void mma_split(v16f (&acc)[2][NT], const v4f (&cur0)[kSpAhead][2],
-                                          const v4f (&cur1)[kSpAhead][2], const f16x8* lds_h,
-                                          const f16x8* lds_l, int jb, int lane, float xs) {
-#pragma unroll
-  for (int u = 0; u < kSpAhead; ++u) {
-    f16x8 ah0, al0, ah1, al1;
-    split8(cur0[u][0], cur0[u][1], xs, ah0, al0);
-    split8(cur1[u][0], cur1[u][1], xs, ah1, al1);
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      const int e = ((jb + u) * NT + t) * kWave + lane;
-      const f16x8 bh = lds_h[e];
-      const f16x8 bl = lds_l[e];
-      acc[0][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al0, bh, acc[0][t], 0, 0, 0);
-      acc[1][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al1, bh, acc[1][t], 0, 0, 0);
-      acc[0][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah0, bl, acc[0][t], 0, 0, 0);
-      acc[1][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah1, bl, acc[1][t], 0, 0, 0);
-      acc[0][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah0, bh, acc[0][t], 0, 0, 0);
-      acc[1][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah1, bh, acc[1][t], 0, 0, 0);
-    }
-  }
-}
-
-template <int NT, int FAM>
-__global__ void __launch_bounds__(kFcThreads) glm_full_chains_split_kernel(FcArgs a) {
-  __shared__ f16x8 lds_h[kSpLdsE];
-  __shared__ f16x8 lds_l[kSpLdsE];
+template <int KB, int S, int NT, int FAM>
+__global__ void __launch_bounds__(kFcThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
+glm_full_chains_split_kernel(FcArgs a) {
+  constexpr int kGroups = kFcWaves / S;       // tiles of a block at a time
+  // A tile is loaded and multiplied in steps of up to four k-blocks; AHEAD steps of loads
+  // are in flight (as the registers beside Theta's allow).
+  constexpr int KL = 4, kSteps = KB / KL;
+  constexpr int AHEAD = 2;
+  constexpr int kSlots = S > 1 ? 2 : 1;
+  __shared__ v4f part[kSlots][kFcWaves][kTile * 16];
   __shared__ double lds_red[kFcWaves][kFcChainsMax];
   __shared__ float lds_sc[kFcChainsMax];
   __shared__ float lds_inv[kFcChainsMax];
   __shared__ int flag;
   const int lane = threadIdx.x & (kWave - 1);
-  const int w = threadIdx.x / kWave;
+  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
   const int rsub = lane & 31;
   const int q = lane >> 5;
+  const int grp = w / S, wp = w % S;
 
   // Per-chain exponent: eight threads per chain find max |theta_c| over finite entries.
   {
@@ -324,9 +344,13 @@ __global__ void __launch_bounds__(kFcThreads) glm_full_chains_split_kernel(FcArg
     float m = 0.0f;
     if (c < a.nchains) {
       const float* th = a.thetas + (int64_t)c * a.ld_theta;
-      for (int k = sub; k < a.D; k += 8) {
-        const float v = fabsf(th[k]);
-        if (v <= 3.0e38f) m = fmaxf(m, v);
+      for (int k0 = sub; k0 < a.D; k0 += 64) {
+        float v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = fabsf(th[min(k0 + 8 * i, a.D - 1)]);
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          if (v[i] <= 3.0e38f) m = fmaxf(m, v[i]);
       }
     }
     m = fmaxf(m, __shfl_xor(m, 1, kWave));
@@ -342,117 +366,189 @@ __global__ void __launch_bounds__(kFcThreads) glm_full_chains_split_kernel(FcArg
   }
   __syncthreads();
 
-  // Theta operands, every load of the thread issued before the first LDS store.
-  const int entries = a.D16r * NT * kWave;
-  constexpr int kPer = kSpLdsE / kFcThreads;
-  f16x8 sh[kPer], sl[kPer];
+  // This wavefront's k-blocks j0 .. j0 + nk - 1 and their Theta operands.
+  const int D16 = (a.D + 15) / 16;
+  const int per = (D16 + S - 1) / S;  // <= KB
+  const int j0 = wp * per;
+  const int nk = max(0, min(per, D16 - j0));
+  f16x8 bh[KB][NT], bl[KB][NT];
 #pragma unroll
-  for (int i = 0; i < kPer; ++i) {
-    const int e = threadIdx.x + i * kFcThreads;
-    const int l = e % kWave;
-    const int t = (e / kWave) % NT;
-    const int j = e / (kWave * NT);
-    const int c = 32 * t + (l & 31);
-    const int k0 = 16 * j + 8 * (l >> 5);
-    const bool live = e < entries && c < a.nchains;
+  for (int t = 0; t < NT; ++t) {
+    const int c = 32 * t + rsub;
+    const bool live = c < a.nchains;
     const float* src = a.thetas + (int64_t)(live ? c : 0) * a.ld_theta;
     const float sc = lds_sc[c];
-    float v[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const bool ok = live && k0 + u < a.D;
-      const float x = src[ok ? k0 + u : 0];
-      v[u] = ok ? x * sc : 0.0f;
-    }
+    for (int u = 0; u < KB; ++u) {
+      const int k0 = 16 * (j0 + u) + 8 * q;
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const _Float16 h = (_Float16)v[u];
-      sh[i][u] = h;
-      sl[i][u] = (_Float16)(v[u] - (float)h);
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < kPer; ++i) {
-    const int e = threadIdx.x + i * kFcThreads;
-    if (e < entries) {
-      lds_h[e] = sh[i];
-      lds_l[e] = sl[i];
+      for (int i = 0; i < 8; ++i) {
+        const bool ok = live && u < nk && k0 + i < a.D;
+        const float x = src[ok ? k0 + i : 0];
+        const float v = ok ? x * sc : 0.0f;
+        const _Float16 h = (_Float16)v;
+        bh[u][t][i] = h;
+        bl[u][t][i] = (_Float16)(v - (float)h);
+      }
     }
   }
-  __syncthreads();
-
   const float xs = ldexpf(1.0f, a.x_exp);
   float inv[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) inv[t] = lds_inv[32 * t + rsub];
+  // Tiles of the block, dealt to its groups in turn; every group makes `turns` passes (the
+  // barriers are the block's), the last ones on tiles past t1 whose rows count for nothing.
   const int64_t t0 = (int64_t)blockIdx.x * a.tiles / gridDim.x;
   const int64_t t1 = (int64_t)(blockIdx.x + 1) * a.tiles / gridDim.x;
+  const int turns = (int)((t1 - t0 + kGroups - 1) / kGroups);
   double sacc[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) sacc[t] = 0.0;
 
-  for (int64_t tile = t0 + w; tile < t1; tile += kFcWaves) {
-    const int64_t r0 = tile * 64 + rsub;
-    const int64_t r1 = r0 + 32;
-    const bool ok0 = r0 < a.N, ok1 = r1 < a.N;
-    const float* x0 = a.X + (ok0 ? r0 : 0) * a.ldx;
-    const float* x1 = a.X + (ok1 ? r1 : 0) * a.ldx;
-    v16f acc[2][NT];
+  // Instruction i of a step loads rows 4 i + l / 16 of the tile, lane l the 16-byte chunk
+  // c = (l % 16) ^ (row % 16) of the wavefront's 16 (its LDS place is then l % 16), through a
+  // buffer resource that begins at the tile and ends with the data: rows past N read as
+  // zero, and chunks that are not the wavefront's or not the row's lie past its end (kOut).
+  constexpr uint32_t kOut = 0x80000000u;
+  v4f x[AHEAD][8];
+  const int lrow = lane >> 4;
+  uint32_t voff[kSteps][4];
 #pragma unroll
-    for (int g = 0; g < 2; ++g)
+  for (int h = 0; h < kSteps; ++h)
 #pragma unroll
-      for (int t = 0; t < NT; ++t) acc[g][t] = v16f{};
-    v4f cur0[kSpAhead][2], cur1[kSpAhead][2];
-#pragma unroll
-    for (int u = 0; u < kSpAhead; ++u)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        cur0[u][h] = load_x4(x0, 4 * u + 2 * q + h, ok0, a.D4);
-        cur1[u][h] = load_x4(x1, 4 * u + 2 * q + h, ok1, a.D4);
-      }
-    const int jlast = a.D16r - kSpAhead;
-    for (int jb = 0; jb < jlast; jb += kSpAhead) {
-      v4f nxt0[kSpAhead][2], nxt1[kSpAhead][2];
-#pragma unroll
-      for (int u = 0; u < kSpAhead; ++u)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int c4 = 4 * (jb + kSpAhead + u) + 2 * q + h;
-          nxt0[u][h] = load_x4(x0, c4, ok0, a.D4);
-          nxt1[u][h] = load_x4(x1, c4, ok1, a.D4);
-        }
-      mma_split<NT>(acc, cur0, cur1, lds_h, lds_l, jb, lane, xs);
-#pragma unroll
-      for (int u = 0; u < kSpAhead; ++u)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          cur0[u][h] = nxt0[u][h];
-          cur1[u][h] = nxt1[u][h];
-        }
+    for (int i = 0; i < 4; ++i) {
+      const int c = (lane & 15) ^ (4 * i + lrow);
+      const int c4 = 4 * (j0 + KL * h) + c;
+      voff[h][i] = c < 4 * (nk - KL * h) && c4 < a.D4
+                       ? (uint32_t)(lrow * a.ldx + 4 * c4) * 4u : kOut;
     }
-    float yv[2][16];
+  const uint32_t row4 = (uint32_t)(16 * a.ldx);  // bytes of four rows
+  auto resource = [&](const float* base, int64_t left) __attribute__((always_inline)) {
+    const int64_t bytes = max((int64_t)0, min(4 * left, (int64_t)0x7FFFFFFF));
+    return __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, (int)bytes, 0x00020000);
+  };
+  auto load = [&](int step, auto hh, v4f (&buf)[8]) __attribute__((always_inline)) {
+    constexpr int H = decltype(hh)::value;
+    const int64_t row0 = (t0 + (int64_t)(step / kSteps) * kGroups + grp) * kTile;
+    const auto rs = resource(a.X + min(row0, a.N) * a.ldx, (a.N - row0) * a.ldx);
 #pragma unroll
-    for (int g = 0; g < 2; ++g)
+    for (int i = 0; i < 8; ++i)
+      buf[i] = __builtin_bit_cast(
+          v4f, __builtin_amdgcn_raw_buffer_load_b128(rs, voff[H][i & 3] + i * row4, 0, 0));
+  };
+  // likelihood of accumulator quad qd (rows 8 (qd % 4) + 4 q + 0..3, chain tile qd / 4)
+  auto count = [&](int64_t tile, int qd, int t, const float (&z)[4], v4f yv)
+                   __attribute__((always_inline)) {
+    const bool whole = tile < t1 && tile * kTile + kTile <= a.N;  // uniform
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int64_t row = tile * 64 + 32 * g + 8 * (r / 4) + 4 * q + (r % 4);
-        yv[g][r] = a.y[row < a.N ? row : a.N - 1];
-      }
-    mma_split<NT>(acc, cur0, cur1, lds_h, lds_l, jlast, lane, xs);
+    for (int i = 0; i < 4; ++i) {
+      const double lik = (double)fam_lik<FAM>(a.L, z[i] * inv[t], yv[i]);
+      if (whole) sacc[t] += lik;
+      else sacc[t] += tile < t1 && tile * kTile + 8 * (qd % 4) + 4 * q + i < a.N ? lik : 0.0;
+    }
+  };
+  constexpr int kQuads = S >= 4 * NT ? 1 : 4 * NT / S;  // per wavefront
+  v16f acc[NT];
+  v4f yv[kQuads];
+  const bool ragged = (a.D & 3) != 0 && nk > 0 && j0 + nk == D16;  // uniform
+  // step `step` (its place H in the tile static); its loads are in cur, which then takes
+  // those of step + AHEAD
+  auto step_of = [&](int step, auto hh, v4f (&cur)[8]) __attribute__((always_inline)) {
+    constexpr int H = decltype(hh)::value;
+    const int turn = step / kSteps;
+    const int64_t tile = t0 + (int64_t)turn * kGroups + grp;
+    v4f* mine = part[step & (kSlots - 1)][w];
+    if (ragged) {
+      // columns past D in the row's last chunk: a scaled padding value could overflow fp16,
+      // and inf times Theta's zero is NaN
 #pragma unroll
-    for (int g = 0; g < 2; ++g)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int64_t row = tile * 64 + 32 * g + 8 * (r / 4) + 4 * q + (r % 4);
-        const bool ok = row < a.N;
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-          const float lik = fam_lik<FAM>(a.L, acc[g][t][r] * inv[t], yv[g][r]);
-          sacc[t] += ok ? (double)lik : 0.0;
+      for (int i = 0; i < 8; ++i) {
+        const int c = (lane & 15) ^ ((4 * i + lrow) & 15);
+        if (4 * (j0 + KL * H) + c == a.D4 - 1) {
+          if ((a.D & 3) == 1) cur[i].y = 0.0f;
+          if ((a.D & 3) <= 2) cur[i].z = 0.0f;
+          cur[i].w = 0.0f;
         }
       }
-  }
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) mine[i * kWave + lane] = cur[i];
+    load(step + AHEAD, std::integral_constant<int, (H + AHEAD) % kSteps>{}, cur);
+    __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of the products
+    if (H == 0) {
+      const int64_t row0 = tile * kTile;
+      const auto ys = resource(a.y + min(row0, a.N), a.N - row0);
+#pragma unroll
+      for (int i = 0; i < kQuads; ++i)
+        yv[i] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(
+                                            ys, 32 * ((wp + i * S) % 4) + 16 * q, 0, 0));
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[t] = v16f{};
+    }
+#pragma unroll
+    for (int u = 0; u < KL; ++u) {
+      if (KL * H + u >= nk) break;
+      f16x8 ah, al;
+      const int c = 4 * u + 2 * q, r = rsub & 15;
+      split8(mine[rsub * 16 + (c ^ r)], mine[rsub * 16 + ((c + 1) ^ r)], xs, ah, al);
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, bh[KL * H + u][t], acc[t], 0, 0, 0);
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bl[KL * H + u][t], acc[t], 0, 0, 0);
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bh[KL * H + u][t], acc[t], 0, 0, 0);
+    }
+    if constexpr (H < kSteps - 1) {
+      if (S > 1) lds_sync();  // the slot's partials of the tile before have been read
+      return;
+    }
+    if constexpr (S == 1) {
+#pragma unroll
+      for (int qd = 0; qd < 4 * NT; ++qd) {
+        const float z[4] = {acc[qd / 4][4 * (qd % 4)], acc[qd / 4][4 * (qd % 4) + 1],
+                            acc[qd / 4][4 * (qd % 4) + 2], acc[qd / 4][4 * (qd % 4) + 3]};
+        count(tile, qd, qd / 4, z, yv[qd]);
+      }
+    } else {
+      auto& buf = part[step & 1];
+#pragma unroll
+      for (int qd = 0; qd < 4 * NT; ++qd)
+        mine[qd * kWave + lane] = v4f{acc[qd / 4][4 * (qd % 4)], acc[qd / 4][4 * (qd % 4) + 1],
+                                      acc[qd / 4][4 * (qd % 4) + 2], acc[qd / 4][4 * (qd % 4) + 3]};
+      lds_sync();  // what this slot is used for next lies behind the next step's barrier
+#pragma unroll
+      for (int i = 0; i < kQuads; ++i) {
+        const int qd = wp + i * S;
+        if (qd >= 4 * NT) break;
+        v4f s = buf[grp * S][qd * kWave + lane];
+#pragma unroll
+        for (int v = 1; v < S; ++v) s += buf[grp * S + v][qd * kWave + lane];
+        const float z[4] = {s.x, s.y, s.z, s.w};
+        // (the chain tile of quad wp + i S; uniform, a register index needs it static)
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+          if (qd / 4 == t) count(tile, qd, t, z, yv[i]);
+      }
+    }
+  };
+  static_assert(AHEAD == 2, "the two steps below");
+  load(0, std::integral_constant<int, 0>{}, x[0]);
+  load(1, std::integral_constant<int, 1 % kSteps>{}, x[1]);
+  // AHEAD kSteps steps per round, so that buffers and places in the tile are static
+  const int steps = turns * kSteps;
+  auto round = [&](int base, auto self, auto bb) __attribute__((always_inline)) {
+    constexpr int B = decltype(bb)::value;
+    if (base + B < steps)
+      step_of(base + B, std::integral_constant<int, B % kSteps>{}, x[B % AHEAD]);
+    if constexpr (B + 1 < AHEAD * kSteps) self(base, self, std::integral_constant<int, B + 1>{});
+  };
+  for (int base = 0; base < steps; base += AHEAD * kSteps)
+    round(base, round, std::integral_constant<int, 0>{});
 
+  // Lanes l and l ^ 32 hold the same chain; then waves in order; then blocks.
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     sacc[t] += __shfl_xor(sacc[t], 32, kWave);
@@ -465,21 +561,7 @@ __global__ void __launch_bounds__(kFcThreads) glm_full_chains_split_kernel(FcArg
     publish(a.partial + (int64_t)blockIdx.x * kFcChainsMax + threadIdx.x, sum);
   }
   if (!arrive_last(a.counter, gridDim.x, &flag)) return;
-  const int c = threadIdx.x;
-  if (c >= a.nchains) return;
-  double tot = 0.0;
-  for (int b = 0; b < (int)gridDim.x; ++b) tot += consume(a.partial + (int64_t)b * kFcChainsMax + c);
-  double lp = 0.0;
-  if (a.pr.has_prior) {
-    const double iv = (double)a.pr.inv_var;
-    const double ln = (double)a.pr.log_norm;
-    const float* th = a.thetas + (int64_t)c * a.ld_theta;
-    for (int k = 0; k < a.D; ++k) {
-      const double wk = (double)th[k];
-      lp += (ln + wk * wk * iv) / -2.0;
-    }
-  }
-  a.out_U[c] = (-tot - lp) / a.temperature;
+  finish_chains(a, lds_red);
 }
 
 }  // namespace
@@ -488,6 +570,31 @@ __global__ void __launch_bounds__(kFcThreads) glm_full_chains_split_kernel(FcArg
 using namespace sgmc;
 
 namespace {
+
+// The wavefronts that share a row's columns: as few as hold them in KB = 4 k-blocks of
+// registers each; all eight with 8 k-blocks each (and one chain tile) beyond 512 columns.
+template <int FAM>
+void launch_split(dim3 grid, hipStream_t s, const FcArgs& a, int D16, bool two) {
+  const dim3 block(kFcThreads);
+#define SGMC_SPLIT(KB, S, NT) \
+  hipLaunchKernelGGL((glm_full_chains_split_kernel<KB, S, NT, FAM>), grid, block, 0, s, a)
+  if (D16 <= 4) {
+    if (two) SGMC_SPLIT(4, 1, 2);
+    else SGMC_SPLIT(4, 1, 1);
+  } else if (D16 <= 8) {
+    if (two) SGMC_SPLIT(4, 2, 2);
+    else SGMC_SPLIT(4, 2, 1);
+  } else if (D16 <= 16) {
+    if (two) SGMC_SPLIT(4, 4, 2);
+    else SGMC_SPLIT(4, 4, 1);
+  } else if (D16 <= 32) {
+    if (two) SGMC_SPLIT(4, 8, 2);
+    else SGMC_SPLIT(4, 8, 1);
+  } else {
+    SGMC_SPLIT(8, 8, 1);
+  }
+#undef SGMC_SPLIT
+}
 
 int launch_full_chains(const char* name, bool split, int x_exp, int family, const float* X,
                        int64_t ldx, const float* y, int64_t N, int D, const float* thetas,
@@ -514,22 +621,21 @@ int launch_full_chains(const char* name, bool split, int x_exp, int family, cons
   a.ldx = ldx;
   a.ld_theta = ld_theta;
   a.N = N;
-  a.tiles = (N + 63) / 64;
+  a.tiles = split ? (N + kTile - 1) / kTile : (N + 63) / 64;
   a.D = D;
   a.D4 = (D + 3) / 4;
   const int D8 = (D + 7) / 8;
   a.D8r = (D8 + kFcAhead - 1) / kFcAhead * kFcAhead;
   const int D16 = (D + 15) / 16;
-  a.D16r = (D16 + kSpAhead - 1) / kSpAhead * kSpAhead;
   a.x_exp = x_exp;
   a.L = make_lik(family, sigma);
   a.pr = make_prior(has_prior, prior_scale);
   a.temperature = temperature;
   a.partial = workspace;
   a.counter = reinterpret_cast<unsigned*>(workspace + (int64_t)nblocks * kFcChainsMax);
-  // Two chain tiles per pass when their operands fit the LDS, else one.
-  const int nt = split ? ((a.D16r * 2 * kWave <= kSpLdsE) ? 2 : 1)
-                       : ((a.D8r * 2 * kWave <= kFcLdsF4) ? 2 : 1);
+  // Two chain tiles per pass when their operands fit the LDS (split: the registers), else
+  // one.
+  const int nt = split ? (D16 <= 32 ? 2 : 1) : ((a.D8r * 2 * kWave <= kFcLdsF4) ? 2 : 1);
   hipStream_t s = as_stream(stream);
   const dim3 grid(nblocks), block(kFcThreads);
   for (int c0 = 0; c0 < nchains; c0 += 32 * nt) {
@@ -539,13 +645,8 @@ int launch_full_chains(const char* name, bool split, int x_exp, int family, cons
     const bool two = a.nchains > 32;
     const bool lg = family == SGMC_LIK_LOGISTIC;
     if (split) {
-      if (lg) {
-        if (two) hipLaunchKernelGGL((glm_full_chains_split_kernel<2, SGMC_LIK_LOGISTIC>), grid, block, 0, s, a);
-        else hipLaunchKernelGGL((glm_full_chains_split_kernel<1, SGMC_LIK_LOGISTIC>), grid, block, 0, s, a);
-      } else {
-        if (two) hipLaunchKernelGGL((glm_full_chains_split_kernel<2, SGMC_LIK_LINEAR_GAUSSIAN>), grid, block, 0, s, a);
-        else hipLaunchKernelGGL((glm_full_chains_split_kernel<1, SGMC_LIK_LINEAR_GAUSSIAN>), grid, block, 0, s, a);
-      }
+      if (lg) launch_split<SGMC_LIK_LOGISTIC>(grid, s, a, D16, two);
+      else launch_split<SGMC_LIK_LINEAR_GAUSSIAN>(grid, s, a, D16, two);
     } else {
       if (lg) {
         if (two) hipLaunchKernelGGL((glm_full_chains_kernel<2, SGMC_LIK_LOGISTIC>), grid, block, 0, s, a);

@@ -99,3 +99,38 @@ def test_full_potential_splits(N, D, rows, family):
     lik, _ = (om.logistic(w, X, y) if family == "logistic" else om.linear_gaussian(w, X, y, 0.7))
     want = (-np.sum(lik) - om.gaussian_logprior(w, 2.0)[0]) / 1.5
     assert abs(out.item() - want) <= 1e-6 * abs(want)
+
+
+@pytest.mark.parametrize("N,D,C", [
+    (1, 1, 1), (31, 16, 3), (33, 17, 33), (700, 64, 64), (701, 65, 32), (1000, 90, 20),
+    (1023, 128, 40), (1000, 129, 7), (999, 256, 64), (650, 257, 33), (640, 300, 64),
+    (1300, 511, 65), (900, 512, 64), (777, 513, 20), (500, 1000, 70), (320, 1024, 33)])
+def test_full_potential_of_chains_splits(N, D, C):
+  """The split-fp16 full potential at the edges of its column shares (64, 128, 256, 512
+  columns over 1, 2, 4 and 8 wavefronts), chain tiles and row tiles, with blocks without rows:
+  2e-6 relative to float64 (1e-6 per row dot product). Padding beyond D holds large values."""
+  print(N, D, C, flush=True)
+  rng = np.random.default_rng(N + D + C)
+  X = (rng.standard_normal((N, D)) / np.sqrt(D)).astype(np.float32)
+  y = (rng.random(N) < 0.5).astype(np.float32)
+  ld = (D + 3) // 4 * 4 + 4
+  Xp = np.full((N, ld), 5.0, np.float32)
+  Xp[:, :D] = X
+  th = (0.5 * rng.standard_normal((C, D))).astype(np.float32)
+  Xd, yd = torch.as_tensor(Xp, device=DEV), torch.as_tensor(y, device=DEV)
+  thd = torch.as_tensor(th, device=DEV)
+  exp = 14 - int(np.frexp(np.abs(X).max())[1])
+  nb = 37
+  ws = torch.zeros(int(L.query("sgmc_glm_full_chains_workspace_doubles", nb)), device=DEV,
+                   dtype=torch.float64)
+  out = torch.empty(C, dtype=torch.float64, device=DEV)
+  z = X.astype(np.float64) @ th.astype(np.float64).T
+  for fam, lik in ((L.LIK_LOGISTIC, y[:, None] * z - np.logaddexp(0, z)),
+                   (L.LIK_LINEAR_GAUSSIAN,
+                    (np.log(2 * np.pi * 0.49) + (y[:, None] - z) ** 2 / 0.49) / -2.0)):
+    L.call("sgmc_glm_full_potential_chains_split", fam, L.ptr(Xd), ld, L.ptr(yd), N, D, L.ptr(thd),
+           D, C, 0.7, 1, 2.0, 1.5, exp, L.ptr(out), L.ptr(ws), ws.numel(), nb, L.stream())
+    got = out.cpu().numpy()
+    for c in range(C):
+      want = (-np.sum(lik[:, c]) - om.gaussian_logprior(th[c], 2.0)[0]) / 1.5
+      assert abs(got[c] - want) <= 2e-6 * abs(want), (fam, c, got[c], want)
