@@ -36,36 +36,15 @@
 
 #include <type_traits>
 
-#include "sgmc_common.h"
-#include "sgmc_device.h"
+#include "mlp_common.h"
 
 namespace sgmc {
 namespace mlp {
 
-typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
-typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16;
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-// GEMM operand precision (template argument) and its element bytes.
-enum Prec { P_BF16 = 0, P_FP8 = 1, P_F32 = 2 };
-template <int PREC>
-constexpr int elem_bytes() {
-  return PREC == P_FP8 ? 1 : PREC == P_BF16 ? 2 : 4;
-}
-
-constexpr int GT = 256;
-constexpr int BM = 64;
-constexpr int BN = 128;
-constexpr int NCLS = 10;
-constexpr int NLEAF = 6;     // W1, W2, W3, b1, b2, b3
-constexpr int kStrip = 32;   // rows per partial sum of the small leaves' gradients
-constexpr int kXcds = 8;         // accelerator complex dies, each with its own L2
 #ifndef SGMC_GATHER_BATCH
 #define SGMC_GATHER_BATCH 12
 #endif
 constexpr int kGatherBatch = SGMC_GATHER_BATCH;  // float4 row loads in flight per lane
-constexpr int kFinalBlocks = 64;
 // Update epilogue tuning: parameters pairs per prefetch chunk (1, 2, 4 or 8 of a lane's
 // 16 pairs) and the waves per SIMD the update GEMMs are compiled for (register budget).
 #ifndef SGMC_UPD_CHUNK
@@ -84,132 +63,6 @@ static_assert(16 % kUpdChunk == 0, "chunks of the 16 pairs");
 // run-time rule of the OBABO updates loses a wave with them)
 constexpr int kUpdChunkDeep = 4;
 static_assert(16 % kUpdChunkDeep == 0, "chunks of the 16 pairs");
-
-__device__ __forceinline__ uint16_t f2bf(float f) {
-  uint32_t u = __float_as_uint(f);
-  u += 0x7FFFu + ((u >> 16) & 1u);
-  return (uint16_t)(u >> 16);
-}
-__device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
-
-// OCP fp8 e4m3 with a per-tensor scale: q = e4m3(clamp(v * scale, +-448)), v = q / scale.
-__device__ __forceinline__ uint8_t f2q(float v) {
-  v = fminf(fmaxf(v, -448.0f), 448.0f);
-  return (uint8_t)(__builtin_amdgcn_cvt_pk_fp8_f32(v, v, 0, false) & 0xFFu);
-}
-__device__ __forceinline__ float q2f(uint8_t b) { return __builtin_amdgcn_cvt_f32_fp8((int)b, 0); }
-
-// fp8 tensors and their per-chain scale words: scales [0, 6), the scale the next weight
-// shadows are written with [6, 8), amax bit patterns [8, 14).
-enum Q8 { Q_X = 0, Q_H1 = 1, Q_DA2 = 2, Q_DA1 = 3, Q_W1 = 4, Q_W2 = 5 };
-constexpr int kQWords = 16;
-constexpr float kQTarget = 224.0f;  // scale = kQTarget / amax: half the e4m3 range as headroom
-
-enum Epi { EPI_BIAS_RELU = 0, EPI_MASK = 1, EPI_UPDATE = 2, EPI_GRAD = 3, EPI_PARTIAL = 4 };
-
-// Per-chain state and step parameters shared by the kernels.
-struct Step {
-  const float* X;          // dataset [N][ldx] float32
-  const int32_t* labels;   // [N]
-  int64_t N, ldx;
-  int D_in, H1, H2, n, C;
-  float* theta;            // [C][P]
-  float* v;                // [C][P] or null (rms_prop)
-  uint16_t* shadow;        // [C][P] bf16 (null for float32 GEMMs)
-  int64_t P;
-  int64_t off[NLEAF];      // leaf offsets
-  int64_t size[NLEAF];     // leaf sizes
-  uint32_t* key;           // [C][2]
-  uint32_t* dkey;          // [C][2]
-  uint32_t* lkey;          // [C][NLEAF][2] noise keys of this update, written by the gather
-  uint32_t rmult, rmagic;  // randint_mult(N), randint_magic(N) of the index draw
-  // activations: bf16; e4m3 except h2 (bf16) in fp8 mode; float32 in fp32 mode
-  void* Xb;                // [C][n][D_in]
-  int32_t* lab;            // [C][n]
-  void* h1;                // [C][n][H1]
-  void* h2;                // [C][n][H2]
-  void* da2;               // [C][n][H2]
-  void* da1;               // [C][n][H1]
-  float* dL;               // [C][n][10]
-  float* lik;              // [C][n]
-  float* prior_part;       // [C][nparts]
-  int nparts;
-  float* U;                // [C]
-  float* grad;             // [C][P] (gradient-only mode) or null
-  float* samples;          // [C][n_slots][P] or null
-  float* samples_U;        // [C][n_slots] or null
-  int n_slots;
-  const float* eps_table;
-  const int32_t* save_slot;
-  int32_t* iter;
-  unsigned* counters;      // [C] arrival counters of the small kernel
-  unsigned* done;
-  int table_len;
-  int rms;
-  int update;              // 0: gradient only (autograd backward)
-  float alpha, lmbd, temperature, noise_temperature;
-  float prior_inv_var, prior_log_norm;
-  int has_prior;
-  // OBABO (update != 0, mode != MLP_SGLD)
-  int mode;
-  float* mom;              // [C][P] momentum
-  float* ke_part;          // [C][nparts] kinetic-energy partials of one evaluation
-  float* col_part;         // [C][n / kStrip][small leaves] row-strip gradient partials
-  double* fin_part;        // [C][kFinalBlocks] log-prior partials of the full pass
-  float* split_part;       // split-K partial products of the forward GEMMs
-  double* ke;              // [C][2] accumulated kinetic energy at start / end
-  float* U_half;           // [C] potential of the step's first evaluation
-  const float* decay_table;  // [table_len] sqrt(exp(-friction eps))
-  const float* noise_table;  // [table_len] sqrt((1 - exp(-friction eps)) T)
-  // full-data forward pass (likelihoods of rows row0 .. row0 + n - 1 only)
-  int full;
-  int64_t row0;
-  // fp8 GEMM operands (Xb, h1, da2, da1 and the W1 / W2 shadows in e4m3)
-  int fp8;
-  int fp32;                // float32 activations and GEMM operands (weights from theta)
-  int plan[5];             // per GEMM (G1..G5): 16 k-tile + split-K factor
-  float* q;                // [C][kQWords]
-  uint8_t* shadow8;        // [C][P] (W1 and W2 leaves)
-};
-
-// Records max |v| of a wavefront for tensor t of chain c (every lane of the wavefront
-// calls this). The atomic is skipped when the recorded maximum already covers the
-// wavefront's: thousands of wavefronts updating one word otherwise serialize at the L2.
-// A stale read is never above the true maximum, so no needed update is skipped.
-__device__ __forceinline__ void q_note_amax(const Step& s, int c, int t, float a) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) a = fmaxf(a, __shfl_xor(a, m, kWave));
-  if ((threadIdx.x & (kWave - 1)) == 0 && a > 0.0f) {
-    unsigned* slot = reinterpret_cast<unsigned*>(s.q + (int64_t)c * kQWords + 8 + t);
-    const unsigned cur = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (__float_as_uint(a) > cur) atomicMax(slot, __float_as_uint(a));
-  }
-}
-
-// Block-wide version (every thread of the block calls it): one check and at most one
-// atomic per block, for kernels whose wavefronts are too short to carry their own.
-__device__ __forceinline__ void q_note_amax_block(const Step& s, int c, int t, float a,
-                                                  float* red) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) a = fmaxf(a, __shfl_xor(a, m, kWave));
-  if ((threadIdx.x & (kWave - 1)) == 0) red[threadIdx.x / kWave] = a;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    float b = red[0];
-    for (int i = 1; i < (int)(blockDim.x / kWave); ++i) b = fmaxf(b, red[i]);
-    if (b > 0.0f) {
-      unsigned* slot = reinterpret_cast<unsigned*>(s.q + (int64_t)c * kQWords + 8 + t);
-      const unsigned cur = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (__float_as_uint(b) > cur) atomicMax(slot, __float_as_uint(b));
-    }
-  }
-}
-
-enum MlpMode { MLP_SGLD = 0, MLP_OBABO_BA = 1, MLP_OBABO_BO = 2 };
-
-__device__ __forceinline__ int cur_iter(const Step& s) {
-  return max(0, min(s.iter[0], s.table_len - 1));
-}
 
 // Gradient-only variant: grad = (gsum + prior) / T, no update.
 __device__ __forceinline__ void grad_param(const Step& s, const float* th, float* gout,
@@ -515,30 +368,6 @@ __global__ void __launch_bounds__(GT) gather_kernel(Step s) {
   if (lane == 0) s.lab[row] = valid ? s.labels[r] : -1;
 }
 
-// ------------------------------------------------------------------ GEMM ------
-// Operands are bf16, e4m3 (P_FP8) with per-tensor scales, or float32 (P_F32): element
-// pointers are byte addresses of 2-, 1- or 4-byte elements, strides are in elements.
-struct Gemm {
-  const void* A;
-  int64_t lda, sA;   // sA: chain stride in elements
-  const void* B;
-  int64_t ldb, sB;
-  int M, N, K;
-  void* out;         // EPI_BIAS_RELU / EPI_MASK
-  int64_t ldo, sO;
-  const float* bias; // chain-strided by sBias
-  int64_t sBias;
-  const void* mask;  // EPI_MASK: ReLU activations (same format as the operands)
-  int64_t ldm, sM;
-  int leaf;          // EPI_UPDATE / EPI_GRAD: parameter leaf of the [M][N] weight
-  int part0;         // first prior-partial slot of this GEMM
-  int splits;        // split-K factor (grid z = chains x splits)
-  float* part;       // EPI_PARTIAL: [splits][C][M][N] float32 partial products
-  int C;
-  int ta, tb;        // P_FP8: scale slots of A and B
-  int tout;          // P_FP8: scale slot of an e4m3 output, or -1 for a bf16 output
-};
-
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
 // ---- operand tiles in LDS ----
@@ -705,32 +534,6 @@ __device__ __forceinline__ void mfma_step(const uint8_t* As, const uint8_t* Bs, 
   }
 }
 
-// ReLU mask of an activation element (bf16, e4m3 or float32): positive and nonzero.
-template <int PREC>
-__device__ __forceinline__ bool mask_on(const void* m, int64_t i) {
-  if constexpr (PREC == P_F32) {
-    const uint32_t u = __float_as_uint(reinterpret_cast<const float*>(m)[i]);
-    return u != 0 && !(u & 0x80000000u);
-  } else if constexpr (PREC == P_FP8) {
-    const uint8_t b = reinterpret_cast<const uint8_t*>(m)[i];
-    return b != 0 && !(b & 0x80u);
-  } else {
-    const uint16_t h = reinterpret_cast<const uint16_t*>(m)[i];
-    return h != 0 && !(h & 0x8000u);
-  }
-}
-
-// Writes an activation: float32 (f32), e4m3 at scale qs (q8), or bf16.
-__device__ __forceinline__ void put_act(void* out, int64_t i, float v, bool q8, float qs,
-                                        bool f32) {
-  if (f32) reinterpret_cast<float*>(out)[i] = v;
-  else if (q8) reinterpret_cast<uint8_t*>(out)[i] = f2q(v * qs);
-  else reinterpret_cast<uint16_t*>(out)[i] = f2bf(v);
-}
-
-// Bytes per element of an activation tensor written with (q8, f32).
-__device__ __forceinline__ int act_bytes(bool q8, bool f32) { return f32 ? 4 : q8 ? 1 : 2; }
-
 // h2 (bf16, or float32 in fp32 mode) and its ReLU mask.
 __device__ __forceinline__ float h2_at(const Step& s, int64_t i) {
   if (s.fp32) return reinterpret_cast<const float*>(s.h2)[i];
@@ -766,9 +569,8 @@ __device__ __forceinline__ void gemm_tile(const Gemm& g, const Step& s, uint32_t
   if (EPI != EPI_UPDATE && T % kXcds == 0) lin = (lin % kXcds) * (T / kXcds) + lin / kXcds;
   const int bm = (int)(lin % gx), bn = (int)((lin / gx) % gy);
   const int bz = (int)(lin / (gx * gy));
-  const int c = bz / g.splits, sp = bz % g.splits;
-  const int kspan = g.K / g.splits;
-  const int kb = sp * kspan, ke = kb + kspan;
+  const int c = bz;
+  const int kb = 0, ke = g.K;
   const int lane = threadIdx.x & (kWave - 1);
   const int w = threadIdx.x / kWave;
   f32x16 acc0, acc1;
@@ -804,43 +606,7 @@ __device__ __forceinline__ void gemm_tile(const Gemm& g, const Step& s, uint32_t
   const float ab = F8 ? 1.0f / (qc[g.ta] * qc[g.tb]) : 1.0f;
   const int half = g.M / 2;
   const int n = bn * BN + w * 32 + (lane & 31);
-  if (EPI == EPI_PARTIAL) {
-    float* pp = g.part + ((int64_t)sp * g.C + c) * g.M * g.N;
-#pragma unroll
-    for (int band = 0; band < 2; ++band) {
-#pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        const int r = 8 * (j >> 2) + 4 * (lane >> 5) + (j & 3);
-        const int m = (band == 0 ? bm * 32 : half + bm * 32) + r;
-        pp[(int64_t)m * g.N + n] = band == 0 ? acc0[j] : acc1[j];
-      }
-    }
-  } else if (EPI == EPI_BIAS_RELU || EPI == EPI_MASK) {
-    const bool q8 = F8 && g.tout >= 0;
-    const bool f32 = PREC == P_F32;
-    const float qs = q8 ? qc[g.tout] : 1.0f;
-    void* out = reinterpret_cast<uint8_t*>(g.out) + (int64_t)c * g.sO * act_bytes(q8, f32);
-    const float bias = (EPI == EPI_BIAS_RELU) ? g.bias[(int64_t)c * g.sBias + n] : 0.f;
-    float amax = 0.f;
-#pragma unroll
-    for (int band = 0; band < 2; ++band) {
-#pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        const int r = 8 * (j >> 2) + 4 * (lane >> 5) + (j & 3);
-        const int m = (band == 0 ? bm * 32 : half + bm * 32) + r;
-        const float a = ab * (band == 0 ? acc0[j] : acc1[j]);
-        float vv;
-        if (EPI == EPI_BIAS_RELU) {
-          vv = fmaxf(a + bias, 0.0f);
-        } else {
-          vv = mask_on<PREC>(g.mask, (int64_t)c * g.sM + (int64_t)m * g.ldm + n) ? a : 0.0f;
-        }
-        amax = fmaxf(amax, fabsf(vv));
-        put_act(out, (int64_t)m * g.ldo + n, vv, q8, qs, f32);
-      }
-    }
-    if (q8) q_note_amax(s, c, g.tout, amax);
-  } else {
+  {
     // Parameter epilogue: element (m, n) of the [M][N] leaf at flat i = m N + n, its
     // noise pair i + M N / 2 sits in acc1 at the same lane and register.
     const Coef k = coef_of(s);
@@ -981,48 +747,6 @@ __global__ void __launch_bounds__(GT, EPI == EPI_UPDATE ? SGMC_UPD_WAVES : 1)
     gemm_tile<BK, PREC, A_K, B_K, EPI, UM>(ga, s, blockIdx.x, gxa, gya, s.C, As, Bs, red);
   else
     gemm_tile<BK, PREC, A_K, B_K, EPI, UM>(gb, s, blockIdx.x - na, gxb, gyb, s.C, As, Bs, red);
-}
-
-// Split-K finish: out = epilogue(ab * sum over splits of the partial products), the
-// splits added in order; four consecutive columns per thread.
-template <int EPI, int PREC>
-__global__ void __launch_bounds__(GT) splitk_finish_kernel(Gemm g, Step s) {
-  constexpr bool F8 = PREC == P_FP8;
-  constexpr bool f32 = PREC == P_F32;
-  __shared__ float red[GT / kWave];
-  const int c = blockIdx.y;
-  const int64_t e = ((int64_t)blockIdx.x * GT + threadIdx.x) * 4;
-  const float* qc = F8 ? s.q + (int64_t)c * kQWords : nullptr;
-  const bool q8 = F8 && g.tout >= 0;
-  float amax = 0.f;
-  if (e < (int64_t)g.M * g.N) {
-    const int m = (int)(e / g.N), n = (int)(e % g.N);
-    const float ab = F8 ? 1.0f / (qc[g.ta] * qc[g.tb]) : 1.0f;
-    const float qs = q8 ? qc[g.tout] : 1.0f;
-    float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int sp = 0; sp < g.splits; ++sp) {
-      const float4 v =
-          *reinterpret_cast<const float4*>(g.part + ((int64_t)sp * g.C + c) * g.M * g.N + e);
-      a.x += v.x;
-      a.y += v.y;
-      a.z += v.z;
-      a.w += v.w;
-    }
-    const float r[4] = {ab * a.x, ab * a.y, ab * a.z, ab * a.w};
-    void* out = reinterpret_cast<uint8_t*>(g.out) + (int64_t)c * g.sO * act_bytes(q8, f32);
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      float v;
-      if (EPI == EPI_BIAS_RELU) {
-        v = fmaxf(r[t] + g.bias[(int64_t)c * g.sBias + n + t], 0.0f);
-      } else {
-        v = mask_on<PREC>(g.mask, (int64_t)c * g.sM + (int64_t)m * g.ldm + n + t) ? r[t] : 0.0f;
-      }
-      amax = fmaxf(amax, fabsf(v));
-      put_act(out, (int64_t)m * g.ldo + n + t, v, q8, qs, f32);
-    }
-  }
-  if (q8) q_note_amax_block(s, c, g.tout, amax, red);
 }
 
 // ------------------------------------------------------------------ head ------
@@ -1572,7 +1296,7 @@ using namespace sgmc::mlp;
 namespace {
 
 struct Layout {
-  int64_t xb, lab, h1, h2, da2, da1, dl, lik, lkey, prior, ke, facc, col, fin, split, total;
+  int64_t xb, lab, h1, h2, da2, da1, dl, lik, lkey, prior, ke, facc, col, fin, total;
   int nparts, g4_blocks, g5_blocks, small_blocks;
 };
 
@@ -1601,7 +1325,6 @@ Layout layout_of(int C, int n, int D_in, int H1, int H2) {
   L.facc = o; o = align256(o + (int64_t)C * 8);
   L.col = o; o = align256(o + (int64_t)C * (n / kStrip) * small_total * 4);
   L.fin = o; o = align256(o + (int64_t)C * kFinalBlocks * 8);
-  L.split = o; o = align256(o + (int64_t)4 * C * n * std::max(H1, H2) * 4);
   L.total = o;
   return L;
 }
@@ -1635,19 +1358,13 @@ namespace {
 // workspace holds 4 C n max(H1, H2) floats).
 constexpr int kMaxSplits = 2;
 
-// GEMM call sites of one evaluation (the tune[] slots): G1 = Xb W1, G2 = H1 W2,
-// G3 = dA2 W2^T, G4 = H1^T dA2 (gW2), G5 = Xb^T dA1 (gW1).
-enum GemmSlot { SLOT_G1 = 0, SLOT_G2, SLOT_G3, SLOT_G4, SLOT_G5, kSlots };
-
 template <int BK, int PREC, bool A_K, bool B_K, int EPI>
-void launch_gemm_bk(dim3 grid, Gemm g, const Step& s, hipStream_t st, float* part,
-                    int splits) {
+void launch_gemm_bk(dim3 grid, Gemm g, const Step& s, hipStream_t st) {
   // parameter updates of SGLD with rms_prop and of the two OBABO halves run the kernel
   // with their rule compiled in
   if constexpr (EPI == EPI_UPDATE) {
-    if (splits <= 1) {
+    {
       g.C = (int)grid.z;
-      g.splits = 1;
       if (s.mode == MLP_SGLD && s.rms) {
         hipLaunchKernelGGL((gemm_kernel<BK, PREC, A_K, B_K, EPI, UM_RMS>), grid, dim3(GT), 0, st,
                            g, s);
@@ -1666,33 +1383,22 @@ void launch_gemm_bk(dim3 grid, Gemm g, const Step& s, hipStream_t st, float* par
     }
   }
   g.C = (int)grid.z;
-  g.splits = splits;
-  if (g.splits > 1) {
-    g.part = part;
-    hipLaunchKernelGGL((gemm_kernel<BK, PREC, A_K, B_K, EPI_PARTIAL>),
-                       dim3(grid.x, grid.y, grid.z * g.splits), dim3(GT), 0, st, g, s);
-    const int64_t quads = (int64_t)g.M * g.N / 4;
-    hipLaunchKernelGGL((splitk_finish_kernel<EPI, PREC>),
-                       dim3((unsigned)((quads + GT - 1) / GT), g.C), dim3(GT), 0, st, g, s);
-  } else {
-    hipLaunchKernelGGL((gemm_kernel<BK, PREC, A_K, B_K, EPI>), grid, dim3(GT), 0, st, g, s);
-  }
+  hipLaunchKernelGGL((gemm_kernel<BK, PREC, A_K, B_K, EPI>), grid, dim3(GT), 0, st, g, s);
 }
 
 // Launches GEMM `slot` with the k-tile depth and split-K factor of s.plan[slot].
 template <bool A_K, bool B_K, int EPI>
 void launch_gemm(dim3 grid, const Gemm& g, const Step& s, hipStream_t st, int slot) {
   const int tv = s.plan[slot];
-  const int splits = tv & 15;
   const bool deep = (tv >> 4) == 128;
   if (s.fp32) {
-    launch_gemm_bk<32, P_F32, A_K, B_K, EPI>(grid, g, s, st, s.split_part, splits);
+    launch_gemm_bk<32, P_F32, A_K, B_K, EPI>(grid, g, s, st);
   } else if (s.fp8) {
-    if (deep) launch_gemm_bk<128, P_FP8, A_K, B_K, EPI>(grid, g, s, st, s.split_part, splits);
-    else launch_gemm_bk<64, P_FP8, A_K, B_K, EPI>(grid, g, s, st, s.split_part, splits);
+    if (deep) launch_gemm_bk<128, P_FP8, A_K, B_K, EPI>(grid, g, s, st);
+    else launch_gemm_bk<64, P_FP8, A_K, B_K, EPI>(grid, g, s, st);
   } else {
-    if (deep) launch_gemm_bk<128, P_BF16, A_K, B_K, EPI>(grid, g, s, st, s.split_part, splits);
-    else launch_gemm_bk<32, P_BF16, A_K, B_K, EPI>(grid, g, s, st, s.split_part, splits);
+    if (deep) launch_gemm_bk<128, P_BF16, A_K, B_K, EPI>(grid, g, s, st);
+    else launch_gemm_bk<32, P_BF16, A_K, B_K, EPI>(grid, g, s, st);
   }
 }
 
@@ -1701,7 +1407,6 @@ void launch_gemm(dim3 grid, const Gemm& g, const Step& s, hipStream_t st, int sl
 template <int BK, int PREC, int EPI>
 void launch_pair_bk(Gemm ga, dim3 ra, Gemm gb, dim3 rb, const Step& s, hipStream_t st) {
   ga.C = gb.C = (int)ra.z;
-  ga.splits = gb.splits = 1;
   const dim3 grid(ra.x * ra.y * ra.z + rb.x * rb.y * rb.z);
   if constexpr (EPI == EPI_UPDATE) {
     if (s.mode == MLP_SGLD && s.rms) {
@@ -1870,7 +1575,6 @@ int make_step(const sgmc_mlp_state* st, int update, Layout& L, Step& s) {
   s.ke_part = reinterpret_cast<float*>(w + L.ke);
   s.col_part = reinterpret_cast<float*>(w + L.col);
   s.fin_part = reinterpret_cast<double*>(w + L.fin);
-  s.split_part = reinterpret_cast<float*>(w + L.split);
   s.nparts = L.nparts;
   s.U = q.U; s.grad = q.grad;
   s.samples = q.samples; s.samples_U = q.samples_U; s.n_slots = q.n_slots;
@@ -1935,12 +1639,10 @@ void launch_forward(const Step& s, const sgmc_mlp_state& q, hipStream_t st_) {
   const void* W2 = gemm_weight(s, q, 1);
   Gemm g1{s.Xb, q.D_in, (int64_t)n * q.D_in, W1, q.H1, q.P, n, q.H1, q.D_in,
           s.h1, q.H1, (int64_t)n * q.H1, q.theta + s.off[3], q.P, nullptr, 0, 0, 0, 0};
-  launch_gemm<true, false, EPI_BIAS_RELU>(dim3(n / BM, q.H1 / BN, C), with_q(g1, Q_X, Q_W1, Q_H1),
-                                          s, st_, SLOT_G1);
+  launch_act_gemm(with_q(g1, Q_X, Q_W1, Q_H1), s, st_, s.plan[SLOT_G1] & 15);
   Gemm g2{s.h1, q.H1, (int64_t)n * q.H1, W2, q.H2, q.P, n, q.H2, q.H1,
           s.h2, q.H2, (int64_t)n * q.H2, q.theta + s.off[4], q.P, nullptr, 0, 0, 0, 0};
-  launch_gemm<true, false, EPI_BIAS_RELU>(dim3(n / BM, q.H2 / BN, C), with_q(g2, Q_H1, Q_W2, -1),
-                                          s, st_, SLOT_G2);
+  launch_act_gemm(with_q(g2, Q_H1, Q_W2, -1), s, st_, s.plan[SLOT_G2] & 15);
   launch_head(s, st_);
 }
 
@@ -1974,8 +1676,7 @@ int sgmc_mlp_step(const sgmc_mlp_state* st, int update, void* stream) {
   // dA1 = (dA2 W2^T) * (H1 > 0): B[k=b][n=a] = W2[a][b], k-contiguous rows of W2.
   Gemm g3{s.da2, q.H2, (int64_t)n * q.H2, W2, q.H2, q.P, n, q.H1, q.H2,
           s.da1, q.H1, (int64_t)n * q.H1, nullptr, 0, s.h1, q.H1, (int64_t)n * q.H1, 0, 0};
-  launch_gemm<true, true, EPI_MASK>(dim3(n / BM, q.H1 / BN, C), with_q(g3, Q_DA2, Q_W2, Q_DA1), s,
-                                    st_, SLOT_G3);
+  launch_act_gemm(with_q(g3, Q_DA2, Q_W2, Q_DA1), s, st_, s.plan[SLOT_G3] & 15);
   // gW2 = H1^T dA2: A[m=a][k=i] = H1[i][a] (m-contiguous), B[k=i][n=b] = dA2[i][b].
   Gemm g4{s.h1, q.H1, (int64_t)n * q.H1, s.da2, q.H2, (int64_t)n * q.H2, q.H1, q.H2, n,
           nullptr, 0, 0, nullptr, 0, nullptr, 0, 0, 1, 0};
