@@ -504,9 +504,9 @@ typedef struct sgmc_mlp_state {
   /* GEMM tiling per call site -- G1 = Xb W1, G2 = h1 W2, G3 = dA2 W2^T, G4 = h1^T dA2
    * (gW2), G5 = Xb^T dA1 (gW1): 0 keeps the built-in choice, else 16 k + s with k the
    * k-tile depth (bf16 32 or 128, e4m3 64 or 128, float32 32) and s the split-K factor
-   * (1, 2 or 4; 1 for G4, G5), the GEMM's K a multiple of k s. The k order of the
-   * matrix instructions changes with the split only for the forward GEMMs, whose
-   * partial products are added in split order. Set by FusedMLP.autotune. */
+   * (1, 2, 3 or 4; 1 for G4, G5), the GEMM's K a multiple of k s. A split GEMM adds
+   * the products of its K slices in order; the k-tile only takes part in which splits
+   * fit K. Set by FusedMLP.autotune. */
   int32_t tune[5];
 } sgmc_mlp_state;
 

@@ -26,17 +26,12 @@
 // stored in float32, weights read from theta itself, no shadow); fp32 accumulation in
 // all three.
 //
-// GEMM tiling (gfx950): a block computes 64 rows x 128
-// columns; its 64 rows are two bands of 32 rows M/2 apart, so each lane's two
-// accumulators hold the element pairs (i, i + size/2) that one Threefry block of
-// random_bits serves (integrator.py:119-135 noise). Four wavefronts own 32 columns
-// each. Operands are staged through LDS with k contiguous (padded rows); a source that
-// is m- or n-contiguous is transposed while being written to LDS.
+// The GEMMs: mlp_fwd.hip (G1-G3) and mlp_param.hip (G4, G5 with the update).
 #include <math.h>
 
 #include <type_traits>
 
-#include "mlp_common.h"
+#include "mlp_update.h"
 
 namespace sgmc {
 namespace mlp {
@@ -45,25 +40,6 @@ namespace mlp {
 #define SGMC_GATHER_BATCH 12
 #endif
 constexpr int kGatherBatch = SGMC_GATHER_BATCH;  // float4 row loads in flight per lane
-// Update epilogue tuning: parameters pairs per prefetch chunk (1, 2, 4 or 8 of a lane's
-// 16 pairs) and the waves per SIMD the update GEMMs are compiled for (register budget).
-#ifndef SGMC_UPD_CHUNK
-#define SGMC_UPD_CHUNK 2
-#endif
-#ifndef SGMC_UPD_NT
-#define SGMC_UPD_NT 0
-#endif
-#ifndef SGMC_UPD_WAVES
-#define SGMC_UPD_WAVES 1
-#endif
-constexpr int kUpdChunk = SGMC_UPD_CHUNK;
-static_assert(16 % kUpdChunk == 0, "chunks of the 16 pairs");
-// The compiled-in rms_prop update at deep k-tiles (two waves per SIMD either way) has the
-// registers for chunks of four pairs (pSGLD 3072-512-512 step 294.9 -> 292.7 us; the
-// run-time rule of the OBABO updates loses a wave with them)
-constexpr int kUpdChunkDeep = 4;
-static_assert(16 % kUpdChunkDeep == 0, "chunks of the 16 pairs");
-
 // Gradient-only variant: grad = (gsum + prior) / T, no update.
 __device__ __forceinline__ void grad_param(const Step& s, const float* th, float* gout,
                                            int64_t i, float gsum, float& lp) {
@@ -76,230 +52,6 @@ __device__ __forceinline__ void grad_param(const Step& s, const float* th, float
   gout[i] = g / s.temperature;
 }
 
-
-// Parameter update of one leaf of chain c, applied to values so that a thread can
-// issue the loads of all its parameters before the arithmetic. The leaf's arrays are
-// addressed from uniform base pointers with 32-bit offsets (a leaf holds < 2^32
-// entries). Update rules (prior gradient and temperature folded into g = (gsum + w /
-// s^2) / T, written with fused multiply-adds: within an ulp or two of the reference's
-// separate roundings, far inside the bf16 / e4m3 GEMM error):
-//   SGLD (integrator.py:882-912): w += (-eps) g + sqrt(2 T eps) xi; with rms_prop
-//     (adaption.py:254-291): v = alpha v + (1 - alpha) g^2, G = 1 / (lmbd + sqrt(v)),
-//     w += G (-eps) g + sqrt(G) sqrt(2 T eps) xi (hardware reciprocal and square roots);
-//   OBABO with the identity mass (integrator.py:181-273), in two halves:
-//     BA: p1 = sqrt(pi) p + sqrt((1 - pi) T) xi(s1); KE_start += p1^2 / 2;
-//         p2 = (-eps/2) g + p1; w += eps p2
-//     BO: p3 = (-eps/2) g(w') + p2; KE_end += p3^2 / 2; p = sqrt(pi) p3 + ... xi(s2).
-struct Upd {
-  float* th;          // theta of the leaf
-  float* aux;         // rms_prop v or OBABO momentum of the leaf, or null (plain SGLD)
-  uint16_t* sh;       // bf16 shadow of the leaf, or null
-  uint8_t* sh8;       // e4m3 shadow (W1, W2 in fp8 mode), or null
-  float q8;           // scale the e4m3 shadow is written with
-  int mode, rms, has_prior;
-  float inv_var, log_norm, inv_T, eps, noise_scale, decay, noise, half, alpha, one_m_alpha,
-      lmbd;
-};
-
-// Per-kernel step coefficients of the current iteration.
-struct Coef {
-  float eps, noise_scale, decay, noise;
-};
-
-__device__ __forceinline__ Coef coef_of(const Step& s) {
-  const int it = cur_iter(s);
-  Coef k;
-  k.eps = s.eps_table[it];
-  k.noise_scale = sqrtf((2.0f * s.noise_temperature) * k.eps);
-  k.decay = s.decay_table ? s.decay_table[it] : 0.0f;
-  k.noise = s.noise_table ? s.noise_table[it] : 0.0f;
-  return k;
-}
-
-__device__ __forceinline__ Upd make_upd(const Step& s, int c, int leaf, int64_t base,
-                                        const Coef& k) {
-  Upd u;
-  u.th = s.theta + base;
-  u.aux = s.mode == MLP_SGLD ? (s.rms ? s.v + base : nullptr) : s.mom + base;
-  u.sh = nullptr;
-  u.sh8 = nullptr;
-  u.q8 = 1.0f;
-  if (s.fp8 && leaf < 2) {
-    u.sh8 = s.shadow8 + base;
-    u.q8 = s.q[(int64_t)c * kQWords + 6 + leaf];
-  } else if (!s.fp32) {
-    u.sh = s.shadow + base;
-  }
-  u.mode = s.mode;
-  u.rms = s.rms;
-  u.has_prior = s.has_prior;
-  u.inv_var = s.prior_inv_var;
-  u.log_norm = s.prior_log_norm;
-  u.inv_T = 1.0f / s.temperature;
-  u.eps = k.eps;
-  u.noise_scale = k.noise_scale;
-  u.decay = k.decay;
-  u.noise = k.noise;
-  u.half = 0.5f * k.eps;
-  u.alpha = s.alpha;
-  u.one_m_alpha = 1.0f - s.alpha;
-  u.lmbd = s.lmbd;
-  return u;
-}
-
-// Parameter state is streamed (read once, written once per launch): with SGMC_UPD_NT the
-// accesses carry the non-temporal hint.
-template <class T>
-__device__ __forceinline__ T upd_ld(const T* p) {
-  if (SGMC_UPD_NT) return __builtin_nontemporal_load(p);
-  return *p;
-}
-template <class T>
-__device__ __forceinline__ void upd_st(T v, T* p) {
-  if (SGMC_UPD_NT) __builtin_nontemporal_store(v, p);
-  else *p = v;
-}
-
-// UM: the update rule compiled in -- UM_RMS: SGLD with rms_prop (state v in aux);
-// UM_OBA / UM_OBO: the O B A and B O halves of an OBABO step (momentum in aux); or
-// UM_ANY: the rule of u.mode / u.rms at run time.
-constexpr int UM_ANY = 0;
-constexpr int UM_RMS = 1;
-constexpr int UM_OBA = 2;
-constexpr int UM_OBO = 3;
-
-// the rule's mode, and whether it carries state in aux / writes theta
-template <int UM>
-__device__ __forceinline__ int um_mode(const Upd& u) {
-  return UM == UM_RMS ? MLP_SGLD : UM == UM_OBA ? MLP_OBABO_BA : UM == UM_OBO ? MLP_OBABO_BO
-                                                                               : u.mode;
-}
-
-template <int UM = UM_ANY>
-__device__ __forceinline__ void upd_load(const Upd& u, uint32_t i, float& w, float& aux) {
-  w = upd_ld(u.th + i);
-  aux = (UM != UM_ANY || u.aux) ? upd_ld(u.aux + i) : 0.0f;
-}
-
-template <int UM = UM_ANY>
-__device__ __forceinline__ void upd_step(const Upd& u, float& w, float& aux, float gsum,
-                                         float xi, float& lp, float& ke) {
-  float g = gsum;
-  if (u.has_prior) {
-    g = __builtin_fmaf(w, u.inv_var, g);
-    lp = __builtin_fmaf(__builtin_fmaf(w * w, u.inv_var, u.log_norm), -0.5f, lp);
-  }
-  g = g * u.inv_T;
-  const int mode = um_mode<UM>(u);
-  if (mode == MLP_SGLD) {
-    const float sg = (-u.eps) * g;
-    const float sn = u.noise_scale * xi;
-    if (UM == UM_RMS || u.rms) {
-      const float vn = __builtin_fmaf(u.alpha, aux, u.one_m_alpha * (g * g));
-      aux = vn;
-      // G = 1 / (lambda + sqrt(v)) and sqrt(G) from one reciprocal square root
-      const float rG = __builtin_amdgcn_rsqf(u.lmbd + __builtin_amdgcn_sqrtf(vn));
-      w = w + __builtin_fmaf(rG, sn, (rG * rG) * sg);
-    } else {
-      w = w + (sg + sn);
-    }
-  } else if (mode == MLP_OBABO_BA) {
-    const float p1 = __builtin_fmaf(u.decay, aux, u.noise * xi);
-    ke = __builtin_fmaf(p1, p1, ke);
-    const float p2 = __builtin_fmaf(-u.half, g, p1);
-    aux = p2;
-    w = __builtin_fmaf(u.eps, p2, w);
-  } else {
-    const float p3 = __builtin_fmaf(-u.half, g, aux);
-    ke = __builtin_fmaf(p3, p3, ke);
-    aux = __builtin_fmaf(u.decay, p3, u.noise * xi);
-  }
-}
-
-// SH: the GEMM copy written -- SH_NONE, SH_BF16, SH_E4M3 (known from the operand
-// precision in the parameter-update GEMMs), or SH_ANY: whichever pointer is set.
-constexpr int SH_ANY = -1, SH_NONE = 0, SH_BF16 = 1, SH_E4M3 = 2;
-
-template <int UM = UM_ANY, int SH = SH_ANY>
-__device__ __forceinline__ void upd_store(const Upd& u, uint32_t i, float w, float aux,
-                                          float& wmax) {
-  if (um_mode<UM>(u) != MLP_OBABO_BO) {
-    upd_st(w, u.th + i);
-    if (SH == SH_E4M3 || (SH == SH_ANY && u.sh8)) {
-      upd_st(f2q(w * u.q8), u.sh8 + i);
-      wmax = fmaxf(wmax, fabsf(w));
-    } else if (SH == SH_BF16 || (SH == SH_ANY && u.sh)) {
-      upd_st(f2bf(w), u.sh + i);
-    }
-  }
-  if (UM != UM_ANY || u.aux) upd_st(aux, u.aux + i);
-}
-
-// Buffer resources of one leaf's state (theta, v, GEMM copy) for the compiled-in
-// rms_prop update: a lane addresses its parameters with one 32-bit offset and the
-// per-element offsets are uniform (scalar offset field), so no per-element address
-// arithmetic runs on the vector ALU.
-constexpr int kRawBufferFlags = 0x00020000;  // word 3 of a raw buffer resource (CDNA)
-
-struct UpdRes {
-  __amdgpu_buffer_rsrc_t th, aux, sh;
-};
-
-template <int SH>
-__device__ __forceinline__ UpdRes make_res(const Upd& u, uint32_t count) {
-  UpdRes r;
-  r.th = __builtin_amdgcn_make_buffer_rsrc(u.th, (short)0, (int)(4 * count), kRawBufferFlags);
-  r.aux = __builtin_amdgcn_make_buffer_rsrc(u.aux, (short)0, (int)(4 * count), kRawBufferFlags);
-  if (SH == SH_E4M3)
-    r.sh = __builtin_amdgcn_make_buffer_rsrc(u.sh8, (short)0, (int)count, kRawBufferFlags);
-  else
-    r.sh = __builtin_amdgcn_make_buffer_rsrc(u.sh, (short)0, (int)(2 * count), kRawBufferFlags);
-  return r;
-}
-
-// element vo + so (vo per lane, so uniform)
-__device__ __forceinline__ void res_load(const UpdRes& r, uint32_t vo, uint32_t so, float& w,
-                                         float& aux) {
-  w = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r.th, 4 * vo, 4 * so, 0));
-  aux = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r.aux, 4 * vo, 4 * so, 0));
-}
-
-// TH: the rule changes theta (and so its GEMM copy); the B O half of OBABO does not.
-template <int SH, bool TH = true>
-__device__ __forceinline__ void res_store(const Upd& u, const UpdRes& r, uint32_t vo,
-                                          uint32_t so, float w, float aux, float& wmax) {
-  if (TH) {
-    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(w), r.th, 4 * vo, 4 * so, 0);
-    if (SH == SH_E4M3) {
-      __builtin_amdgcn_raw_buffer_store_b8(f2q(w * u.q8), r.sh, vo, so, 0);
-      wmax = fmaxf(wmax, fabsf(w));
-    } else if (SH == SH_BF16) {
-      __builtin_amdgcn_raw_buffer_store_b16(f2bf(w), r.sh, 2 * vo, 2 * so, 0);
-    }
-  }
-  __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(aux), r.aux, 4 * vo, 4 * so, 0);
-}
-
-// Key of leaf `leaf` of the noise tree of this update: random_tree(sub) with
-// (key, sub) = split(key) for SGLD; s1 / s2 of (key, s1, s2) = split(key, 3) for the
-// two momentum refreshes of an OBABO step.
-__device__ __forceinline__ Key derive_leaf_key(const Step& s, int chain, int leaf) {
-  const Key k = load_key(s.key + 2 * chain);
-  Key a, b, c;
-  if (s.mode == MLP_SGLD) {
-    split2(k, a, b);
-    return split_key(b, NLEAF, (uint32_t)leaf);
-  }
-  split3(k, a, b, c);
-  return split_key(s.mode == MLP_OBABO_BA ? b : c, NLEAF, (uint32_t)leaf);
-}
-
-// The same key as stored by the step's gather kernel (the chain key does not change
-// until the step's last kernel), so the update epilogues load two words instead of
-// running four to seven Threefry blocks per wave.
-__device__ __forceinline__ Key leaf_key(const Step& s, int chain, int leaf) {
-  return load_key(s.lkey + 2 * (chain * NLEAF + leaf));
-}
 
 // ------------------------------------------------------------------ gather ----
 // Xb[c][j] = bf16(X[idx_j]), lab[c][j] = labels[idx_j]; one wavefront per row.
@@ -368,172 +120,6 @@ __global__ void __launch_bounds__(GT) gather_kernel(Step s) {
   if (lane == 0) s.lab[row] = valid ? s.labels[r] : -1;
 }
 
-typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-
-// ---- operand tiles in LDS ----
-// A tile: BM rows (m) x BK (k); B tile: BN rows (n) x BK. A row holds BK elements in
-// 16-byte chunks (8 bf16 or 16 e4m3); chunk c of row r sits at position c ^ swz(r), so
-// that the MFMA fragment reads (consecutive rows, one chunk) and the stores of
-// transposed 8x8 blocks (row groups 8 apart) spread over the LDS banks.
-template <int CH>
-__device__ __forceinline__ int swz(int r) {
-  return (r ^ (r >> 3)) & (CH - 1);
-}
-
-// 8x8 transpose of 16-bit elements: in[i] holds 8 consecutive columns of row i; out[j]
-// holds rows 0..7 of column j.
-__device__ __forceinline__ void transpose8x8(const u32x4 (&in)[8], u32x4 (&out)[8]) {
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-#pragma unroll
-    for (int d = 0; d < 4; ++d) {
-      const u32x4& x = in[2 * d];
-      const u32x4& y = in[2 * d + 1];
-      const uint32_t a = (j >> 1) == 0 ? x.x : (j >> 1) == 1 ? x.y : (j >> 1) == 2 ? x.z : x.w;
-      const uint32_t b = (j >> 1) == 0 ? y.x : (j >> 1) == 1 ? y.y : (j >> 1) == 2 ? y.z : y.w;
-      const uint32_t v = (j & 1) ? ((a >> 16) | (b & 0xFFFF0000u)) : ((a & 0xFFFFu) | (b << 16));
-      if (d == 0) out[j].x = v;
-      else if (d == 1) out[j].y = v;
-      else if (d == 2) out[j].z = v;
-      else out[j].w = v;
-    }
-  }
-}
-
-// 4x4 transpose of 32-bit elements: in[i] holds 4 consecutive columns of row i.
-__device__ __forceinline__ void transpose8x8(const u32x4 (&in)[4], u32x4 (&out)[4]) {
-#pragma unroll
-  for (int j = 0; j < 4; ++j) out[j] = u32x4{in[0][j], in[1][j], in[2][j], in[3][j]};
-}
-
-// 8x8 transpose of bytes: in[i] holds 8 consecutive columns of row i.
-__device__ __forceinline__ void transpose8x8(const u32x2 (&in)[8], u32x2 (&out)[8]) {
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    uint32_t lo = 0, hi = 0;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const uint32_t w = (j < 4) ? in[i].x : in[i].y;
-      const uint32_t byte = (w >> (8 * (j & 3))) & 0xFFu;
-      if (i < 4) lo |= byte << (8 * i);
-      else hi |= byte << (8 * (i - 4));
-    }
-    out[j].x = lo;
-    out[j].y = hi;
-  }
-}
-
-// Loads of one operand tile (ROWS x BK elements of EB bytes, at k0) into registers and
-// their stores to LDS. KC: the source is k-contiguous (row r at grow(r) * ld);
-// otherwise it is row-contiguous (k-row k at k * ld) and each thread moves one TBxTB
-// block (8x8 of 1- or 2-byte elements, 4x4 of 4-byte ones), transposed in registers.
-// grow maps tile rows to source rows (contiguous within a block).
-template <int ROWS, int BK, bool KC, int EB>
-struct Tile {
-  static constexpr int EPC = 16 / EB;                 // elements per chunk
-  static constexpr int CH = BK / EPC;                 // chunks per row
-  static constexpr int ROWB = BK * EB;                // bytes per LDS row
-  static constexpr int TB = EB == 4 ? 4 : 8;          // transposed block edge
-  static constexpr int NR = KC ? ROWS * CH / GT : TB;  // registers per thread
-  static constexpr int BLOCKS = ROWS * BK / (TB * TB);  // blocks (transposed case)
-  using R = typename std::conditional<KC || EB >= 2, u32x4, u32x2>::type;
-  static_assert(KC || BLOCKS <= GT, "transposed tile: one block per thread at most");
-  static_assert(!KC || (ROWS * CH) % GT == 0, "k-contiguous tile: whole chunks per thread");
-  R r[NR];
-
-  __device__ __forceinline__ static int off(int row, int chunk) {
-    return row * ROWB + ((chunk ^ swz<CH>(row)) << 4);
-  }
-
-  template <typename Grow>
-  __device__ __forceinline__ void load(const uint8_t* src, int64_t ld, int k0, Grow grow) {
-    const int t = threadIdx.x;
-    if constexpr (KC) {
-#pragma unroll
-      for (int h = 0; h < NR; ++h) {
-        const int u = t + h * GT;
-        const int row = u / CH, ch = u % CH;
-        r[h] = *reinterpret_cast<const u32x4*>(src + (grow(row) * ld + k0 + ch * EPC) * EB);
-      }
-    } else {
-      if (!(BLOCKS >= GT || t < BLOCKS)) return;
-      const int r8 = (t % (ROWS / TB)) * TB, k8 = (t / (ROWS / TB)) * TB;
-#pragma unroll
-      for (int i = 0; i < TB; ++i)
-        r[i] = *reinterpret_cast<const R*>(src + ((int64_t)(k0 + k8 + i) * ld + grow(r8)) * EB);
-    }
-  }
-
-  __device__ __forceinline__ void store(uint8_t* lds) const {
-    const int t = threadIdx.x;
-    if constexpr (KC) {
-#pragma unroll
-      for (int h = 0; h < NR; ++h) {
-        const int u = t + h * GT;
-        const int row = u / CH, ch = u % CH;
-        *reinterpret_cast<u32x4*>(lds + off(row, ch)) = r[h];
-      }
-    } else {
-      if (!(BLOCKS >= GT || t < BLOCKS)) return;
-      const int r8 = (t % (ROWS / TB)) * TB, k8 = (t / (ROWS / TB)) * TB;
-      R o[TB];
-      transpose8x8(r, o);
-      const int kb = k8 * EB;  // byte offset of the block's k range in a row
-#pragma unroll
-      for (int j = 0; j < TB; ++j)
-        *reinterpret_cast<R*>(lds + off(r8 + j, kb >> 4) + (kb & 15)) = o[j];
-    }
-  }
-};
-
-// k-values one mfma_step consumes: 16 (one 32x32x16 instruction per band), or 8 for
-// float32 (four 32x32x2 instructions per band).
-template <int PREC>
-constexpr int k_step() {
-  return PREC == P_F32 ? 8 : 16;
-}
-
-// One MFMA step: a and b are read at chunk/offset of rows ra and rb. bf16 / e4m3: lanes
-// 0-31 hold k .. k + 7 and lanes 32-63 k + 8 .. k + 15 of one 32x32x16 instruction.
-// float32: each lane reads one 16-byte chunk (4 k-values; lanes 32-63 the next chunk)
-// and feeds its elements to four 32x32x2 instructions, instruction u taking k + u from
-// lanes 0-31 and k + 4 + u from lanes 32-63 (the same k for A and B, so every product
-// of the 8 k-values enters once).
-template <int BK, int PREC>
-__device__ __forceinline__ void mfma_step(const uint8_t* As, const uint8_t* Bs, int kk, int lane,
-                                          int w, f32x16& acc0, f32x16& acc1) {
-  constexpr int EB = elem_bytes<PREC>();
-  using TA = Tile<BM, BK, true, EB>;
-  const int k = kk + (k_step<PREC>() / 2) * (lane >> 5);   // this lane's first k
-  const int kb = k * EB;
-  const int ra0 = lane & 31, ra1 = 32 + (lane & 31), rb0 = w * 32 + (lane & 31);
-  const int o0 = TA::off(ra0, kb >> 4) + (kb & 15);
-  const int o1 = TA::off(ra1, kb >> 4) + (kb & 15);
-  const int ob = TA::off(rb0, kb >> 4) + (kb & 15);
-  if constexpr (PREC == P_F32) {
-    const f32x4 a0 = *reinterpret_cast<const f32x4*>(As + o0);
-    const f32x4 a1 = *reinterpret_cast<const f32x4*>(As + o1);
-    const f32x4 b = *reinterpret_cast<const f32x4*>(Bs + ob);
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[u], b[u], acc0, 0, 0, 0);
-      acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[u], b[u], acc1, 0, 0, 0);
-    }
-  } else if constexpr (PREC == P_FP8) {
-    const long a0 = *reinterpret_cast<const long*>(As + o0);
-    const long a1 = *reinterpret_cast<const long*>(As + o1);
-    const long b = *reinterpret_cast<const long*>(Bs + ob);
-    acc0 = __builtin_amdgcn_mfma_f32_32x32x16_fp8_fp8(a0, b, acc0, 0, 0, 0);
-    acc1 = __builtin_amdgcn_mfma_f32_32x32x16_fp8_fp8(a1, b, acc1, 0, 0, 0);
-  } else {
-    const bf16x8 a0 = *reinterpret_cast<const bf16x8*>(As + o0);
-    const bf16x8 a1 = *reinterpret_cast<const bf16x8*>(As + o1);
-    const bf16x8 b = *reinterpret_cast<const bf16x8*>(Bs + ob);
-    acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, b, acc0, 0, 0, 0);
-    acc1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, b, acc1, 0, 0, 0);
-  }
-}
-
 // h2 (bf16, or float32 in fp32 mode) and its ReLU mask.
 __device__ __forceinline__ float h2_at(const Step& s, int64_t i) {
   if (s.fp32) return reinterpret_cast<const float*>(s.h2)[i];
@@ -549,204 +135,6 @@ __device__ __forceinline__ float get_act(const Step& s, int c, int t, const void
   if (s.fp32) return reinterpret_cast<const float*>(p)[i];
   if (s.fp8) return q2f(reinterpret_cast<const uint8_t*>(p)[i]) / s.q[(int64_t)c * kQWords + t];
   return bf2f(reinterpret_cast<const uint16_t*>(p)[i]);
-}
-
-// One block's tile of GEMM g: block lin (linear id) of a gx x gy x gz grid.
-template <int BK, int PREC, bool A_K, bool B_K, int EPI, int UM>
-__device__ __forceinline__ void gemm_tile(const Gemm& g, const Step& s, uint32_t lin,
-                                          uint32_t gx, uint32_t gy, uint32_t gz, uint8_t* As,
-                                          uint8_t* Bs, float* red) {
-  static_assert(BN == 2 * BM, "tile shapes");
-  constexpr bool F8 = PREC == P_FP8;
-  constexpr int EB = elem_bytes<PREC>();
-  // Blocks go to the XCDs round-robin by linear id. In the GEMMs without a parameter
-  // update, XCD x takes the contiguous range [x T / 8, (x + 1) T / 8) of logical tiles
-  // (bm fastest, then bn, then chain and split), so the blocks that share an operand tile
-  // read it through one L2 instead of fetching it from HBM once per XCD (Xb W1 of a
-  // 3072-512 net: 390 -> 75 MB per launch). The update GEMMs keep the linear order, whose
-  // state stream measured faster.
-  const uint32_t T = gx * gy * gz;
-  if (EPI != EPI_UPDATE && T % kXcds == 0) lin = (lin % kXcds) * (T / kXcds) + lin / kXcds;
-  const int bm = (int)(lin % gx), bn = (int)((lin / gx) % gy);
-  const int bz = (int)(lin / (gx * gy));
-  const int c = bz;
-  const int kb = 0, ke = g.K;
-  const int lane = threadIdx.x & (kWave - 1);
-  const int w = threadIdx.x / kWave;
-  f32x16 acc0, acc1;
-#pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    acc0[j] = 0.f;
-    acc1[j] = 0.f;
-  }
-  const uint8_t* A = reinterpret_cast<const uint8_t*>(g.A) + (int64_t)c * g.sA * EB;
-  const uint8_t* B = reinterpret_cast<const uint8_t*>(g.B) + (int64_t)c * g.sB * EB;
-  const int hm = g.M / 2;
-  auto growA = [&](int r) -> int64_t { return r < 32 ? bm * 32 + r : hm + bm * 32 + (r - 32); };
-  auto growB = [&](int r) -> int64_t { return (int64_t)bn * BN + r; };
-  Tile<BM, BK, A_K, EB> ta;
-  Tile<BN, BK, B_K, EB> tb;
-  ta.load(A, g.lda, kb, growA);
-  tb.load(B, g.ldb, kb, growB);
-  for (int k0 = kb; k0 < ke; k0 += BK) {
-    __syncthreads();
-    ta.store(As);
-    tb.store(Bs);
-    __syncthreads();
-    if (k0 + BK < ke) {
-      ta.load(A, g.lda, k0 + BK, growA);
-      tb.load(B, g.ldb, k0 + BK, growB);
-    }
-#pragma unroll
-    for (int kk = 0; kk < BK; kk += k_step<PREC>()) mfma_step<BK, PREC>(As, Bs, kk, lane, w, acc0, acc1);
-  }
-
-  // F8: products carry the operand scales; ab undoes them
-  const float* qc = F8 ? s.q + (int64_t)c * kQWords : nullptr;
-  const float ab = F8 ? 1.0f / (qc[g.ta] * qc[g.tb]) : 1.0f;
-  const int half = g.M / 2;
-  const int n = bn * BN + w * 32 + (lane & 31);
-  {
-    // Parameter epilogue: element (m, n) of the [M][N] leaf at flat i = m N + n, its
-    // noise pair i + M N / 2 sits in acc1 at the same lane and register.
-    const Coef k = coef_of(s);
-    const int64_t base = (int64_t)c * s.P + s.off[g.leaf];
-    const float* th = s.theta + base;
-    const uint32_t S = (uint32_t)((int64_t)g.M * g.N);
-    float lp = 0.0f, ke = 0.0f, wmax = 0.0f;
-    if (EPI == EPI_UPDATE) {
-      const Key lk = leaf_key(s, c, g.leaf);
-      const Upd up = make_upd(s, c, g.leaf, base, k);
-      // 32-bit offsets of this lane's parameters: element j of band 0 at
-      // o0 + j_row * N, its band-1 pair half * N further
-      const uint32_t o0 = (uint32_t)(bm * 32 + 4 * (lane >> 5)) * (uint32_t)g.N + (uint32_t)n;
-      const uint32_t oh = (uint32_t)half * (uint32_t)g.N;
-      auto off = [&](int j) -> uint32_t {
-        return o0 + (uint32_t)(8 * (j >> 2) + (j & 3)) * (uint32_t)g.N;
-      };
-      // Chunks of kUpdChunk pairs, software-pipelined: the next chunk's loads go out
-      // before this chunk's noise arithmetic and stores (each parameter is read and
-      // written by this thread only), so its memory time overlaps the arithmetic.
-      constexpr int CJ = (BK >= 64 && UM == UM_RMS) ? kUpdChunkDeep : kUpdChunk;
-      float w0[CJ], a0[CJ], w1[CJ], a1[CJ];
-      constexpr int SH = PREC == P_BF16 ? SH_BF16 : PREC == P_FP8 ? SH_E4M3 : SH_NONE;
-      // compiled-in rms_prop: buffer-resource accesses, lane offset o0 plus the uniform
-      // row offset of element j (and oh for its band-1 pair)
-      const UpdRes rs = UM != UM_ANY ? make_res<SH>(up, (uint32_t)s.size[g.leaf]) : UpdRes{};
-      auto so = [&](int j) -> uint32_t { return (uint32_t)(8 * (j >> 2) + (j & 3)) * (uint32_t)g.N; };
-      auto load2 = [&](int j, float& wa, float& aa, float& wb, float& ab_) {
-        if constexpr (UM != UM_ANY) {
-          res_load(rs, o0, so(j), wa, aa);
-          res_load(rs, o0, so(j) + oh, wb, ab_);
-        } else {
-          upd_load<UM>(up, off(j), wa, aa);
-          upd_load<UM>(up, off(j) + oh, wb, ab_);
-        }
-      };
-#pragma unroll
-      for (int u = 0; u < CJ; ++u) load2(u, w0[u], a0[u], w1[u], a1[u]);
-#pragma unroll
-      for (int j0 = 0; j0 < 16; j0 += CJ) {
-        float nw0[CJ], na0[CJ], nw1[CJ], na1[CJ];
-        if (j0 + CJ < 16) {
-#pragma unroll
-          for (int u = 0; u < CJ; ++u) load2(j0 + CJ + u, nw0[u], na0[u], nw1[u], na1[u]);
-        }
-#pragma unroll
-        for (int u = 0; u < CJ; ++u) {
-          const int j = j0 + u;
-          const uint32_t i0 = off(j);
-          uint32_t b0, b1;
-          bits_pair(lk, S, i0, b0, b1);
-          upd_step<UM>(up, w0[u], a0[u], ab * acc0[j], bits_to_normal_fast(b0), lp, ke);
-          upd_step<UM>(up, w1[u], a1[u], ab * acc1[j], bits_to_normal_fast(b1), lp, ke);
-          if constexpr (UM != UM_ANY) {
-            res_store<SH, UM != UM_OBO>(up, rs, o0, so(j), w0[u], a0[u], wmax);
-            res_store<SH, UM != UM_OBO>(up, rs, o0, so(j) + oh, w1[u], a1[u], wmax);
-          } else {
-            upd_store<UM, SH>(up, i0, w0[u], a0[u], wmax);
-            upd_store<UM, SH>(up, i0 + oh, w1[u], a1[u], wmax);
-          }
-        }
-        if (j0 + CJ < 16) {
-#pragma unroll
-          for (int u = 0; u < CJ; ++u) {
-            w0[u] = nw0[u];
-            a0[u] = na0[u];
-            w1[u] = nw1[u];
-            a1[u] = na1[u];
-          }
-        }
-      }
-    } else {
-      float w0v[16], w1v[16];
-#pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        const int r = 8 * (j >> 2) + 4 * (lane >> 5) + (j & 3);
-        const int64_t i0 = (int64_t)(bm * 32 + r) * g.N + n;
-        w0v[j] = th[i0];
-        w1v[j] = th[i0 + (int64_t)half * g.N];
-      }
-      float* go = s.grad + base;
-#pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        const int r = 8 * (j >> 2) + 4 * (lane >> 5) + (j & 3);
-        const int64_t i0 = (int64_t)(bm * 32 + r) * g.N + n;
-        const int64_t i1 = i0 + (int64_t)half * g.N;
-        const float gs[2] = {ab * acc0[j], ab * acc1[j]};
-        const float wv[2] = {w0v[j], w1v[j]};
-        const int64_t ii[2] = {i0, i1};
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          float gg = gs[h];
-          if (s.has_prior) {
-            gg = gg + wv[h] * s.prior_inv_var;
-            lp += (s.prior_log_norm + (wv[h] * wv[h]) * s.prior_inv_var) / -2.0f;
-          }
-          go[ii[h]] = gg / s.temperature;
-        }
-      }
-    }
-    if (EPI == EPI_UPDATE && s.fp8 && g.leaf < 2) q_note_amax(s, c, Q_W1 + g.leaf, wmax);
-    const int64_t slot = (int64_t)c * s.nparts + g.part0 + bm * gy + bn;
-    const float tot = block_sum<GT>(lp, red);
-    if (threadIdx.x == 0) s.prior_part[slot] = tot;
-    if (EPI == EPI_UPDATE && UM != UM_RMS && s.mode != MLP_SGLD) {
-      const float kt = block_sum<GT>(ke, red);
-      if (threadIdx.x == 0) s.ke_part[slot] = kt;
-    }
-  }
-}
-
-template <int BK, int PREC, bool A_K, bool B_K, int EPI, int UM = UM_ANY>
-__global__ void __launch_bounds__(GT, EPI == EPI_UPDATE ? SGMC_UPD_WAVES : 1)
-    gemm_kernel(Gemm g, Step s) {
-  constexpr int EB = elem_bytes<PREC>();
-  __shared__ __attribute__((aligned(16))) uint8_t As[BM * BK * EB];
-  __shared__ __attribute__((aligned(16))) uint8_t Bs[BN * BK * EB];
-  __shared__ float red[GT / kWave];
-  gemm_tile<BK, PREC, A_K, B_K, EPI, UM>(
-      g, s, blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), gridDim.x,
-      gridDim.y, gridDim.z, As, Bs, red);
-}
-
-// The two parameter GEMMs of an evaluation in one launch (one k-tile depth): a 1-D grid
-// whose first ga.gx ga.gy C blocks take gW1's tiles (ga) in their linear order and the
-// rest gW2's (gb), so gW2's blocks fill the last round of gW1's instead of a launch and
-// a latency-bound round of their own.
-template <int BK, int PREC, bool A_K, bool B_K, int EPI, int UM = UM_ANY>
-__global__ void __launch_bounds__(GT, EPI == EPI_UPDATE ? SGMC_UPD_WAVES : 1)
-    gemm_pair_kernel(Gemm ga, Gemm gb, Step s, uint32_t gxa, uint32_t gya, uint32_t gxb,
-                     uint32_t gyb) {
-  constexpr int EB = elem_bytes<PREC>();
-  __shared__ __attribute__((aligned(16))) uint8_t As[BM * BK * EB];
-  __shared__ __attribute__((aligned(16))) uint8_t Bs[BN * BK * EB];
-  __shared__ float red[GT / kWave];
-  const uint32_t na = gxa * gya * (uint32_t)s.C;
-  if (blockIdx.x < na)
-    gemm_tile<BK, PREC, A_K, B_K, EPI, UM>(ga, s, blockIdx.x, gxa, gya, s.C, As, Bs, red);
-  else
-    gemm_tile<BK, PREC, A_K, B_K, EPI, UM>(gb, s, blockIdx.x - na, gxb, gyb, s.C, As, Bs, red);
 }
 
 // ------------------------------------------------------------------ head ------
@@ -1354,103 +742,8 @@ int sgmc_mlp_shadow(const float* theta, uint16_t* shadow, int64_t count, void* s
 
 namespace {
 
-// Split-K factor of the heuristic; a tuned GEMM may take 4 (the partial-product
-// workspace holds 4 C n max(H1, H2) floats).
+// Split-K factor of the heuristic; a tuned GEMM may take 4.
 constexpr int kMaxSplits = 2;
-
-template <int BK, int PREC, bool A_K, bool B_K, int EPI>
-void launch_gemm_bk(dim3 grid, Gemm g, const Step& s, hipStream_t st) {
-  // parameter updates of SGLD with rms_prop and of the two OBABO halves run the kernel
-  // with their rule compiled in
-  if constexpr (EPI == EPI_UPDATE) {
-    {
-      g.C = (int)grid.z;
-      if (s.mode == MLP_SGLD && s.rms) {
-        hipLaunchKernelGGL((gemm_kernel<BK, PREC, A_K, B_K, EPI, UM_RMS>), grid, dim3(GT), 0, st,
-                           g, s);
-        return;
-      }
-      if (s.mode == MLP_OBABO_BA) {
-        hipLaunchKernelGGL((gemm_kernel<BK, PREC, A_K, B_K, EPI, UM_OBA>), grid, dim3(GT), 0, st,
-                           g, s);
-        return;
-      }
-      if (s.mode == MLP_OBABO_BO) {
-        hipLaunchKernelGGL((gemm_kernel<BK, PREC, A_K, B_K, EPI, UM_OBO>), grid, dim3(GT), 0, st,
-                           g, s);
-        return;
-      }
-    }
-  }
-  g.C = (int)grid.z;
-  hipLaunchKernelGGL((gemm_kernel<BK, PREC, A_K, B_K, EPI>), grid, dim3(GT), 0, st, g, s);
-}
-
-// Launches GEMM `slot` with the k-tile depth and split-K factor of s.plan[slot].
-template <bool A_K, bool B_K, int EPI>
-void launch_gemm(dim3 grid, const Gemm& g, const Step& s, hipStream_t st, int slot) {
-  const int tv = s.plan[slot];
-  const bool deep = (tv >> 4) == 128;
-  if (s.fp32) {
-    launch_gemm_bk<32, P_F32, A_K, B_K, EPI>(grid, g, s, st);
-  } else if (s.fp8) {
-    if (deep) launch_gemm_bk<128, P_FP8, A_K, B_K, EPI>(grid, g, s, st);
-    else launch_gemm_bk<64, P_FP8, A_K, B_K, EPI>(grid, g, s, st);
-  } else {
-    if (deep) launch_gemm_bk<128, P_BF16, A_K, B_K, EPI>(grid, g, s, st);
-    else launch_gemm_bk<32, P_BF16, A_K, B_K, EPI>(grid, g, s, st);
-  }
-}
-
-// gW1 (ga, grid ra) and gW2 (gb, grid rb) in one launch at k-tile BK, with the update rule
-// compiled in as launch_gemm_bk chooses it.
-template <int BK, int PREC, int EPI>
-void launch_pair_bk(Gemm ga, dim3 ra, Gemm gb, dim3 rb, const Step& s, hipStream_t st) {
-  ga.C = gb.C = (int)ra.z;
-  const dim3 grid(ra.x * ra.y * ra.z + rb.x * rb.y * rb.z);
-  if constexpr (EPI == EPI_UPDATE) {
-    if (s.mode == MLP_SGLD && s.rms) {
-      hipLaunchKernelGGL((gemm_pair_kernel<BK, PREC, false, false, EPI, UM_RMS>), grid, dim3(GT),
-                         0, st, ga, gb, s, ra.x, ra.y, rb.x, rb.y);
-      return;
-    }
-    if (s.mode == MLP_OBABO_BA) {
-      hipLaunchKernelGGL((gemm_pair_kernel<BK, PREC, false, false, EPI, UM_OBA>), grid, dim3(GT),
-                         0, st, ga, gb, s, ra.x, ra.y, rb.x, rb.y);
-      return;
-    }
-    if (s.mode == MLP_OBABO_BO) {
-      hipLaunchKernelGGL((gemm_pair_kernel<BK, PREC, false, false, EPI, UM_OBO>), grid, dim3(GT),
-                         0, st, ga, gb, s, ra.x, ra.y, rb.x, rb.y);
-      return;
-    }
-  }
-  hipLaunchKernelGGL((gemm_pair_kernel<BK, PREC, false, false, EPI>), grid, dim3(GT), 0, st, ga,
-                     gb, s, ra.x, ra.y, rb.x, rb.y);
-}
-
-// The parameter GEMMs of an evaluation: gW2 (g4) and gW1 (g5) in one launch when their
-// plans agree (the same k-tile; they never split), else one launch each.
-template <int EPI>
-void launch_param_gemms(const Gemm& g4, dim3 r4, const Gemm& g5, dim3 r5, const Step& s,
-                        hipStream_t st) {
-  const int t4 = s.plan[SLOT_G4], t5 = s.plan[SLOT_G5];
-  if (t4 != t5 || (t5 & 15) != 1) {
-    launch_gemm<false, false, EPI>(r4, g4, s, st, SLOT_G4);
-    launch_gemm<false, false, EPI>(r5, g5, s, st, SLOT_G5);
-    return;
-  }
-  const int bk = t5 >> 4;
-  if (s.fp32) {
-    launch_pair_bk<32, P_F32, EPI>(g5, r5, g4, r4, s, st);
-  } else if (s.fp8) {
-    if (bk == 128) launch_pair_bk<128, P_FP8, EPI>(g5, r5, g4, r4, s, st);
-    else launch_pair_bk<64, P_FP8, EPI>(g5, r5, g4, r4, s, st);
-  } else {
-    if (bk == 128) launch_pair_bk<128, P_BF16, EPI>(g5, r5, g4, r4, s, st);
-    else launch_pair_bk<32, P_BF16, EPI>(g5, r5, g4, r4, s, st);
-  }
-}
 
 // Checks tune[] against the shapes: each nonzero entry is 16 k + s with k a k-tile of
 // the precision (bf16 32 / 128, e4m3 64 / 128, float32 32), s in {1, 2, 3, 4} (s > 1 for
@@ -1474,16 +767,12 @@ int check_tune(int D_in, int H1, int H2, int n, int precision, const int32_t* tu
 
 // The k-tile depth and split-K factor of each GEMM (16 k + s): tune[i] where set, else
 // the built-in choice --
-// - k-tiles of 128 when K allows (bf16, e4m3), so the register prefetch of the next tile
-//   has a whole tile of matrix work to land behind; 32 (bf16) or 64 (e4m3) otherwise;
-//   float32 always 32 (the transposed tiles of 4-byte elements fit one 4x4 block per
-//   thread). The bf16 parameter-update GEMMs (G4, G5 with update) take 32: their short
-//   K (the minibatch) gains little from deep tiles, and the smaller staging registers
-//   give three waves per SIMD instead of two to the update epilogue (+3.4% on a
-//   784-1024-1024 MLP). The k order of the matrix instructions is the same either way,
-//   so the results are identical.
+// - a k-tile of 128 when K allows (bf16, e4m3), 32 (bf16) or 64 (e4m3) otherwise; 32 for
+//   float32 and for the bf16 parameter updates. The k-tile takes part in which splits a
+//   code may name; the kernels' stages have one depth.
 // - forward GEMMs G1-G3 split K in two while the grid holds at most about four blocks
-//   per CU: they have few output tiles but long K. The parameter GEMMs never split.
+//   per CU: they have few output tiles but long K. The parameter GEMMs never split. The
+//   sums over K follow the split, so it decides last bits and is kept as it is.
 void plan_gemms(int D_in, int H1, int H2, int n, int C, int precision, int update,
                 const int32_t* tune, int* plan) {
   const int K[kSlots] = {D_in, H1, H2, n, n};
@@ -1685,9 +974,7 @@ int sgmc_mlp_step(const sgmc_mlp_state* st, int update, void* stream) {
           nullptr, 0, 0, nullptr, 0, nullptr, 0, 0, 0, L.g4_blocks};
   g4 = with_q(g4, Q_H1, Q_DA2, -1);
   g5 = with_q(g5, Q_X, Q_DA1, -1);
-  const dim3 r4(q.H1 / BM, q.H2 / BN, C), r5(q.D_in / BM, q.H1 / BN, C);
-  if (update) launch_param_gemms<EPI_UPDATE>(g4, r4, g5, r5, s, st_);
-  else launch_param_gemms<EPI_GRAD>(g4, r4, g5, r5, s, st_);
+  launch_param_gemms(g4, g5, s, st_);
   const dim3 col_grid((q.H2 + GT - 1) / GT + (q.H1 + GT - 1) / GT + 1, n / kStrip, C);
   if (s.fp32) hipLaunchKernelGGL(colsum_kernel<P_F32>, col_grid, dim3(GT), 0, st_, s);
   else if (s.fp8) hipLaunchKernelGGL(colsum_kernel<P_FP8>, col_grid, dim3(GT), 0, st_, s);

@@ -42,6 +42,20 @@ __device__ __forceinline__ uint8_t f2q(float v) {
 }
 __device__ __forceinline__ float q2f(uint8_t b) { return __builtin_amdgcn_cvt_f32_fp8((int)b, 0); }
 
+// Four values packed: bf16 (as f2bf) and e4m3 (as f2q).
+typedef uint32_t u32x2_4 __attribute__((ext_vector_type(2), aligned(4)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ u32x2_4 pack_bf(f32x4 v) {
+  return u32x2_4{(uint32_t)f2bf(v.x) | ((uint32_t)f2bf(v.y) << 16),
+                 (uint32_t)f2bf(v.z) | ((uint32_t)f2bf(v.w) << 16)};
+}
+__device__ __forceinline__ uint32_t pack_q(f32x4 v) {
+#pragma unroll
+  for (int u = 0; u < 4; ++u) v[u] = fminf(fmaxf(v[u], -448.0f), 448.0f);
+  const int lo = __builtin_amdgcn_cvt_pk_fp8_f32(v.x, v.y, 0, false);
+  return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(v.z, v.w, lo, true);
+}
+
 // fp8 tensors and their per-chain scale words: scales [0, 6), the scale the next weight
 // shadows are written with [6, 8), amax bit patterns [8, 14).
 enum Q8 { Q_X = 0, Q_H1 = 1, Q_DA2 = 2, Q_DA1 = 3, Q_W1 = 4, Q_W2 = 5 };
@@ -206,6 +220,9 @@ __device__ __forceinline__ void put_act(void* out, int64_t i, float v, bool q8, 
 // The activation GEMMs G1-G3 (bias and ReLU, or a ReLU mask where g.mask is set), K split
 // over `splits` groups of wavefronts (1 to 4).
 void launch_act_gemm(const Gemm& g, const Step& s, hipStream_t st, int splits);
+
+// The parameter GEMMs gW2 (g4) and gW1 (g5) with their update (s.update) or gradient.
+void launch_param_gemms(const Gemm& g4, const Gemm& g5, const Step& s, hipStream_t st);
 
 // Bytes per element of an activation tensor written with (q8, f32).
 __device__ __forceinline__ int act_bytes(bool q8, bool f32) { return f32 ? 4 : q8 ? 1 : 2; }

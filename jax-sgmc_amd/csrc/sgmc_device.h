@@ -249,8 +249,10 @@ __device__ __forceinline__ float bits_to_normal(uint32_t bits) {
 // divergent log branches).
 __device__ __forceinline__ float bits_to_normal_fast(uint32_t bits) {
   const float lo = -0.99999994f;
-  const float f = unit_float(bits);
-  const float x = fmaxf(lo, f * 2.0f + lo);
+  // unit_float(bits) * 2 + lo in three instructions: the exponent comes in by the shift, the
+  // product is exact in the multiply-add, and at f >= 0 the sum is never below lo
+  const float f = __uint_as_float(__builtin_amdgcn_alignbit(0x7Fu, bits, 9)) - 1.0f;
+  const float x = __builtin_fmaf(f, 2.0f, lo);
   const float x2 = x * x;
   const float w = -0.693147182f * __builtin_amdgcn_logf(1.0f - x2);
   // central branch (w < 5) on every lane; the tail (|x| > 0.9966, about 1 lane in 300)

@@ -264,7 +264,7 @@ class FusedMLP:
     problem (HIP events on the launch stream around `reps` back-to-back units after one
     warm-up unit): whole iterations for SGLD, one OBABO step (two evaluations, the unit
     OBABO and SGGMC iterations repeat) otherwise. The forward GEMMs one at a time, then the
-    two parameter GEMMs jointly (they share a launch at equal depths), starting from the
+    two parameter GEMMs jointly (they share a launch), starting from the
     built-in choice; a candidate replaces the current one only if it is faster by more
     than `min_gain`. Each timing starts from a snapshot of the engine's state (the
     iteration counter runs at most reps + 1 past it; the schedule tables clamp it),
@@ -308,8 +308,8 @@ class FusedMLP:
         if t < best * (1.0 - min_gain):
           best, best_code = t, code
       self.tune[slot] = best_code
-    # the parameter GEMMs jointly: gW2 runs in gW1's launch when both take the same
-    # k-tile, so their depths are not independent (tune_ms[(3, c4, c5)])
+    # the parameter GEMMs jointly: gW2 runs in gW1's launch,
+    # so they are timed together (tune_ms[(3, c4, c5)])
     best_pair = (self.tune[3], self.tune[4])
     self.tune_ms[(3,) + best_pair] = best
     for c4 in self.tile_candidates(3):
