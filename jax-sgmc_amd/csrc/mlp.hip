@@ -120,16 +120,6 @@ __global__ void __launch_bounds__(GT) gather_kernel(Step s) {
   if (lane == 0) s.lab[row] = valid ? s.labels[r] : -1;
 }
 
-// h2 (bf16, or float32 in fp32 mode) and its ReLU mask.
-__device__ __forceinline__ float h2_at(const Step& s, int64_t i) {
-  if (s.fp32) return reinterpret_cast<const float*>(s.h2)[i];
-  return bf2f(reinterpret_cast<const uint16_t*>(s.h2)[i]);
-}
-__device__ __forceinline__ bool h2_on(const Step& s, int64_t i) {
-  if (s.fp32) return mask_on<P_F32>(s.h2, i);
-  return mask_on<P_BF16>(s.h2, i);
-}
-
 // Reads an activation of tensor t (e4m3 tensors in fp8 mode, bf16 otherwise).
 __device__ __forceinline__ float get_act(const Step& s, int c, int t, const void* p, int64_t i) {
   if (s.fp32) return reinterpret_cast<const float*>(p)[i];
@@ -144,74 +134,123 @@ __device__ __forceinline__ float get_act(const Step& s, int c, int t, const void
 // and each W3 row read serves all of the wavefront's rows; otherwise W3 comes from global
 // memory. For every row the sums run in the same order either way: lane-partial sums
 // over the columns a = lane + 64 u in ascending u, then wave sums.
+// What bounds it: latency, then the vector ALU (8192 rows of H2 = 1024 read 17 MB, 3.3 us,
+// and take 4.3 us of multiplies and adds). So a batch of h2 is always in flight (the first
+// behind the staging of W3), the 10 R sums of a wavefront share their lane swaps (100
+// instructions for 40 sums where 40 separate ones take 320), and the softmax of row r runs
+// on lane r instead of R times on all: 36 -> 13 us per launch (4096 rows of H2 = 512: 16 ->
+// 10 us).
 constexpr int kW3Stride = NCLS + 1;
 
-template <bool W3S, int R>
-__global__ void __launch_bounds__(GT) head_kernel(Step s) {
-  extern __shared__ float w3s[];  // W3S: [H2][kW3Stride]
+// h2 element as loaded (bf16 or float32) and its value; the ReLU mask of the raw element.
+template <bool F32>
+__device__ __forceinline__ uint32_t h2_raw(const void* h2, int64_t i) {
+  if (F32) return reinterpret_cast<const uint32_t*>(h2)[i];
+  return reinterpret_cast<const uint16_t*>(h2)[i];
+}
+template <bool F32>
+__device__ __forceinline__ float h2_val(uint32_t raw) {
+  return __uint_as_float(F32 ? raw : raw << 16);
+}
+template <bool F32>
+__device__ __forceinline__ bool h2_on(uint32_t raw) {
+  return raw != 0 && !(raw & (F32 ? 0x80000000u : 0x8000u));
+}
+
+template <int PREC, bool W3S, int R, int NW>
+__global__ void __launch_bounds__(kWave* NW) head_kernel(Step s) {
+  constexpr bool F32 = PREC == P_F32;
+  constexpr int NB = 4;             // columns per lane and batch
+  constexpr int kZ = R * NCLS;      // logits of a wavefront
+  constexpr int kZ4 = (kZ + 3) / 4 * 4;
+  extern __shared__ float w3s[];    // W3S: [H2][kW3Stride]
+  __shared__ __attribute__((aligned(16))) float zs[NW][kZ4];
   const int c = blockIdx.y;
   const int lane = threadIdx.x & (kWave - 1);
+  const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
   const float* th = s.theta + (int64_t)c * s.P;
   const float* W3 = th + s.off[2];
   const float* b3 = th + s.off[5];
+  const int U = s.H2 / kWave;       // columns per lane (a multiple of 2)
+  const int j0 = (blockIdx.x * NW + wv) * R;  // s.n is a multiple of NW R
+  const int64_t row0 = (int64_t)c * s.n + j0;
+  uint32_t nx[R][NB];
+  auto fetch = [&](int u0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int u = 0; u < NB; ++u)
+        nx[r][u] = h2_raw<F32>(s.h2, (row0 + r) * s.H2 + lane + min(u0 + u, U - 1) * kWave);
+  };
+  fetch(0);
   if (W3S) {
     // 16 loads per thread go out before their LDS stores (indices past W3 are clamped
     // to its last element and not stored)
+    constexpr int kNT = kWave * NW;
     const int total = s.H2 * NCLS;
-    for (int i0 = threadIdx.x; i0 < total; i0 += 16 * GT) {
+    for (int i0 = threadIdx.x; i0 < total; i0 += 16 * kNT) {
       float v[16];
 #pragma unroll
-      for (int u = 0; u < 16; ++u) v[u] = W3[min(i0 + u * GT, total - 1)];
+      for (int u = 0; u < 16; ++u) v[u] = W3[min(i0 + u * kNT, total - 1)];
 #pragma unroll
       for (int u = 0; u < 16; ++u) {
-        const int i = i0 + u * GT;
+        const int i = i0 + u * kNT;
         if (i < total) w3s[(i / NCLS) * kW3Stride + i % NCLS] = v[u];
       }
     }
-    __syncthreads();
+    lds_sync();
   }
-  auto w3at = [&](int a, int k) -> float {
+  auto w3at = [&](int a, int k) __attribute__((always_inline)) -> float {
     return W3S ? w3s[a * kW3Stride + k] : W3[(int64_t)a * NCLS + k];
   };
-  const int j0 = (blockIdx.x * (GT / kWave) + threadIdx.x / kWave) * R;
-  if (j0 >= s.n) return;  // s.n is a multiple of 4 R: rows j0 .. j0 + R - 1 exist
-  const int64_t row0 = (int64_t)c * s.n + j0;
-  float z[R][NCLS];
+  float z[kZ4];
 #pragma unroll
-  for (int r = 0; r < R; ++r)
+  for (int i = 0; i < kZ4; ++i) z[i] = 0.f;
+  for (int u0 = 0; u0 < U; u0 += NB) {
+    uint32_t h[R][NB];
 #pragma unroll
-    for (int k = 0; k < NCLS; ++k) z[r][k] = 0.f;
-  // columns in batches of four per lane (then pairs: H2 is a multiple of 128); the h2
-  // loads of a batch go out together
-  auto zbatch = [&](int a0, auto nb) {
-    constexpr int NB = decltype(nb)::value;
-    float h[R][NB], w[NB][NCLS];
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int u = 0; u < NB; ++u) h[r][u] = nx[r][u];
+    fetch(u0 + NB < U ? u0 + NB : 0);  // at the end: the masks' first batch
 #pragma unroll
     for (int u = 0; u < NB; ++u) {
+      if (u == 2 && u0 + 2 >= U) break;
+      float w[NCLS];
 #pragma unroll
-      for (int r = 0; r < R; ++r) h[r][u] = h2_at(s, (row0 + r) * s.H2 + a0 + u * kWave);
-#pragma unroll
-      for (int k = 0; k < NCLS; ++k) w[u][k] = w3at(a0 + u * kWave, k);
-    }
-#pragma unroll
-    for (int u = 0; u < NB; ++u)
+      for (int k = 0; k < NCLS; ++k) w[k] = w3at(lane + (u0 + u) * kWave, k);
 #pragma unroll
       for (int r = 0; r < R; ++r)
 #pragma unroll
-        for (int k = 0; k < NCLS; ++k) z[r][k] += h[r][u] * w[u][k];
-  };
-  {
-    int a0 = lane;
-    for (; a0 + 3 * kWave < s.H2; a0 += 4 * kWave) zbatch(a0, std::integral_constant<int, 4>{});
-    for (; a0 < s.H2; a0 += 2 * kWave) zbatch(a0, std::integral_constant<int, 2>{});
+        for (int k = 0; k < NCLS; ++k) z[r * NCLS + k] += h2_val<F32>(h[r][u]) * w[k];
+    }
   }
-  const float cscale = ((float)(-s.N) / (float)s.n) / s.temperature;
-  float dl[R][NCLS];
+  // The wavefront sums of the kZ logits, the additions of wave_sum: the xor-32 and xor-16
+  // steps of two values share a lane swap, which leaves in row of 16 g, register j the
+  // value 4 j + 2 (g % 2) + g / 2.
+  float q[kZ4 / 4];
+  {
+    float p[kZ4 / 2];
 #pragma unroll
-  for (int r = 0; r < R; ++r) {
+    for (int i = 0; i < kZ4 / 2; ++i) p[i] = pair_add32(z[2 * i], z[2 * i + 1]);
+#pragma unroll
+    for (int j = 0; j < kZ4 / 4; ++j) q[j] = pair_add16(p[2 * j], p[2 * j + 1]);
+  }
+#pragma unroll
+  for (int j = 0; j < kZ4 / 4; ++j)
+    q[j] = ror_add<1>(ror_add<2>(ror_add<4>(ror_add<8>(q[j]))));
+  if ((lane & 15) == 0) {
+    const int g = lane >> 4;
+#pragma unroll
+    for (int j = 0; j < kZ4 / 4; ++j) zs[wv][4 * j + 2 * (g & 1) + (g >> 1)] = q[j];
+  }
+  __builtin_amdgcn_wave_barrier();
+  // lane r: softmax of row r (a wavefront's LDS accesses complete in order)
+  const float cscale = ((float)(-s.N) / (float)s.n) / s.temperature;
+  if (lane < R) {
     float zr[NCLS];
 #pragma unroll
-    for (int k = 0; k < NCLS; ++k) zr[k] = wave_sum(z[r][k]) + b3[k];
+    for (int k = 0; k < NCLS; ++k) zr[k] = zs[wv][lane * NCLS + k] + b3[k];
     float mx = zr[0];
 #pragma unroll
     for (int k = 1; k < NCLS; ++k) mx = fmaxf(mx, zr[k]);
@@ -219,63 +258,56 @@ __global__ void __launch_bounds__(GT) head_kernel(Step s) {
 #pragma unroll
     for (int k = 0; k < NCLS; ++k) se += expf(zr[k] - mx);
     const float lse = mx + logf(se);
-    int lab = s.lab[row0 + r];
-    if (s.full) {  // likelihood only; padding rows (label -1) contribute 0
-      const int lb = lab < 0 ? 0 : (lab >= NCLS ? NCLS - 1 : lab);
-      float zl = zr[0];
+    const int lab = s.lab[row0 + lane];
+    const int lb = lab < 0 ? 0 : (lab >= NCLS ? NCLS - 1 : lab);
+    float zl = zr[0];
 #pragma unroll
-      for (int k = 1; k < NCLS; ++k)
-        if (k == lb) zl = zr[k];
-      if (lane == 0) s.lik[row0 + r] = lab < 0 ? 0.0f : zl - lse;
-      continue;
-    }
-    lab = lab < 0 ? 0 : (lab >= NCLS ? NCLS - 1 : lab);
-    float zl = 0.f;
+    for (int k = 1; k < NCLS; ++k)
+      if (k == lb) zl = zr[k];
+    // the full pass wants the likelihood only; its padding rows (label -1) contribute 0
+    s.lik[row0 + lane] = s.full && lab < 0 ? 0.0f : zl - lse;
+    if (!s.full) {
 #pragma unroll
-    for (int k = 0; k < NCLS; ++k) {
-      const float p = expf(zr[k] - lse);
-      dl[r][k] = cscale * ((k == lab ? 1.0f : 0.0f) - p);
-      if (k == lab) zl = zr[k];
-    }
-    if (lane == 0) {
-      s.lik[row0 + r] = zl - lse;
-#pragma unroll
-      for (int k = 0; k < NCLS; ++k) s.dL[(row0 + r) * NCLS + k] = dl[r][k];
+      for (int k = 0; k < NCLS; ++k) {
+        const float d = cscale * ((k == lb ? 1.0f : 0.0f) - expf(zr[k] - lse));
+        s.dL[(row0 + lane) * NCLS + k] = d;
+        zs[wv][lane * NCLS + k] = d;
+      }
     }
   }
   if (s.full) return;
-  const float qs = s.fp8 ? s.q[(int64_t)c * kQWords + Q_DA2] : 1.0f;
+  __builtin_amdgcn_wave_barrier();
+  float dl[kZ];
+#pragma unroll
+  for (int i = 0; i < kZ; ++i) dl[i] = zs[wv][i];
+  const float qs = PREC == P_FP8 ? s.q[(int64_t)c * kQWords + Q_DA2] : 1.0f;
   float amax = 0.f;
-  auto dbatch = [&](int a0, auto nb) {
-    constexpr int NB = decltype(nb)::value;
-    float w[NB][NCLS];
-    bool on[R][NB];
+  for (int u0 = 0; u0 < U; u0 += NB) {
+    uint32_t h[R][NB];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int u = 0; u < NB; ++u) h[r][u] = nx[r][u];
+    if (u0 + NB < U) fetch(u0 + NB);
 #pragma unroll
     for (int u = 0; u < NB; ++u) {
+      if (u == 2 && u0 + 2 >= U) break;
+      const int a = lane + (u0 + u) * kWave;
+      float w[NCLS];
 #pragma unroll
-      for (int r = 0; r < R; ++r) on[r][u] = h2_on(s, (row0 + r) * s.H2 + a0 + u * kWave);
-#pragma unroll
-      for (int k = 0; k < NCLS; ++k) w[u][k] = w3at(a0 + u * kWave, k);
-    }
-#pragma unroll
-    for (int u = 0; u < NB; ++u) {
+      for (int k = 0; k < NCLS; ++k) w[k] = w3at(a, k);
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         float d = 0.f;
 #pragma unroll
-        for (int k = 0; k < NCLS; ++k) d += dl[r][k] * w[u][k];
-        const float v = on[r][u] ? d : 0.0f;
+        for (int k = 0; k < NCLS; ++k) d += dl[r * NCLS + k] * w[k];
+        const float v = h2_on<F32>(h[r][u]) ? d : 0.0f;
         amax = fmaxf(amax, fabsf(v));
-        put_act(s.da2, (row0 + r) * s.H2 + a0 + u * kWave, v, s.fp8 != 0, qs, s.fp32 != 0);
+        put_act(s.da2, (row0 + r) * s.H2 + a, v, PREC == P_FP8, qs, F32);
       }
     }
-  };
-  {
-    int a0 = lane;
-    for (; a0 + 3 * kWave < s.H2; a0 += 4 * kWave) dbatch(a0, std::integral_constant<int, 4>{});
-    for (; a0 < s.H2; a0 += 2 * kWave) dbatch(a0, std::integral_constant<int, 2>{});
   }
-  if (s.fp8) q_note_amax(s, c, Q_DA2, amax);
+  if (PREC == P_FP8) q_note_amax(s, c, Q_DA2, amax);
 }
 
 // ------------------------------------------------------- small-leaf sums -----
@@ -901,22 +933,32 @@ const void* gemm_weight(const Step& s, const sgmc_mlp_state& q, int l) {
   return q.shadow + s.off[l];
 }
 
-// The head over rows [0, n) of every chain: W3 through LDS while it fits in 64 KB; four
-// rows per wavefront when that still leaves two blocks per CU (measured: 3072-1024-1024,
-// 8192 rows, 46.8 against 55.4 us), else one (3072-512-512, 4096 rows: 17.3 against 31.1).
-void launch_head(const Step& s, hipStream_t st) {
+template <int PREC, int R, int NW>
+void launch_head_as(const Step& s, hipStream_t st) {
   const size_t lds = (size_t)s.H2 * kW3Stride * sizeof(float);
-  const int rows_per_block4 = (GT / kWave) * 4;
-  const bool four = (int64_t)s.C * s.n / rows_per_block4 >= 512;
-  const int per_block = (GT / kWave) * (four ? 4 : 1);
-  const dim3 grid(s.n / per_block, s.C);
-  if (lds <= 65536) {
-    if (four) hipLaunchKernelGGL((head_kernel<true, 4>), grid, dim3(GT), lds, st, s);
-    else hipLaunchKernelGGL((head_kernel<true, 1>), grid, dim3(GT), lds, st, s);
-  } else {
-    if (four) hipLaunchKernelGGL((head_kernel<false, 4>), grid, dim3(GT), 0, st, s);
-    else hipLaunchKernelGGL((head_kernel<false, 1>), grid, dim3(GT), 0, st, s);
-  }
+  const dim3 grid(s.n / (R * NW), s.C), block(kWave * NW);
+  if (lds <= 65536) hipLaunchKernelGGL((head_kernel<PREC, true, R, NW>), grid, block, lds, st, s);
+  else hipLaunchKernelGGL((head_kernel<PREC, false, R, NW>), grid, block, 0, st, s);
+}
+// Rows per wavefront and wavefronts per block: as many rows as still give every CU two
+// blocks of eight wavefronts (a block stages W3 once, a read of a W3 row serves all rows of
+// the wavefront), one row and four wavefronts when there are few. Measured, us per launch:
+// 8192 rows of H2 = 1024 (98 full passes and 20 evaluations): 4 x 8 13.1, 4 x 4 15.3,
+// 2 x 8 14.7, 2 x 4 21.5; 4096 rows of H2 = 512: 2 x 8 9.7, 2 x 4 11.1, 1 x 8 10.7,
+// 1 x 4 12.2.
+template <int PREC>
+void launch_head_by(const Step& s, hipStream_t st) {
+  const int64_t rows = (int64_t)s.C * s.n;
+  if (rows >= 8192) launch_head_as<PREC, 4, 8>(s, st);
+  else if (rows >= 4096) launch_head_as<PREC, 2, 8>(s, st);
+  else launch_head_as<PREC, 1, 4>(s, st);
+}
+
+// The head over rows [0, n) of every chain.
+void launch_head(const Step& s, hipStream_t st) {
+  if (s.fp32) launch_head_by<P_F32>(s, st);
+  else if (s.fp8) launch_head_by<P_FP8>(s, st);
+  else launch_head_by<P_BF16>(s, st);
 }
 
 // gather, forward GEMMs and the head (likelihood, and its backward unless s.full).

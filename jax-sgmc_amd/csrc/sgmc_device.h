@@ -353,6 +353,18 @@ __device__ __forceinline__ float xor16_add(float v) {
   const uint32_t a = lane_swap16(__float_as_uint(v), b);
   return __uint_as_float(a) + __uint_as_float(b);
 }
+// xor32_add / xor16_add of two values with one lane swap: lanes 0-31 (even rows of 16) get
+// a's sum, lanes 32-63 (odd rows) b's.
+__device__ __forceinline__ float pair_add32(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false,
+                                                  false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float pair_add16(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false,
+                                                  false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
 // v rotated by N lanes inside each row of 16 (the same lane as l ^ 8 for N = 8).
 template <int N>
 __device__ __forceinline__ uint32_t row_ror(uint32_t v) {

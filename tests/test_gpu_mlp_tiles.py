@@ -1,4 +1,4 @@
-"""Tile edges of the MLP engine's activation GEMMs (GPU).
+"""Tile edges of the MLP engine's GEMMs and head (GPU).
 
 Potential and gradient at shapes that reach every tile and split of the GEMMs and their
 remainders: K below one stage, K / splits that ends inside a stage (a half stage of e4m3 is
@@ -31,7 +31,9 @@ SHAPES = [
     ((192, 384, 384), 64, 1, (3, 3, 3)),       # three groups
     ((256, 256, 512), 128, 2, (4, 4, 4)),      # four groups
     ((128, 512, 512), 256, 8, (0, 0, 0)),      # 64 x 128 tiles
-    ((64, 1024, 1024), 512, 16, (1, 1, 1)),    # 128 x 128 tiles
+    ((64, 1024, 1024), 512, 16, (1, 1, 1)),    # 128 x 128 tiles; the head's largest blocks
+    ((128, 128, 384), 256, 16, (0, 0, 0)),     # the head at 4096 rows, columns in twos at the end
+    ((64, 128, 1536), 64, 2, (0, 0, 0)),       # the head with W3 past its LDS
 ]
 
 
