@@ -54,70 +54,100 @@ __device__ __forceinline__ void grad_param(const Step& s, const float* th, float
 
 
 // ------------------------------------------------------------------ gather ----
-// Xb[c][j] = bf16(X[idx_j]), lab[c][j] = labels[idx_j]; one wavefront per row.
-__global__ void __launch_bounds__(GT) gather_kernel(Step s) {
-  const int c = blockIdx.y;
-  if (s.update && blockIdx.x == 0 && threadIdx.x < NLEAF)
-    store_key(s.lkey + 2 * (c * NLEAF + threadIdx.x), derive_leaf_key(s, c, threadIdx.x));
-  const int j = blockIdx.x * (GT / kWave) + threadIdx.x / kWave;
-  if (j >= s.n) return;
+// Xb[c][j] = bf16(X[idx_j]), lab[c][j] = labels[idx_j]; one wavefront per row,
+// kGatherRows rows per block.
+// What bounds it: the rows' HBM reads (16 x 512 rows of 3072: 100 MB, 16 us at the 6.5 TB/s
+// of a random gather, 32 us measured behind an update's stores). The block's first
+// wavefront draws all its indices (five dependent Threefry blocks each, 500 instructions
+// that every wavefront ran for its own row), the e4m3 maximum costs a block one atomic at
+// most (with one per wavefront 512 of them queued on each chain's word: 67 us), and a
+// minibatch's rows are read with the non-temporal hint, which leaves the last-level cache
+// to the weights (16 x 256 rows: 24 -> 19 us, and the Xb W1 that follows 36 -> 30 us).
+// FULL: the rows of a full-data pass, the same for all chains; a wavefront reads its row
+// once for kGatherChains of them (16 x 512 rows: 10.9 us, with 1 chain 11.9, with 4 11.3).
+constexpr int kGatherRows = 8;
+constexpr int kGatherChains = 2;
+template <bool FULL>
+__global__ void __launch_bounds__(kGatherRows* kWave) gather_kernel(Step s) {
+  __shared__ int64_t rows[kGatherRows];
+  __shared__ float red[kGatherRows];
+  const int c0 = blockIdx.y * (FULL ? kGatherChains : 1);
+  const int c1 = FULL ? min(c0 + kGatherChains, s.C) : c0 + 1;
+  if (s.update && !FULL && blockIdx.x == 0 && threadIdx.x < NLEAF)
+    store_key(s.lkey + 2 * (c0 * NLEAF + threadIdx.x), derive_leaf_key(s, c0, threadIdx.x));
+  const int w = threadIdx.x / kWave;
+  const int j = blockIdx.x * kGatherRows + w;  // s.n is a multiple of kGatherRows
   const int lane = threadIdx.x & (kWave - 1);
   int64_t r;
   bool valid = true;
-  if (s.full) {  // rows row0 + j of the full-data pass; rows past N are zero
+  if (FULL) {  // rows row0 + j of the full-data pass; rows past N are zero
     r = s.row0 + j;
     valid = r < s.N;
     if (!valid) r = 0;
   } else {
-    Key next, sub, k1, k2;
-    split2(load_key(s.dkey + 2 * c), next, sub);
-    split2(sub, k1, k2);
-    const uint32_t span = (uint32_t)s.N;
-    r = (int64_t)draw_index(k1, k2, (uint32_t)s.n, (uint32_t)j, span, s.rmult, s.rmagic);
-    if (r < 0 || r >= s.N) r = 0;
+    if (threadIdx.x < kGatherRows) {
+      Key next, sub, k1, k2;
+      split2(load_key(s.dkey + 2 * c0), next, sub);
+      split2(sub, k1, k2);
+      const uint32_t span = (uint32_t)s.N;
+      r = (int64_t)draw_index(k1, k2, (uint32_t)s.n,
+                              (uint32_t)(blockIdx.x * kGatherRows + threadIdx.x), span, s.rmult,
+                              s.rmagic);
+      if (r < 0 || r >= s.N) r = 0;
+      rows[threadIdx.x] = r;
+    }
+    lds_sync();
+    r = rows[w];
   }
   const float* __restrict__ src = s.X + r * s.ldx;
-  const int64_t row = (int64_t)c * s.n + j;
   // kGatherBatch float4 loads per lane go out before their conversions and stores, so a
   // row costs D_in / (256 kGatherBatch) memory round trips instead of D_in / 256. The
   // loads are unconditional: offsets past the row are clamped to its last float4 (and
   // not stored), a row past N reads row 0 and is zeroed.
   constexpr int kStep = kWave * 4;
-  const float4 zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
-  auto rowcopy = [&](auto&& put) {
+  const f32x4 zero4{0.f, 0.f, 0.f, 0.f};
+  auto rowcopy = [&](auto&& put) __attribute__((always_inline)) {
     for (int f0 = lane * 4; f0 < s.D_in; f0 += kGatherBatch * kStep) {
-      float4 xs[kGatherBatch];
+      f32x4 xs[kGatherBatch];
 #pragma unroll
-      for (int u = 0; u < kGatherBatch; ++u)
-        xs[u] = *reinterpret_cast<const float4*>(src + min(f0 + u * kStep, s.D_in - 4));
+      for (int u = 0; u < kGatherBatch; ++u) {
+        const f32x4* p = reinterpret_cast<const f32x4*>(src + min(f0 + u * kStep, s.D_in - 4));
+        if constexpr (FULL) xs[u] = *p;
+        else xs[u] = __builtin_nontemporal_load(p);
+      }
 #pragma unroll
-      for (int u = 0; u < kGatherBatch; ++u)
-        if (f0 + u * kStep < s.D_in) put(f0 + u * kStep, valid ? xs[u] : zero4);
+      for (int u = 0; u < kGatherBatch; ++u) xs[u] = valid ? xs[u] : zero4;
+      for (int c = c0; c < c1; ++c) {
+        const int64_t row = ((int64_t)c * s.n + j) * s.D_in;
+        const float qs = s.fp8 ? s.q[(int64_t)c * kQWords + Q_X] : 1.0f;
+#pragma unroll
+        for (int u = 0; u < kGatherBatch; ++u)
+          if (f0 + u * kStep < s.D_in) put(row + f0 + u * kStep, xs[u], qs);
+      }
     }
   };
   if (s.fp8) {
-    const float qs = s.q[(int64_t)c * kQWords + Q_X];
-    uint8_t* __restrict__ dst = reinterpret_cast<uint8_t*>(s.Xb) + row * s.D_in;
+    uint8_t* __restrict__ dst = reinterpret_cast<uint8_t*>(s.Xb);
     float amax = 0.f;
-    rowcopy([&](int f, float4 x) {
+    rowcopy([&](int64_t i, f32x4 x, float qs) {
       amax = fmaxf(amax, fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w))));
-      const uint32_t v = (uint32_t)f2q(x.x * qs) | ((uint32_t)f2q(x.y * qs) << 8) |
-                         ((uint32_t)f2q(x.z * qs) << 16) | ((uint32_t)f2q(x.w * qs) << 24);
-      *reinterpret_cast<uint32_t*>(dst + f) = v;
+      *reinterpret_cast<uint32_t*>(dst + i) = pack_q(x * qs);
     });
-    q_note_amax(s, c, Q_X, amax);
+    if constexpr (FULL)
+      for (int c = c0; c < c1; ++c) q_note_amax(s, c, Q_X, amax);
+    else
+      q_note_amax_block(s, c0, Q_X, amax, red);
   } else if (s.fp32) {
-    float* __restrict__ dst = reinterpret_cast<float*>(s.Xb) + row * s.D_in;
-    rowcopy([&](int f, float4 x) { *reinterpret_cast<float4*>(dst + f) = x; });
+    float* __restrict__ dst = reinterpret_cast<float*>(s.Xb);
+    rowcopy([&](int64_t i, f32x4 x, float) { *reinterpret_cast<f32x4*>(dst + i) = x; });
   } else {
-    uint16_t* __restrict__ dst = reinterpret_cast<uint16_t*>(s.Xb) + row * s.D_in;
-    rowcopy([&](int f, float4 x) {
-      const uint32_t lo = (uint32_t)f2bf(x.x) | ((uint32_t)f2bf(x.y) << 16);
-      const uint32_t hi = (uint32_t)f2bf(x.z) | ((uint32_t)f2bf(x.w) << 16);
-      *reinterpret_cast<uint2*>(dst + f) = make_uint2(lo, hi);
+    uint16_t* __restrict__ dst = reinterpret_cast<uint16_t*>(s.Xb);
+    rowcopy([&](int64_t i, f32x4 x, float) {
+      *reinterpret_cast<u32x2_4*>(dst + i) = pack_bf(x);
     });
   }
-  if (lane == 0) s.lab[row] = valid ? s.labels[r] : -1;
+  if (lane == 0)
+    for (int c = c0; c < c1; ++c) s.lab[(int64_t)c * s.n + j] = valid ? s.labels[r] : -1;
 }
 
 // Reads an activation of tensor t (e4m3 tensors in fp8 mode, bf16 otherwise).
@@ -165,6 +195,7 @@ __global__ void __launch_bounds__(kWave* NW) head_kernel(Step s) {
   constexpr int kZ4 = (kZ + 3) / 4 * 4;
   extern __shared__ float w3s[];    // W3S: [H2][kW3Stride]
   __shared__ __attribute__((aligned(16))) float zs[NW][kZ4];
+  __shared__ float red[NW];
   const int c = blockIdx.y;
   const int lane = threadIdx.x & (kWave - 1);
   const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
@@ -307,7 +338,7 @@ __global__ void __launch_bounds__(kWave* NW) head_kernel(Step s) {
       }
     }
   }
-  if (PREC == P_FP8) q_note_amax(s, c, Q_DA2, amax);
+  if (PREC == P_FP8) q_note_amax_block(s, c, Q_DA2, amax, red);
 }
 
 // ------------------------------------------------------- small-leaf sums -----
@@ -964,8 +995,13 @@ void launch_head(const Step& s, hipStream_t st) {
 // gather, forward GEMMs and the head (likelihood, and its backward unless s.full).
 void launch_forward(const Step& s, const sgmc_mlp_state& q, hipStream_t st_) {
   const int C = q.C, n = q.n;
-  const dim3 rows_grid((n + 3) / 4, C);
-  hipLaunchKernelGGL(gather_kernel, rows_grid, dim3(GT), 0, st_, s);
+  const dim3 gblock(kGatherRows * kWave);
+  if (s.full)
+    hipLaunchKernelGGL(gather_kernel<true>,
+                       dim3(n / kGatherRows, (C + kGatherChains - 1) / kGatherChains), gblock, 0,
+                       st_, s);
+  else
+    hipLaunchKernelGGL(gather_kernel<false>, dim3(n / kGatherRows, C), gblock, 0, st_, s);
   const void* W1 = gemm_weight(s, q, 0);
   const void* W2 = gemm_weight(s, q, 1);
   Gemm g1{s.Xb, q.D_in, (int64_t)n * q.D_in, W1, q.H1, q.P, n, q.H1, q.D_in,

@@ -11,8 +11,8 @@
 // (the weights as they lie in theta) is staged as it is and read with the transposing LDS
 // loads: transposing 8x8 blocks in registers kept the vector ALU busier than the matrix
 // cores. Against register transposes, one stage and a partial-product array: 16 chains of
-// 3072-512-512 in bf16, the three GEMMs 83 -> 57 us; 3072-1024-1024 in e4m3, n = 512,
-// 138 -> 95 us; 4 chains of 3072-512-512 in float32 105 -> 62 us. The k order of the matrix instructions and of the sum over the groups does not
+// 3072-512-512 in bf16, the three GEMMs 83 -> 50 us (7 of them by the gather's loads); 3072-1024-1024 in e4m3, n = 512,
+// 138 -> 90 us; 4 chains of 3072-512-512 in float32 105 -> 62 us. The k order of the matrix instructions and of the sum over the groups does not
 // depend on the tile, so neither do the results.
 #include "mlp_tile.h"
 
@@ -218,19 +218,20 @@ void launch(const Gemm& g, const Step& s, hipStream_t st) {
                      dim3(gx * gy * (uint32_t)s.C), dim3(kWave * WM * WN * G), 0, st, g, s, gx, gy);
 }
 
-// Tile of a GEMM: the largest that still gives every CU a block (one resident block of
-// 96 KB for two groups, two of 64 KB for one), since a tile's operand traffic per output
-// falls with its edges. Measured, Xb W1 and H1 W2 of 16 chains together: e4m3
-// 3072-1024-1024, n = 512, one group: 128 x 128 (512 blocks) 71 us against 82 us with
-// 64 x 128; bf16 3072-512-512, n = 256, two groups: 64 x 128 (256 blocks) 47 us against
-// 54 us with 64 x 64. Float32 is bound by the matrix cores, and at few tiles by the number
-// of SIMDs that have one: 32 x 64 tiles at 4 chains take 52 us where one group per K half
-// in launches of their own took 81 us.
+// Tile of a GEMM: the largest that still gives every CU a block (one resident block of 96 or
+// 128 KB, two of 64 KB), since a tile's operand traffic per output falls with its edges.
+// Measured, Xb W1 and H1 W2 of 16 chains together: e4m3 3072-1024-1024, n = 512, one group:
+// 256 x 128 (256 blocks) 66 us, 128 x 128 (512 blocks) 71 us, 64 x 128 82 us; bf16
+// 3072-512-512, n = 256, two groups: 64 x 128 (256 blocks) 47 us, 64 x 64 54 us. Float32 is
+// bound by the matrix cores, and at few tiles by the number of SIMDs that have one: 32 x 64
+// tiles at 4 chains take 52 us where one group per K half in launches of their own took
+// 81 us.
 template <int PREC, bool B_K, int EPI>
 void dispatch(const Gemm& g, const Step& s, hipStream_t st, int splits) {
   const int64_t blocks = (int64_t)(g.M / 64) * (g.N / 128) * s.C;  // of 64 x 128
   if (splits == 1) {
-    if (g.M % 128 == 0 && blocks >= 1024) launch<PREC, 128, 128, 2, 2, 1, B_K, EPI>(g, s, st);
+    if (g.M % 256 == 0 && blocks >= 1024) launch<PREC, 256, 128, 4, 2, 1, B_K, EPI>(g, s, st);
+    else if (g.M % 128 == 0 && blocks >= 1024) launch<PREC, 128, 128, 2, 2, 1, B_K, EPI>(g, s, st);
     else if (blocks >= 256) launch<PREC, 64, 128, 2, 2, 1, B_K, EPI>(g, s, st);
     else launch<PREC, 64, 64, 2, 2, 1, B_K, EPI>(g, s, st);
   } else if (splits == 2) {

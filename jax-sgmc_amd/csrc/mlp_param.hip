@@ -208,7 +208,8 @@ __device__ __forceinline__ void param_tile(const Gemm& g, const Step& s, uint32_
       }
     }
   }
-  if constexpr (EPI == EPI_UPDATE && F8) q_note_amax(s, c, Q_W1 + g.leaf, wmax);
+  if constexpr (EPI == EPI_UPDATE && F8)
+    if (UM != UM_OBO) q_note_amax_block(s, c, Q_W1 + g.leaf, wmax, red);
   const int64_t slot = (int64_t)c * s.nparts + g.part0 + bm * (int)gy + bn;
   const float tot = block_sum<GT>(lp, red);
   if (threadIdx.x == 0) s.prior_part[slot] = tot;

@@ -3,7 +3,7 @@
 Potential and gradient at shapes that reach every tile and split of the GEMMs and their
 remainders: K below one stage, K / splits that ends inside a stage (a half stage of e4m3 is
 64 values, of bf16 32), an odd number of stages, one to four groups over K, and the largest
-tile (128 x 128, 16 chains). The reference is the evaluation in float64 with the operands
+tile (256 x 128, 16 chains). The reference is the evaluation in float64 with the operands
 rounded where the engine rounds them (bf16, or e4m3 at the engine's scales; nowhere for
 float32): what is left is float32 accumulation and, layer by layer, the operands that its
 differences move over a rounding boundary. Tolerances: the engine's at its benchmark shapes
@@ -31,7 +31,8 @@ SHAPES = [
     ((192, 384, 384), 64, 1, (3, 3, 3)),       # three groups
     ((256, 256, 512), 128, 2, (4, 4, 4)),      # four groups
     ((128, 512, 512), 256, 8, (0, 0, 0)),      # 64 x 128 tiles
-    ((64, 1024, 1024), 512, 16, (1, 1, 1)),    # 128 x 128 tiles; the head's largest blocks
+    ((64, 1024, 1024), 512, 16, (1, 1, 1)),    # 256 x 128 tiles; the head's largest blocks
+    ((64, 1024, 1024), 384, 22, (1, 1, 1)),    # 128 x 128 tiles
     ((128, 128, 384), 256, 16, (0, 0, 0)),     # the head at 4096 rows, columns in twos at the end
     ((64, 128, 1536), 64, 2, (0, 0, 0)),       # the head with W3 past its LDS
 ]
