@@ -55,7 +55,7 @@ __device__ __forceinline__ void grad_param(const Step& s, const float* th, float
 
 // ------------------------------------------------------------------ gather ----
 // Xb[c][j] = bf16(X[idx_j]), lab[c][j] = labels[idx_j]; one wavefront per row,
-// kGatherRows rows per block.
+// ROWS rows per block.
 // What bounds it: the rows' HBM reads (16 x 512 rows of 3072: 100 MB, 16 us at the 6.5 TB/s
 // of a random gather, 32 us measured behind an update's stores). The block's first
 // wavefront draws all its indices (five dependent Threefry blocks each, 500 instructions
@@ -65,18 +65,18 @@ __device__ __forceinline__ void grad_param(const Step& s, const float* th, float
 // to the weights (16 x 256 rows: 24 -> 19 us, and the Xb W1 that follows 36 -> 30 us).
 // FULL: the rows of a full-data pass, the same for all chains; a wavefront reads its row
 // once for kGatherChains of them (16 x 512 rows: 10.9 us, with 1 chain 11.9, with 4 11.3).
-constexpr int kGatherRows = 8;
 constexpr int kGatherChains = 2;
-template <bool FULL>
-__global__ void __launch_bounds__(kGatherRows* kWave) gather_kernel(Step s) {
-  __shared__ int64_t rows[kGatherRows];
-  __shared__ float red[kGatherRows];
+template <bool FULL, int ROWS>
+__global__ void __launch_bounds__(ROWS* kWave) gather_kernel(Step s) {
+  __shared__ int64_t rows[ROWS];
+  __shared__ float red[ROWS];
+  __shared__ double red_d[ROWS];
   const int c0 = blockIdx.y * (FULL ? kGatherChains : 1);
   const int c1 = FULL ? min(c0 + kGatherChains, s.C) : c0 + 1;
   if (s.update && !FULL && blockIdx.x == 0 && threadIdx.x < NLEAF)
     store_key(s.lkey + 2 * (c0 * NLEAF + threadIdx.x), derive_leaf_key(s, c0, threadIdx.x));
   const int w = threadIdx.x / kWave;
-  const int j = blockIdx.x * kGatherRows + w;  // s.n is a multiple of kGatherRows
+  const int j = blockIdx.x * ROWS + w;  // s.n is a multiple of ROWS
   const int lane = threadIdx.x & (kWave - 1);
   int64_t r;
   bool valid = true;
@@ -85,13 +85,13 @@ __global__ void __launch_bounds__(kGatherRows* kWave) gather_kernel(Step s) {
     valid = r < s.N;
     if (!valid) r = 0;
   } else {
-    if (threadIdx.x < kGatherRows) {
+    if (threadIdx.x < ROWS) {
       Key next, sub, k1, k2;
       split2(load_key(s.dkey + 2 * c0), next, sub);
       split2(sub, k1, k2);
       const uint32_t span = (uint32_t)s.N;
       r = (int64_t)draw_index(k1, k2, (uint32_t)s.n,
-                              (uint32_t)(blockIdx.x * kGatherRows + threadIdx.x), span, s.rmult,
+                              (uint32_t)(blockIdx.x * ROWS + threadIdx.x), span, s.rmult,
                               s.rmagic);
       if (r < 0 || r >= s.N) r = 0;
       rows[threadIdx.x] = r;
@@ -145,6 +145,20 @@ __global__ void __launch_bounds__(kGatherRows* kWave) gather_kernel(Step s) {
     rowcopy([&](int64_t i, f32x4 x, float) {
       *reinterpret_cast<u32x2_4*>(dst + i) = pack_bf(x);
     });
+  }
+  if constexpr (FULL) {
+    // the chunk before this one: its likelihoods, which the head behind this launch
+    // overwrites, go to the pass's float64 sum (fixed order); the first chunk clears it
+    if (blockIdx.x == 0) {
+      for (int c = c0; c < c1; ++c) {
+        double t = 0.0;
+        if (s.row0 > 0)
+          for (int i = threadIdx.x; i < s.n; i += ROWS * kWave)
+            t += (double)s.lik[(int64_t)c * s.n + i];
+        t = block_sum_d<ROWS * kWave>(t, red_d);
+        if (threadIdx.x == 0) s.facc[c] = s.row0 > 0 ? s.facc[c] + t : 0.0;
+      }
+    }
   }
   if (lane == 0)
     for (int c = c0; c < c1; ++c) s.lab[(int64_t)c * s.n + j] = valid ? s.labels[r] : -1;
@@ -435,16 +449,6 @@ __global__ void __launch_bounds__(GT) small_kernel(Step s, int part0) {
   if (p < total) {
     int leaf;
     int64_t i;
-    const int strips = s.n / kStrip;
-    const float* cp = s.col_part + (int64_t)c * strips * total + p;
-    float gsum = 0.f;
-    for (int t = 0; t < strips; t += 8) {
-      float x[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) x[u] = t + u < strips ? cp[(int64_t)(t + u) * total] : 0.f;
-#pragma unroll
-      for (int u = 0; u < 8; ++u) gsum += x[u];
-    }
     if (p < nW3) {
       leaf = 2;
       i = p;
@@ -459,12 +463,26 @@ __global__ void __launch_bounds__(GT) small_kernel(Step s, int part0) {
       i = p - nW3 - s.H1 - s.H2;
     }
     const int64_t base = (int64_t)c * s.P + s.off[leaf];
+    // the parameter's state and its key are in flight with the first strips' sums
+    const Upd up = make_upd(s, c, leaf, base, cf);
+    float wmax = 0.f, w = 0.f, aux = 0.f;
+    Key lk{};
     if (s.update) {
-      const Key lk = leaf_key(s, c, leaf);
-      const float xi = bits_to_normal_fast(bits_word(lk, (uint32_t)s.size[leaf], (uint32_t)i));
-      float wmax = 0.f, w, aux;
-      const Upd up = make_upd(s, c, leaf, base, cf);
+      lk = leaf_key(s, c, leaf);
       upd_load(up, (uint32_t)i, w, aux);
+    }
+    const int strips = s.n / kStrip;
+    const float* cp = s.col_part + (int64_t)c * strips * total + p;
+    float gsum = 0.f;
+    for (int t = 0; t < strips; t += 8) {
+      float x[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) x[u] = t + u < strips ? cp[(int64_t)(t + u) * total] : 0.f;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) gsum += x[u];
+    }
+    if (s.update) {
+      const float xi = bits_to_normal_fast(bits_word(lk, (uint32_t)s.size[leaf], (uint32_t)i));
       upd_step(up, w, aux, gsum, xi, lp, ke);
       upd_store(up, (uint32_t)i, w, aux, wmax);
     } else {
@@ -480,18 +498,36 @@ __global__ void __launch_bounds__(GT) small_kernel(Step s, int part0) {
     if (threadIdx.x == 0) publish(s.ke_part + slot, kt);
   }
   if (!arrive_last(s.counters + c, gridDim.x, &flag)) return;
+  // One memory round trip for all the tail reads: the records and likelihoods go out
+  // together, and the next keys are derived behind them.
+  Key k_next{}, d_next{};
   double kin = 0.0;
-  if (obabo) {
-    for (int q = threadIdx.x; q < s.nparts; q += GT)
-      kin += (double)consume(s.ke_part + (int64_t)c * s.nparts + q);
-    kin = block_sum_d<GT>(kin, red_d);
+  float lsum = 0.f, prior = 0.f;
+  for (int q0 = threadIdx.x; q0 < max(s.nparts, s.n); q0 += 4 * GT) {
+    float xk[4], xl[4], xp[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int q = q0 + u * GT;
+      xp[u] = q < s.nparts ? consume(s.prior_part + (int64_t)c * s.nparts + q) : 0.f;
+      xk[u] = obabo && q < s.nparts ? consume(s.ke_part + (int64_t)c * s.nparts + q) : 0.f;
+      xl[u] = q < s.n ? s.lik[(int64_t)c * s.n + q] : 0.f;
+    }
+    if (q0 == 0 && s.update) {
+      Key a, b;
+      const Key k0 = load_key(s.key + 2 * c), d0 = load_key(s.dkey + 2 * c);
+      split2(d0, d_next, a);
+      if (obabo) split3(k0, k_next, a, b);
+      else split2(k0, k_next, a);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      prior += xp[u];
+      kin += (double)xk[u];
+      lsum += xl[u];
+    }
   }
-  float lsum = 0.f;
-  for (int r = threadIdx.x; r < s.n; r += GT) lsum += s.lik[(int64_t)c * s.n + r];
+  if (obabo) kin = block_sum_d<GT>(kin, red_d);
   lsum = block_sum<GT>(lsum, red);
-  float prior = 0.f;
-  for (int q = threadIdx.x; q < s.nparts; q += GT)
-    prior += consume(s.prior_part + (int64_t)c * s.nparts + q);
   prior = block_sum<GT>(prior, red);
   if (threadIdx.x == 0) {
     const float mean = lsum / (float)s.n;
@@ -499,18 +535,14 @@ __global__ void __launch_bounds__(GT) small_kernel(Step s, int part0) {
     if (obabo) {
       // ObaboState bookkeeping (integrator.py:203-273): the step's potential is the mean
       // of its two evaluations; the key advances once per step, the data key per draw.
-      Key next, sub;
-      split2(load_key(s.dkey + 2 * c), next, sub);
-      store_key(s.dkey + 2 * c, next);
+      store_key(s.dkey + 2 * c, d_next);
       if (s.mode == MLP_OBABO_BA) {
         s.U_half[c] = Uc;
         s.ke[2 * c] += 0.5 * kin;
       } else {
         s.U[c] = 0.5f * (s.U_half[c] + Uc);
         s.ke[2 * c + 1] += 0.5 * kin;
-        Key a, b, cc;
-        split3(load_key(s.key + 2 * c), a, b, cc);
-        store_key(s.key + 2 * c, a);
+        store_key(s.key + 2 * c, k_next);
       }
     } else {
       s.U[c] = Uc;
@@ -520,16 +552,21 @@ __global__ void __launch_bounds__(GT) small_kernel(Step s, int part0) {
       // written by this update carries the scale it was written with
       float* qc = s.q + (int64_t)c * kQWords;
       unsigned* am = reinterpret_cast<unsigned*>(qc + 8);
+      float a[6], next[2];
+#pragma unroll
+      for (int t = 0; t < 6; ++t) a[t] = __uint_as_float(am[t]);
+      next[0] = qc[6];
+      next[1] = qc[7];
+#pragma unroll
       for (int t = Q_X; t <= Q_DA1; ++t) {
-        const float a = __uint_as_float(am[t]);
-        if (a > 0.0f) qc[t] = kQTarget / a;
+        if (a[t] > 0.0f) qc[t] = kQTarget / a[t];
         am[t] = 0u;
       }
       if (s.update) {
+#pragma unroll
         for (int l = 0; l < 2; ++l) {
-          qc[Q_W1 + l] = qc[6 + l];
-          const float a = __uint_as_float(am[Q_W1 + l]);
-          if (a > 0.0f) qc[6 + l] = kQTarget / a;
+          qc[Q_W1 + l] = next[l];
+          if (a[Q_W1 + l] > 0.0f) qc[6 + l] = kQTarget / a[Q_W1 + l];
           am[Q_W1 + l] = 0u;
         }
       }
@@ -537,11 +574,8 @@ __global__ void __launch_bounds__(GT) small_kernel(Step s, int part0) {
     if (s.update && !obabo) {
       const int ss = s.save_slot ? s.save_slot[it] : -1;
       if (ss >= 0 && ss < s.n_slots && s.samples_U) s.samples_U[(int64_t)c * s.n_slots + ss] = Uc;
-      Key next, sub;
-      split2(load_key(s.key + 2 * c), next, sub);
-      store_key(s.key + 2 * c, next);
-      split2(load_key(s.dkey + 2 * c), next, sub);
-      store_key(s.dkey + 2 * c, next);
+      store_key(s.key + 2 * c, k_next);
+      store_key(s.dkey + 2 * c, d_next);
       // the last chain advances the iteration counter (read by the next launch)
       const unsigned prev = atomicAdd(s.done, 1u);
       if (prev == (unsigned)s.C - 1) {
@@ -616,24 +650,11 @@ __global__ void __launch_bounds__(GT) w_quant_kernel(Step s) {
 }
 
 // ------------------------------------------------------ full-data potential ----
-__global__ void __launch_bounds__(GT) zero_d_kernel(double* a, int n) {
-  const int i = blockIdx.x * GT + threadIdx.x;
-  if (i < n) a[i] = 0.0;
-}
-
-// acc[c] += sum of the pass's per-row likelihoods in float64 (fixed order).
-__global__ void __launch_bounds__(GT) full_acc_kernel(Step s, double* acc) {
-  __shared__ double red[GT / kWave];
-  const int c = blockIdx.x;
-  double t = 0.0;
-  for (int r = threadIdx.x; r < s.n; r += GT) t += (double)s.lik[(int64_t)c * s.n + r];
-  t = block_sum_d<GT>(t, red);
-  if (threadIdx.x == 0) acc[c] += t;
-}
-
-// out[c] = (-acc[c] - log p(theta_c)) / T with the float64 Gaussian log prior; grid
-// (kFinalBlocks, C), the chain's last-arriving block combines the block sums.
-__global__ void __launch_bounds__(GT) full_final_kernel(Step s, const double* acc, double* out) {
+// out[c] = (-likelihood - log p(theta_c)) / T with the float64 Gaussian log prior; the
+// likelihood is facc plus the last chunk's rows. Grid (kFinalBlocks, C), the chain's
+// last-arriving block combines the block sums. The parameters are read 16 bytes at a time,
+// eight reads in flight (16 chains of 4.2 M, 268 MB: 130 -> 57 us).
+__global__ void __launch_bounds__(GT) full_final_kernel(Step s, double* out) {
   __shared__ double red[GT / kWave];
   __shared__ int flag;
   const int c = blockIdx.y;
@@ -641,11 +662,25 @@ __global__ void __launch_bounds__(GT) full_final_kernel(Step s, const double* ac
   if (s.has_prior) {
     const double iv = (double)s.prior_inv_var, ln = (double)s.prior_log_norm;
     const float* th = s.theta + (int64_t)c * s.P;
-    for (int64_t i = (int64_t)blockIdx.x * GT + threadIdx.x; i < s.P;
-         i += (int64_t)gridDim.x * GT) {
-      const double w = (double)th[i];
-      lp += (ln + w * w * iv) / -2.0;
+    constexpr int kIn = 8;  // reads in flight
+    const int64_t quads = s.P / 4, step = (int64_t)gridDim.x * GT;
+    const int64_t t0 = (int64_t)blockIdx.x * GT + threadIdx.x;
+    auto add = [&](float wf) __attribute__((always_inline)) {
+      const double w = (double)wf;
+      lp += (ln + w * w * iv) * -0.5;
+    };
+    for (int64_t q0 = t0; q0 < quads; q0 += kIn * step) {
+      f32x4u x[kIn];
+#pragma unroll
+      for (int u = 0; u < kIn; ++u)
+        x[u] = *reinterpret_cast<const f32x4u*>(th + 4 * min(q0 + u * step, quads - 1));
+#pragma unroll
+      for (int u = 0; u < kIn; ++u)
+        if (q0 + u * step < quads)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) add(x[u][e]);
     }
+    if (4 * quads + t0 < s.P) add(th[4 * quads + t0]);  // the last P % 4
   }
   lp = block_sum_d<GT>(lp, red);
   if (threadIdx.x == 0) publish(s.fin_part + (int64_t)c * gridDim.x + blockIdx.x, lp);
@@ -653,8 +688,11 @@ __global__ void __launch_bounds__(GT) full_final_kernel(Step s, const double* ac
   double t = 0.0;
   for (int b = threadIdx.x; b < (int)gridDim.x; b += GT)
     t += consume(s.fin_part + (int64_t)c * gridDim.x + b);
+  double lk = 0.0;
+  for (int r = threadIdx.x; r < s.n; r += GT) lk += (double)s.lik[(int64_t)c * s.n + r];
   t = block_sum_d<GT>(t, red);
-  if (threadIdx.x == 0) out[c] = (-acc[c] - t) / (double)s.temperature;
+  lk = block_sum_d<GT>(lk, red);
+  if (threadIdx.x == 0) out[c] = (-(s.facc[c] + lk) - t) / (double)s.temperature;
 }
 
 // ----------------------------------------------------------------- SGGMC MH ----
@@ -692,24 +730,48 @@ __global__ void __launch_bounds__(GT) mh_kernel(Step s, MH m) {
   float* moo = m.mom_old + (int64_t)c * s.P;
   uint16_t* sh = s.fp32 ? nullptr : s.shadow + (int64_t)c * s.P;
   float* smp = save ? s.samples + ((int64_t)c * s.n_slots + slot) * s.P : nullptr;
-  for (int64_t i = (int64_t)blockIdx.x * GT + threadIdx.x; i < s.P;
-       i += (int64_t)gridDim.x * GT) {
-    float w;
-    if (accept) {
-      w = th[i];
-      tho[i] = w;
-      moo[i] = mo[i];
-    } else {
-      w = tho[i];
-      th[i] = w;
-      mo[i] = moo[i];
-      if (s.fp8 && i < s.off[2]) {
-        const int l = i < s.off[1] ? 0 : 1;
-        s.shadow8[(int64_t)c * s.P + i] = f2q(w * s.q[(int64_t)c * kQWords + Q_W1 + l]);
-      } else if (!s.fp32) {
-        sh[i] = f2bf(w);
-      }
+  auto shadow = [&](int64_t i, float w) __attribute__((always_inline)) {
+    if (s.fp8 && i < s.off[2]) {
+      const int l = i < s.off[1] ? 0 : 1;
+      s.shadow8[(int64_t)c * s.P + i] = f2q(w * s.q[(int64_t)c * kQWords + Q_W1 + l]);
+    } else if (!s.fp32) {
+      sh[i] = f2bf(w);
     }
+  };
+  // the kept pair goes from (th, mo) to (tho, moo) or back, 16 bytes at a time, with the
+  // reads of four quads in flight (16 chains of 4.2 M, 1.07 GB: 327 -> 229 us)
+  const float* ws = accept ? th : tho;
+  const float* ms = accept ? mo : moo;
+  float* wd = accept ? tho : th;
+  float* md = accept ? moo : mo;
+  constexpr int kIn = 4;
+  const int64_t quads = s.P / 4, step = (int64_t)gridDim.x * GT;
+  const int64_t t0 = (int64_t)blockIdx.x * GT + threadIdx.x;
+  for (int64_t q0 = t0; q0 < quads; q0 += kIn * step) {
+    f32x4u w[kIn], m4[kIn];
+#pragma unroll
+    for (int u = 0; u < kIn; ++u) {
+      const int64_t i = 4 * min(q0 + u * step, quads - 1);
+      w[u] = *reinterpret_cast<const f32x4u*>(ws + i);
+      m4[u] = *reinterpret_cast<const f32x4u*>(ms + i);
+    }
+#pragma unroll
+    for (int u = 0; u < kIn; ++u) {
+      const int64_t i = 4 * (q0 + u * step);
+      if (i >= 4 * quads) break;
+      *reinterpret_cast<f32x4u*>(wd + i) = w[u];
+      *reinterpret_cast<f32x4u*>(md + i) = m4[u];
+      if (!accept)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) shadow(i + e, w[u][e]);
+      if (save) *reinterpret_cast<f32x4u*>(smp + i) = w[u];
+    }
+  }
+  for (int64_t i = 4 * quads + t0; i < s.P; i += step) {  // the last P % 4
+    const float w = ws[i];
+    wd[i] = w;
+    md[i] = ms[i];
+    if (!accept) shadow(i, w);
     if (save) smp[i] = w;
   }
   if (!arrive_last(s.counters + c, gridDim.x, &flag)) return;
@@ -927,6 +989,7 @@ int make_step(const sgmc_mlp_state* st, int update, Layout& L, Step& s) {
   s.ke_part = reinterpret_cast<float*>(w + L.ke);
   s.col_part = reinterpret_cast<float*>(w + L.col);
   s.fin_part = reinterpret_cast<double*>(w + L.fin);
+  s.facc = reinterpret_cast<double*>(w + L.facc);
   s.nparts = L.nparts;
   s.U = q.U; s.grad = q.grad;
   s.samples = q.samples; s.samples_U = q.samples_U; s.n_slots = q.n_slots;
@@ -995,13 +1058,16 @@ void launch_head(const Step& s, hipStream_t st) {
 // gather, forward GEMMs and the head (likelihood, and its backward unless s.full).
 void launch_forward(const Step& s, const sgmc_mlp_state& q, hipStream_t st_) {
   const int C = q.C, n = q.n;
-  const dim3 gblock(kGatherRows * kWave);
+  // eight rows per block share a draw and an atomic; two while eight would leave CUs without
+  // a block (4 x 256 rows: 9.9 us for 11.7)
   if (s.full)
-    hipLaunchKernelGGL(gather_kernel<true>,
-                       dim3(n / kGatherRows, (C + kGatherChains - 1) / kGatherChains), gblock, 0,
+    hipLaunchKernelGGL((gather_kernel<true, 8>),
+                       dim3(n / 8, (C + kGatherChains - 1) / kGatherChains), dim3(8 * kWave), 0,
                        st_, s);
+  else if ((int64_t)C * n >= 4096)
+    hipLaunchKernelGGL((gather_kernel<false, 8>), dim3(n / 8, C), dim3(8 * kWave), 0, st_, s);
   else
-    hipLaunchKernelGGL(gather_kernel<false>, dim3(n / kGatherRows, C), gblock, 0, st_, s);
+    hipLaunchKernelGGL((gather_kernel<false, 2>), dim3(n / 2, C), dim3(2 * kWave), 0, st_, s);
   const void* W1 = gemm_weight(s, q, 0);
   const void* W2 = gemm_weight(s, q, 1);
   Gemm g1{s.Xb, q.D_in, (int64_t)n * q.D_in, W1, q.H1, q.P, n, q.H1, q.D_in,
@@ -1088,15 +1154,12 @@ int sgmc_mlp_full_potential(const sgmc_mlp_state* st, double* out, void* stream)
   SGMC_REQUIRE(out, SGMC_E_ARG, "sgmc_mlp_full_potential: null output");
   const sgmc_mlp_state& q = *st;
   hipStream_t st_ = as_stream(stream);
-  double* acc = reinterpret_cast<double*>(static_cast<uint8_t*>(q.work) + L.facc);
-  hipLaunchKernelGGL(zero_d_kernel, dim3((q.C + GT - 1) / GT), dim3(GT), 0, st_, acc, q.C);
   s.full = 1;
   for (int64_t r0 = 0; r0 < q.N; r0 += q.n) {
     s.row0 = r0;
     launch_forward(s, q, st_);
-    hipLaunchKernelGGL(full_acc_kernel, dim3(q.C), dim3(GT), 0, st_, s, acc);
   }
-  hipLaunchKernelGGL(full_final_kernel, dim3(kFinalBlocks, q.C), dim3(GT), 0, st_, s, acc, out);
+  hipLaunchKernelGGL(full_final_kernel, dim3(kFinalBlocks, q.C), dim3(GT), 0, st_, s, out);
   return check_launch("sgmc_mlp_full_potential");
 }
 
@@ -1113,7 +1176,7 @@ int sgmc_mlp_mh(const sgmc_mlp_state* st, void* stream) {
   s.mom = q.mom;
   s.ke = q.ke;
   MH m{q.U_full, q.U_prop, q.theta_old, q.mom_old, q.U_old, q.mh_key, q.mh_stats, q.accepted};
-  const int64_t blocks = std::min<int64_t>((q.P + GT - 1) / GT, 1024);
+  const int64_t blocks = std::min<int64_t>((q.P + 16 * GT - 1) / (16 * GT), 1024);
   hipLaunchKernelGGL(mh_kernel, dim3((unsigned)blocks, q.C), dim3(GT), 0, as_stream(stream), s,
                      m);
   return check_launch("sgmc_mlp_mh");

@@ -112,6 +112,7 @@ struct Step {
   float* mom;              // [C][P] momentum
   float* ke_part;          // [C][nparts] kinetic-energy partials of one evaluation
   float* col_part;         // [C][n / kStrip][small leaves] row-strip gradient partials
+  double* facc;            // [C] float64 likelihood of the full pass's chunks before this one
   double* fin_part;        // [C][kFinalBlocks] log-prior partials of the full pass
   double* ke;              // [C][2] accumulated kinetic energy at start / end
   float* U_half;           // [C] potential of the step's first evaluation
