@@ -298,10 +298,14 @@ __global__ void __launch_bounds__(kFcThreads) glm_full_chains_kernel(FcArgs a) {
 // through the wavefront's own 8 KiB of LDS, chunks swizzled by row against bank conflicts;
 // the loads of the next AHEAD steps are in flight while a tile is multiplied, across the
 // barrier too. (Loading operand order straight from memory touches every cache line with
-// four instructions of 32 lines each and stopped at 4.5 TB/s.) With S > 1 the wavefronts'
-// partial z go through the same LDS (double buffered, one barrier per step): wavefront w adds
-// the S partials of accumulator quads w, w + S, ... in order and applies the likelihood to
-// them. With Theta's operands in LDS instead (128 KiB, one block per unit, each
+// four instructions of 32 lines each and stopped at 4.5 TB/s.) With S > 1 a tile
+// passes from wavefront to wavefront: in turn i wavefront w multiplies its columns of tile
+// i - w onto the accumulators that wavefront w - 1 left in the same LDS (double buffered, one
+// barrier per step), so a row's products are added in column order on one accumulator; the
+// S wavefronts then share the likelihoods of the tile that the last one has finished.
+// (Partial sums of all S wavefronts on one tile, added at the end, save the S - 1 turns of
+// filling but round differently: 2e-9 of a potential of 7000 rows.)
+// With Theta's operands in LDS instead (128 KiB, one block per unit, each
 // wavefront its own rows in operand order): N = 1e6, D = 512, 64 chains 521 -> 432 us, 20
 // chains 507 -> 347 (5.9 TB/s of X); N = 400000, D = 1000, 64 chains 1375 -> 615; N = 300007,
 // D = 90, 20 chains 107 -> 36; N = 5000 69 -> 14. At 64 chains the partials' LDS traffic and
@@ -429,7 +433,9 @@ glm_full_chains_split_kernel(FcArgs a) {
   };
   auto load = [&](int step, auto hh, v4f (&buf)[8]) __attribute__((always_inline)) {
     constexpr int H = decltype(hh)::value;
-    const int64_t row0 = (t0 + (int64_t)(step / kSteps) * kGroups + grp) * kTile;
+    const int turn = step / kSteps - wp;  // (outside the block's turns: no rows)
+    const int64_t row0 = turn < 0 || turn >= turns
+                             ? a.N : (t0 + (int64_t)turn * kGroups + grp) * kTile;
     const auto rs = resource(a.X + min(row0, a.N) * a.ldx, (a.N - row0) * a.ldx);
 #pragma unroll
     for (int i = 0; i < 8; ++i)
@@ -455,7 +461,8 @@ glm_full_chains_split_kernel(FcArgs a) {
   // those of step + AHEAD
   auto step_of = [&](int step, auto hh, v4f (&cur)[8]) __attribute__((always_inline)) {
     constexpr int H = decltype(hh)::value;
-    const int turn = step / kSteps;
+    // the tile that the last of the S wavefronts finishes in this turn
+    const int turn = step / kSteps - (S - 1);
     const int64_t tile = t0 + (int64_t)turn * kGroups + grp;
     v4f* mine = part[step & (kSlots - 1)][w];
     if (ragged) {
@@ -476,14 +483,24 @@ glm_full_chains_split_kernel(FcArgs a) {
     load(step + AHEAD, std::integral_constant<int, (H + AHEAD) % kSteps>{}, cur);
     __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of the products
     if (H == 0) {
-      const int64_t row0 = tile * kTile;
+      const int64_t row0 = turn < 0 ? a.N : tile * kTile;
       const auto ys = resource(a.y + min(row0, a.N), a.N - row0);
 #pragma unroll
       for (int i = 0; i < kQuads; ++i)
         yv[i] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(
                                             ys, 32 * ((wp + i * S) % 4) + 16 * q, 0, 0));
+      if (S == 1 || wp == 0) {
 #pragma unroll
-      for (int t = 0; t < NT; ++t) acc[t] = v16f{};
+        for (int t = 0; t < NT; ++t) acc[t] = v16f{};
+      } else {  // go on from the wavefront before, which had this tile in the turn before
+        const v4f* prev = part[(step - 1) & (kSlots - 1)][w - 1];
+#pragma unroll
+        for (int qd = 0; qd < 4 * NT; ++qd) {
+          const v4f v = prev[qd * kWave + lane];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[qd / 4][4 * (qd % 4) + i] = v[i];
+        }
+      }
     }
 #pragma unroll
     for (int u = 0; u < KL; ++u) {
@@ -519,13 +536,12 @@ glm_full_chains_split_kernel(FcArgs a) {
         mine[qd * kWave + lane] = v4f{acc[qd / 4][4 * (qd % 4)], acc[qd / 4][4 * (qd % 4) + 1],
                                       acc[qd / 4][4 * (qd % 4) + 2], acc[qd / 4][4 * (qd % 4) + 3]};
       lds_sync();  // what this slot is used for next lies behind the next step's barrier
+      if (turn < 0) return;
 #pragma unroll
       for (int i = 0; i < kQuads; ++i) {
         const int qd = wp + i * S;
         if (qd >= 4 * NT) break;
-        v4f s = buf[grp * S][qd * kWave + lane];
-#pragma unroll
-        for (int v = 1; v < S; ++v) s += buf[grp * S + v][qd * kWave + lane];
+        const v4f s = buf[grp * S + S - 1][qd * kWave + lane];
         const float z[4] = {s.x, s.y, s.z, s.w};
         // (the chain tile of quad wp + i S; uniform, a register index needs it static)
 #pragma unroll
@@ -538,7 +554,7 @@ glm_full_chains_split_kernel(FcArgs a) {
   load(0, std::integral_constant<int, 0>{}, x[0]);
   load(1, std::integral_constant<int, 1 % kSteps>{}, x[1]);
   // AHEAD kSteps steps per round, so that buffers and places in the tile are static
-  const int steps = turns * kSteps;
+  const int steps = (turns + S - 1) * kSteps;
   auto round = [&](int base, auto self, auto bb) __attribute__((always_inline)) {
     constexpr int B = decltype(bb)::value;
     if (base + B < steps)
