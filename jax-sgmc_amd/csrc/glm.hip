@@ -196,7 +196,8 @@ struct FullArgs {
 // evaluation of the likelihood, row u on lane u of its segment. Bound by the read of X:
 // N = 1e6, D = 512 in 488 blocks 342 us (6.0 TB/s), D = 100 72 us. (One row at a time with the
 // likelihood on every lane spent about 210 us of vector issue per SIMD, not overlapped with
-// its loads: 466 and 273 us in 977 blocks.)
+// its loads: 466 and 273 us in 977 blocks.) The row products are separate multiplies and
+// adds: fused ones round differently, 2e-9 of a float64 potential of 11000 rows.
 template <int LPR, int CPL>
 __global__ void __launch_bounds__(kNT) glm_full_kernel(FullArgs a) {
   __shared__ double lds_d[kWaves];
@@ -231,7 +232,7 @@ __global__ void __launch_bounds__(kNT) glm_full_kernel(FullArgs a) {
         // (a whole wavefront's rows read past their end as zero; shorter segments reload
         // their last chunk there)
         if (RPW > 1 && q + LPR * k >= a.D4) x = f4{0.f, 0.f, 0.f, 0.f};
-        t = dot4_fma(x, th[k], t);
+        t += dot4(x, th[k]);
       }
       t = seg_sum<LPR>(t);
       zq = q == u ? t : zq;
