@@ -164,13 +164,6 @@ __global__ void __launch_bounds__(ROWS* kWave) gather_kernel(Step s) {
     for (int c = c0; c < c1; ++c) s.lab[(int64_t)c * s.n + j] = valid ? s.labels[r] : -1;
 }
 
-// Reads an activation of tensor t (e4m3 tensors in fp8 mode, bf16 otherwise).
-__device__ __forceinline__ float get_act(const Step& s, int c, int t, const void* p, int64_t i) {
-  if (s.fp32) return reinterpret_cast<const float*>(p)[i];
-  if (s.fp8) return q2f(reinterpret_cast<const uint8_t*>(p)[i]) / s.q[(int64_t)c * kQWords + t];
-  return bf2f(reinterpret_cast<const uint16_t*>(p)[i]);
-}
-
 // ------------------------------------------------------------------ head ------
 // logits = h2 W3 + b3; p = softmax; lik = logits[label] - lse; dL = c (onehot - p);
 // dA2 = (dL W3^T) * (h2 > 0). A wavefront takes R rows of one chain. W3S: W3 is staged in

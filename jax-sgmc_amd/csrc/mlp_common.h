@@ -186,7 +186,6 @@ struct Gemm {
   int64_t ldm, sM;
   int leaf;          // EPI_UPDATE / EPI_GRAD: parameter leaf of the [M][N] weight
   int part0;         // first prior-partial slot of this GEMM
-  int C;
   int ta, tb;        // P_FP8: scale slots of A and B
   int tout;          // P_FP8: scale slot of an e4m3 output, or -1 for a bf16 output
 };

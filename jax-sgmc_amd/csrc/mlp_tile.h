@@ -68,7 +68,9 @@ struct Stage {
     for (int h = 0; h < NR; ++h) {
       const int rr = row + h * RPP;
       const int s = KC ? swz_k(rr) : swz_n<PREC, R>(rr);
-      *reinterpret_cast<u32x4*>(lds + rr * (CPR * 16) + ((ch ^ s) << 4)) = r[h];
+      u32x4 v = r[h];
+      if (KC && PREC == P_FP8 && (rr & 16)) v = u32x4{v.z, v.w, v.x, v.y};  // see frag_k
+      *reinterpret_cast<u32x4*>(lds + rr * (CPR * 16) + ((ch ^ s) << 4)) = v;
     }
   }
 };
@@ -87,15 +89,18 @@ struct FragOf<P_F32> {
 };
 
 // Matrix fragment of rows r0 + lane % 32 of a k-contiguous tile, k-values kk + 8 (lane / 32)
-// ... (float32: kk + 4 (lane / 32) ...).
+// ... (float32: kk + 4 (lane / 32) ...). e4m3 takes half a chunk per lane: rows with bit 4 set
+// hold a chunk's halves swapped, so the 32 rows that one half-wavefront reads use both (in one
+// half of the chunks they met two by two on the banks, 20% of the LDS cycles).
 template <int PREC>
 __device__ __forceinline__ typename FragOf<PREC>::T frag_k(const uint8_t* lds, int r0, int kk,
                                                            int lane) {
   constexpr int EB = elem_bytes<PREC>();
   const int r = r0 + (lane & 31);
   const int kb = (kk + (k_span<PREC>() / 2) * (lane >> 5)) * EB;
+  const int half = PREC == P_FP8 ? (kb & 15) ^ ((r & 16) >> 1) : kb & 15;
   return *reinterpret_cast<const typename FragOf<PREC>::T*>(
-      lds + r * kStage + (((kb >> 4) ^ swz_k(r)) << 4) + (kb & 15));
+      lds + r * kStage + (((kb >> 4) ^ swz_k(r)) << 4) + half);
 }
 
 // The same fragment of columns n0 + lane % 32 of an n-contiguous tile. A transposing read

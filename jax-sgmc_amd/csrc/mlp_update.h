@@ -84,17 +84,16 @@ constexpr int UM_RMS = 1;
 constexpr int UM_OBA = 2;
 constexpr int UM_OBO = 3;
 
-// the rule's mode, and whether it carries state in aux / writes theta
+// the rule's mode
 template <int UM>
 __device__ __forceinline__ int um_mode(const Upd& u) {
   return UM == UM_RMS ? MLP_SGLD : UM == UM_OBA ? MLP_OBABO_BA : UM == UM_OBO ? MLP_OBABO_BO
                                                                                : u.mode;
 }
 
-template <int UM = UM_ANY>
 __device__ __forceinline__ void upd_load(const Upd& u, uint32_t i, float& w, float& aux) {
   w = u.th[i];
-  aux = (UM != UM_ANY || u.aux) ? u.aux[i] : 0.0f;
+  aux = u.aux ? u.aux[i] : 0.0f;
 }
 
 template <int UM = UM_ANY>
@@ -132,23 +131,18 @@ __device__ __forceinline__ void upd_step(const Upd& u, float& w, float& aux, flo
   }
 }
 
-// SH: the GEMM copy written -- SH_NONE, SH_BF16, SH_E4M3 (known from the operand
-// precision in the parameter-update GEMMs), or SH_ANY: whichever pointer is set.
-constexpr int SH_ANY = -1, SH_NONE = 0, SH_BF16 = 1, SH_E4M3 = 2;
-
-template <int UM = UM_ANY, int SH = SH_ANY>
 __device__ __forceinline__ void upd_store(const Upd& u, uint32_t i, float w, float aux,
                                           float& wmax) {
-  if (um_mode<UM>(u) != MLP_OBABO_BO) {
+  if (u.mode != MLP_OBABO_BO) {
     u.th[i] = w;
-    if (SH == SH_E4M3 || (SH == SH_ANY && u.sh8)) {
+    if (u.sh8) {
       u.sh8[i] = f2q(w * u.q8);
       wmax = fmaxf(wmax, fabsf(w));
-    } else if (SH == SH_BF16 || (SH == SH_ANY && u.sh)) {
+    } else if (u.sh) {
       u.sh[i] = f2bf(w);
     }
   }
-  if (UM != UM_ANY || u.aux) u.aux[i] = aux;
+  if (u.aux) u.aux[i] = aux;
 }
 
 // Key of leaf `leaf` of the noise tree of this update: random_tree(sub) with
