@@ -26,7 +26,8 @@
 // stored in float32, weights read from theta itself, no shadow); fp32 accumulation in
 // all three.
 //
-// The GEMMs: mlp_fwd.hip (G1-G3) and mlp_param.hip (G4, G5 with the update).
+// The GEMMs: mlp_fwd.hip (G1-G3) and mlp_param.hip (G4, G5 with the update, beside the small
+// leaves' column sums of mlp_colsum.h).
 #include <math.h>
 
 #include <type_traits>
@@ -346,82 +347,6 @@ __global__ void __launch_bounds__(kWave* NW) head_kernel(Step s) {
     }
   }
   if (PREC == P_FP8) q_note_amax_block(s, c, Q_DA2, amax, red);
-}
-
-// ------------------------------------------------------- small-leaf sums -----
-// Element i of an activation tensor stored at precision PREC (e4m3 at scale qs).
-template <int PREC>
-__device__ __forceinline__ float act_of(const void* p, int64_t i, float qs) {
-  if constexpr (PREC == P_F32) return reinterpret_cast<const float*>(p)[i];
-  else if constexpr (PREC == P_FP8) return q2f(reinterpret_cast<const uint8_t*>(p)[i]) / qs;
-  else return bf2f(reinterpret_cast<const uint16_t*>(p)[i]);
-}
-
-// Row-strip partial sums of the small leaves' gradients (flat order W3 [H2][10], b1,
-// b2, b3): for strip t, part[t][.] = sum over its kStrip rows of h2^T dL, dA1, dA2, dL.
-// Grid x: ceil(H2 / GT) blocks for W3 and b2, ceil(H1 / GT) for b1, one for b3.
-// PREC: the evaluation's GEMM precision (h2 is bf16 in e4m3 mode). A thread loads its
-// column's kStrip rows before summing them (in ascending row order), one memory round
-// trip per strip; the strip's dL rows are staged in LDS.
-template <int PREC>
-__global__ void __launch_bounds__(GT) colsum_kernel(Step s) {
-  constexpr int H2P = PREC == P_F32 ? P_F32 : P_BF16;
-  __shared__ float dls[kStrip * NCLS];
-  const int c = blockIdx.z, t = blockIdx.y;
-  const int nb2 = (s.H2 + GT - 1) / GT, nb1 = (s.H1 + GT - 1) / GT;
-  const int64_t nW3 = (int64_t)s.H2 * NCLS;
-  const int64_t total = nW3 + s.H1 + s.H2 + NCLS;
-  float* out = s.col_part + ((int64_t)c * (s.n / kStrip) + t) * total;
-  const int64_t r0 = (int64_t)c * s.n + (int64_t)t * kStrip;
-  const float* dL = s.dL + r0 * NCLS;
-  const int bx = blockIdx.x;
-  if (bx < nb2) {
-    for (int q = threadIdx.x; q < kStrip * NCLS; q += GT) dls[q] = dL[q];
-    __syncthreads();
-    const int a = bx * GT + threadIdx.x;
-    if (a >= s.H2) return;
-    const float qs = PREC == P_FP8 ? s.q[(int64_t)c * kQWords + Q_DA2] : 1.0f;
-    float h[kStrip], d2[kStrip];
-#pragma unroll
-    for (int r = 0; r < kStrip; ++r) {
-      h[r] = act_of<H2P>(s.h2, (r0 + r) * s.H2 + a, 1.0f);
-      d2[r] = act_of<PREC>(s.da2, (r0 + r) * s.H2 + a, qs);
-    }
-    float w3[NCLS];
-#pragma unroll
-    for (int k = 0; k < NCLS; ++k) w3[k] = 0.f;
-    float b2 = 0.f;
-#pragma unroll
-    for (int r = 0; r < kStrip; ++r) {
-      b2 += d2[r];
-#pragma unroll
-      for (int k = 0; k < NCLS; ++k) w3[k] += h[r] * dls[r * NCLS + k];
-    }
-#pragma unroll
-    for (int k = 0; k < NCLS; ++k) out[(int64_t)a * NCLS + k] = w3[k];
-    out[nW3 + s.H1 + a] = b2;
-  } else if (bx < nb2 + nb1) {
-    const int i = (bx - nb2) * GT + threadIdx.x;
-    if (i >= s.H1) return;
-    const float qs = PREC == P_FP8 ? s.q[(int64_t)c * kQWords + Q_DA1] : 1.0f;
-    float d1[kStrip];
-#pragma unroll
-    for (int r = 0; r < kStrip; ++r) d1[r] = act_of<PREC>(s.da1, (r0 + r) * s.H1 + i, qs);
-    float b1 = 0.f;
-#pragma unroll
-    for (int r = 0; r < kStrip; ++r) b1 += d1[r];
-    out[nW3 + i] = b1;
-  } else {
-    const int k = threadIdx.x;
-    if (k >= NCLS) return;
-    float dk[kStrip];
-#pragma unroll
-    for (int r = 0; r < kStrip; ++r) dk[r] = dL[r * NCLS + k];
-    float b3 = 0.f;
-#pragma unroll
-    for (int r = 0; r < kStrip; ++r) b3 += dk[r];
-    out[nW3 + s.H1 + s.H2 + k] = b3;
-  }
 }
 
 // ----------------------------------------------------------- small params -----
@@ -1111,11 +1036,7 @@ int sgmc_mlp_step(const sgmc_mlp_state* st, int update, void* stream) {
           nullptr, 0, 0, nullptr, 0, nullptr, 0, 0, 0, L.g4_blocks};
   g4 = with_q(g4, Q_H1, Q_DA2, -1);
   g5 = with_q(g5, Q_X, Q_DA1, -1);
-  launch_param_gemms(g4, g5, s, st_);
-  const dim3 col_grid((q.H2 + GT - 1) / GT + (q.H1 + GT - 1) / GT + 1, n / kStrip, C);
-  if (s.fp32) hipLaunchKernelGGL(colsum_kernel<P_F32>, col_grid, dim3(GT), 0, st_, s);
-  else if (s.fp8) hipLaunchKernelGGL(colsum_kernel<P_FP8>, col_grid, dim3(GT), 0, st_, s);
-  else hipLaunchKernelGGL(colsum_kernel<P_BF16>, col_grid, dim3(GT), 0, st_, s);
+  launch_param_gemms(g4, g5, s, st_);  // and the strips' column sums
   hipLaunchKernelGGL(small_kernel, dim3(L.small_blocks, C), dim3(GT), 0, st_, s,
                      L.g4_blocks + L.g5_blocks);
   if (update && s.mode == MLP_SGLD && q.samples && q.save_slot) {

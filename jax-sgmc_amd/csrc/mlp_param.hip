@@ -14,6 +14,7 @@
 // that step's update 163 -> 121 us (694 MB of traffic with the operands, 5.7 TB/s); 16
 // chains of 3072-1024-1024 in e4m3, n = 512: OBA half 378 -> 279 us, BO half 252 -> 204 us,
 // gradient 210 -> 161 us; float32 gradient of 4 chains of 3072-512-512 55 -> 47 us.
+#include "mlp_colsum.h"
 #include "mlp_tile.h"
 #include "mlp_update.h"
 
@@ -223,17 +224,27 @@ __device__ __forceinline__ void param_tile(const Gemm& g, const Step& s, uint32_
 // step) runs through it backwards, so that it begins with the state which the one before
 // wrote last and the last-level cache still holds (pSGLD 3072-512-512, 16 chains: iteration
 // 244 -> 237 us of kernels). The first blocks take gW1's tiles (ga) and the rest gW2's (gb), so
-// gW2's fill the last round of gW1's.
+// gW2's fill the last round of gW1's. Ahead of both come the ncol blocks of the small leaves'
+// column sums (colx per strip), which need the same activations and none of the parameters:
+// latency-bound on their own (20 us in e4m3, 8 in bf16, 6 in float32), here they run beside the
+// update (16 chains of 3072-512-512 bf16 121 + 8 -> 125 us, 4 chains in float32 47 + 6 -> 47).
 template <int PREC, int BW, int EPI, int UM>
 __global__ void __launch_bounds__(GT, kWavesPerSimd)
-    param_kernel(Gemm ga, Gemm gb, Step s, uint32_t gxa, uint32_t gya, uint32_t gxb,
-                 uint32_t gyb) {
+    param_kernel(Gemm ga, Gemm gb, Step s, uint32_t gxa, uint32_t gya, uint32_t gxb, uint32_t gyb,
+                 uint32_t ncol, uint32_t colx) {
   constexpr int kProd = 2 * 4096 * 4, kStages = (2 * BW + 4096 / BW) * kStage;
   __shared__ __attribute__((aligned(16))) uint8_t lds[kProd > kStages ? kProd : kStages];
   __shared__ float red[GT / kWave];
+  if (blockIdx.x < ncol) {
+    const uint32_t strips = (uint32_t)(s.n / kStrip), b = blockIdx.x;
+    if (b < colx * strips * (uint32_t)s.C)
+      colsum_block<PREC>(s, (int)(b % colx), (int)(b / colx % strips), (int)(b / (colx * strips)),
+                         reinterpret_cast<float*>(lds));
+    return;
+  }
   const uint32_t na = gxa * gya * (uint32_t)s.C;
   const bool rev = s.mode == MLP_SGLD ? (cur_iter(s) & 1) != 0 : s.mode == MLP_OBABO_BO;
-  const uint32_t lin = rev ? gridDim.x - 1 - blockIdx.x : blockIdx.x;
+  const uint32_t lin = rev ? gridDim.x - 1 - blockIdx.x : blockIdx.x - ncol;
   if (lin < na)
     param_tile<PREC, BW, EPI, UM>(ga, s, lin, gxa, gya, lds, red);
   else
@@ -245,9 +256,12 @@ void launch(const Gemm& ga, const Gemm& gb, const Step& s, hipStream_t st) {
   constexpr int W = 2 * BW, TN = 4096 / BW;
   const uint32_t gxa = (uint32_t)(ga.M / W), gya = (uint32_t)(ga.N / TN);
   const uint32_t gxb = (uint32_t)(gb.M / W), gyb = (uint32_t)(gb.N / TN);
+  // the column sums' blocks first, padded to whole rounds over the XCDs
+  const uint32_t colx = (uint32_t)colsum_blocks(s);
+  const uint32_t ncol = (colx * (uint32_t)(s.n / kStrip) * (uint32_t)s.C + kXcds - 1) / kXcds * kXcds;
   hipLaunchKernelGGL((param_kernel<PREC, BW, EPI, UM>),
-                     dim3((gxa * gya + gxb * gyb) * (uint32_t)s.C), dim3(GT), 0, st, ga, gb, s,
-                     gxa, gya, gxb, gyb);
+                     dim3(ncol + (gxa * gya + gxb * gyb) * (uint32_t)s.C), dim3(GT), 0, st, ga, gb,
+                     s, gxa, gya, gxb, gyb, ncol, colx);
 }
 
 // the update rule compiled in: rms_prop SGLD and the two OBABO halves; plain SGLD at run time
