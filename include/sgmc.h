@@ -154,7 +154,8 @@ int sgmc_glm_full_potential_chains(int family, const float* X, int64_t ldx, cons
  * 6e-8) for a fifth of the matrix time; sums stay FP64. X is scaled by 2^x_exp, chosen
  * once for the dataset so that max |X| 2^x_exp < 2^14 (for example 14 - the frexp
  * exponent of max |X|; -64 <= x_exp <= 64); each chain's position is scaled by its own
- * power of two from its largest finite entry. */
+ * power of two from its largest finite entry. Row strides beyond 31-bit offsets within a
+ * tile of 32 rows (124 ldx + 16 ceil(D/4) > 2^31 - 1 bytes) take the float32 products. */
 int sgmc_glm_full_potential_chains_split(int family, const float* X, int64_t ldx,
                                          const float* y, int64_t N, int D, const float* thetas,
                                          int64_t ld_theta, int nchains, float sigma,

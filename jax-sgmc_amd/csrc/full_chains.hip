@@ -631,6 +631,11 @@ int launch_full_chains(const char* name, bool split, int x_exp, int family, cons
   SGMC_REQUIRE(temperature != 0.0, SGMC_E_ARG, "%s: temperature is zero", name);
   SGMC_REQUIRE(x_exp >= -64 && x_exp <= 64, SGMC_E_ARG, "%s: x_exp=%d outside [-64, 64]", name,
                x_exp);
+  // The split kernel reaches the rows of a tile by 31-bit byte offsets from its first row:
+  // 31 rows on and a row's columns further. Longer strides (over about 17.3 M floats: a column
+  // slice of a very wide matrix) take the float32 kernel, which addresses every row in 64 bits.
+  const bool far = (kTile - 1) * 4 * ldx + 16 * (int64_t)((D + 3) / 4) > 0x7FFFFFFF;
+  split = split && !far;
   FcArgs a;
   a.X = X;
   a.y = y;
