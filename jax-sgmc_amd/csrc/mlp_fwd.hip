@@ -56,10 +56,12 @@ __global__ void __launch_bounds__(kWave* WM* WN* G) fwd_kernel(Gemm g, Step s, u
 
   const int kspan = g.K / G, kfirst = grp * kspan;
   const uint32_t lda = (uint32_t)(g.lda * EB), ldb = (uint32_t)(g.ldb * EB);
+  typedef Stage<PREC, TM, NT, true> StageA;
+  typedef Stage<PREC, TN, NT, B_K> StageB;
   const uint8_t* A = reinterpret_cast<const uint8_t*>(g.A) + (int64_t)c * g.sA * EB +
-                     (int64_t)(bm * TM) * lda + (int64_t)kfirst * EB;
+                     (int64_t)(bm * TM + StageA::first(t)) * lda + (int64_t)kfirst * EB;
   const uint8_t* B = reinterpret_cast<const uint8_t*>(g.B) + (int64_t)c * g.sB * EB +
-                     (B_K ? (int64_t)(bn * TN) * ldb + (int64_t)kfirst * EB
+                     (B_K ? (int64_t)(bn * TN + StageB::first(t)) * ldb + (int64_t)kfirst * EB
                           : (int64_t)kfirst * ldb + (int64_t)(bn * TN) * EB);
   const int stages = (kspan + KE - 1) / KE;
   const int64_t stepB = B_K ? (int64_t)kStage : (int64_t)KE * ldb;
@@ -72,8 +74,8 @@ __global__ void __launch_bounds__(kWave* WM* WN* G) fwd_kernel(Gemm g, Step s, u
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
 
-  Stage<PREC, TM, NT, true> pa, qa;
-  Stage<PREC, TN, NT, B_K> pb, qb;
+  StageA pa, qa;
+  StageB pb, qb;
   auto load = [&](auto& a, auto& b, int st) __attribute__((always_inline)) {
     a.load(A + (int64_t)st * kStage, lda, kspan - st * KE, t);
     b.load(B + st * stepB, ldb, kspan - st * KE, t);

@@ -27,8 +27,10 @@ namespace {
 constexpr int kWavesPerSimd = 3;
 constexpr int kRawBufferFlags = 0x00020000;  // word 3 of a raw buffer resource (CDNA)
 
+// 2^32 - 16 bytes from p: the 32 rows of a band span less at the widest layer (a leaf has fewer
+// than 2^32 entries and at least 128 rows or columns: rows of up to 2^25 floats).
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* p, bool on = true) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, on ? 0x7FFFFFFF : 0,
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, on ? (int)0xFFFFFFF0u : 0,
                                            kRawBufferFlags);
 }
 // State is stored with the non-temporal hint, which leaves the last-level cache to what the

@@ -44,14 +44,24 @@ struct Stage {
   static_assert(NT % CPR == 0 && (R * (kStage / 16)) % NT == 0, "whole chunks per thread");
   u32x4 r[NR];
 
-  // src: first row / column of the tile at k = k0; left: k-values left in the range; gap:
-  // bytes between the two halves of a row's columns that lie apart (n-contiguous tiles)
+  // First row of this wavefront in a pass over a k-contiguous tile. Its resources begin there,
+  // with a base of 64 bits, so that lane offsets span eight rows and stay below 2^31 at every
+  // accepted width (over all rows of a pass they went past it at inputs of 17 M float32
+  // columns). A pass over an n-contiguous tile spans 16 NT / R <= 64 bytes per column of the
+  // operand, below 2^31 for fewer than 2^25 columns, and begins at row 0.
+  static __device__ __forceinline__ int first(int t) {
+    return KC ? __builtin_amdgcn_readfirstlane(t / kWave) * (kWave / CPR) : 0;
+  }
+
+  // src: row first(t) (n-contiguous: first column) of the tile at k = k0; left: k-values left
+  // in the range; gap: bytes between the two halves of a row's columns that lie apart
+  // (n-contiguous tiles)
   __device__ __forceinline__ void load(const uint8_t* src, uint32_t ldb, int left, int t,
                                        uint32_t gap = 0) {
-    const uint32_t row = (uint32_t)t / CPR, ch = (uint32_t)t % CPR;
+    const uint32_t row = (uint32_t)(KC ? t % kWave : t) / CPR, ch = (uint32_t)t % CPR;
     uint32_t vo = row * ldb + ch * 16 + (ch >= CPR / 2 ? gap : 0);
     if (KC && (int)ch * (16 / EB) >= left) vo = 0x80000000u;
-    // a resource per pass: its base moves in 64 bits, lane offsets stay below 2^31
+    // a resource per pass: its base moves in 64 bits
 #pragma unroll
     for (int h = 0; h < NR; ++h) {
       const int rest = KC ? 0x7FFFFFFF : min(max(left - h * RPP, 0), RPP) * (int)ldb;
