@@ -487,9 +487,12 @@ int64_t sgmc_glm_workspace_floats(int n, int D, int nblocks) {
 // One block per compute unit (two at 256 < D <= 512), each with at least one row group of its
 // four wavefronts. n = 40001, D = 301: 19.3 us at 507 blocks, 20.8 at 256; n = 60000,
 // D = 1000: 49.2 and 45.9; n = 20000, D = 100: 13.8 and 12.7; n = 60000, D = 64: 14.2 and
-// 13.2. (256 rows per block, whatever the size: 87.5, 270.7, 38.2 and 63.3 us.)
+// 13.2. (256 rows per block, whatever the size: 87.5, 270.7, 38.2 and 63.3 us.) Never more
+// records than the scratch of sgmc_glm_potential_noalloc holds (509 blocks at D = 512, 255 at
+// D = 1024) unless the rows of a block need them.
 int sgmc_glm_blocks(int n, int D) {
-  const int blocks = D > 256 && D <= 512 ? 512 : 256;
+  const int held = (int)(kScratchRecordFloats / (4 * ((D + 3) / 4) + 2));
+  const int blocks = std::min(D > 256 && D <= 512 ? 512 : 256, held);
   const int least = D <= 16 ? 256 : D <= 32 ? 128 : D <= 64 ? 64 : 32;
   const int rows = std::max(least, (int)(((int64_t)n + blocks - 1) / blocks));
   const int b = (int)(((int64_t)n + rows - 1) / rows);
