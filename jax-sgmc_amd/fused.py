@@ -659,13 +659,14 @@ class TableGroup:
     return self.engines[t], i - int(self.offsets[t])
 
   def _ordered_by_null(self):
-    """Whether the current stream is the legacy default (null) stream: the pool's streams
-    are blocking streams (created without hipStreamNonBlocking), which start behind all
-    earlier null-stream work and which all later null-stream work waits for, so a fork
-    and a join need no events. Each event operation on the null stream waits for every
+    """Whether the current stream is the legacy default (null) stream of the tables' device
+    (another device's orders nothing there): the pool's streams are blocking streams
+    (created without hipStreamNonBlocking), which start behind all earlier null-stream work
+    and which all later null-stream work waits for, so a fork and a join need no events. Each event operation on the null stream waits for every
     blocking stream, so two tables' fork and join by events cost 100 us (ten iterations
     of two small tables 246 us with them, 112 without)."""
-    return torch.cuda.current_stream().cuda_stream == 0
+    cur = torch.cuda.current_stream()
+    return cur.cuda_stream == 0 and cur.device == self.streams[0].device
 
   def _fork(self):
     if self._ordered_by_null():
@@ -691,7 +692,8 @@ class TableGroup:
 
   def _run_plans(self, plan_of):
     self._fork()
-    _execute_tables([(e, s, plan_of(e)) for e, s in zip(self.engines, self._table_streams())])
+    with torch.cuda.device(self.streams[0].device):  # whatever the caller's is
+      _execute_tables([(e, s, plan_of(e)) for e, s in zip(self.engines, self._table_streams())])
     self._join()
 
   def iteration(self):
