@@ -270,6 +270,10 @@ __device__ __forceinline__ void process_group(RowGroup<LPR, CPL>& g, int row0, i
 // the row ids of the next 64-row chunk are drawn before the current chunk is done. mid()
 // runs (on every wavefront, also one without rows) when the first loads are in flight: it
 // sets th, and whatever else does not depend on the rows is hidden behind them.
+// The float32 sums are kept in two levels, chunks of 64 rows and their sum: a wavefront of a
+// long block adds hundreds of rows per lane (256 at 64 chains of n = 4096), and one running
+// sum over them rounds more than the many short blocks of a finer split did (SGHMC of 64
+// chains against 64 bits: @ERR@).
 template <int LPR, int CPL, class Mid>
 __device__ __forceinline__ void accumulate_rows(gcfloat* __restrict__ X, int64_t ldx,
                                                 gcfloat* __restrict__ y, int D4,
@@ -287,6 +291,20 @@ __device__ __forceinline__ void accumulate_rows(gcfloat* __restrict__ X, int64_t
   int cb = r0;
   int rid = chunk_rows(src, cb, r1);
   RowGroup<LPR, CPL> ga, gb;
+  float4 tot[CPL];
+  float lik_tot = 0.0f;
+#pragma unroll
+  for (int k = 0; k < CPL; ++k) tot[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+  auto fold = [&] {
+#pragma unroll
+    for (int k = 0; k < CPL; ++k) {
+      tot[k] = make_float4(tot[k].x + acc[k].x, tot[k].y + acc[k].y, tot[k].z + acc[k].z,
+                           tot[k].w + acc[k].w);
+      acc[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    lik_tot += lik_acc;
+    lik_acc = 0.0f;
+  };
   load_group<LPR, CPL>(X, ldx, y, D4, 0, rid, ga);
   int rid_n = cb + kWave < r1 ? chunk_rows(src, cb + kWave, r1) : -1;
   mid();
@@ -302,6 +320,7 @@ __device__ __forceinline__ void accumulate_rows(gcfloat* __restrict__ X, int64_t
     process_group<LPR, CPL>(ga, cb + gl, D4, th, L, acc, lik_acc, lds_lik, lds_row0);
     if (!more) break;
     if (next) {
+      fold();
       cb += kWave;
       nl = 0;
       rid = rid_n;
@@ -315,12 +334,19 @@ __device__ __forceinline__ void accumulate_rows(gcfloat* __restrict__ X, int64_t
     process_group<LPR, CPL>(gb, cb + gl, D4, th, L, acc, lik_acc, lds_lik, lds_row0);
     if (!more) break;
     if (next) {
+      fold();
       cb += kWave;
       nl = 0;
       rid = rid_n;
       rid_n = cb + kWave < r1 ? chunk_rows(src, cb + kWave, r1) : -1;
     }
     gl = nl;
+  }
+  if (r1 - r0 > kWave) {
+    fold();
+#pragma unroll
+    for (int k = 0; k < CPL; ++k) acc[k] = tot[k];
+    lik_acc = lik_tot;
   }
 }
 
