@@ -394,8 +394,10 @@ int scratch_of_current_device(void* stream, float** out) {
 // ---- launches of one chain table ----
 bool known_mode(int mode) { return mode >= SGMC_MODE_SGLD && mode <= SGMC_MODE_SGGMC; }
 
-// Launches of one iteration: OBABO modes take two per leapfrog step.
+// Launches of one iteration: modes without leapfrog steps take one whatever `steps` says,
+// OBABO modes two per leapfrog step.
 int launches_of(const sgmc_glm_run& r) {
+  if (r.mode == SGMC_MODE_SGLD || r.mode == SGMC_MODE_SGLD_RMS) return 1;
   return (r.mode == SGMC_MODE_OBABO || r.mode == SGMC_MODE_SGGMC) ? 2 * r.steps : r.steps;
 }
 
@@ -686,8 +688,9 @@ int sgmc_glm_fused_step(const sgmc_glm_chain* chains, int nchains, const int32_t
   r.lmbd = lmbd;
   const int rc = check_run("sgmc_glm_fused_step", r);
   if (rc != SGMC_OK) return rc;
-  SGMC_REQUIRE(step >= 0 && step < launches_of(r), SGMC_E_ARG,
-               "sgmc_glm_fused_step: launch %d of %d", step, launches_of(r));
+  const int launches = std::max(steps, launches_of(r));  // SGLD: any of the caller's steps
+  SGMC_REQUIRE(step >= 0 && step < launches, SGMC_E_ARG,
+               "sgmc_glm_fused_step: launch %d of %d", step, launches);
   FusedArgs a = run_args(r);
   a.step = step;
   a.advance = advance_iter ? 1 : 0;
