@@ -478,8 +478,10 @@ glm_full_chains_split_kernel(FcArgs a) {
         }
       }
     }
+    wave_sync();  // the step before has read the slot
 #pragma unroll
     for (int i = 0; i < 8; ++i) mine[i * kWave + lane] = cur[i];
+    wave_sync();
     load(step + AHEAD, std::integral_constant<int, (H + AHEAD) % kSteps>{}, cur);
     __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of the products
     if (H == 0) {

@@ -283,7 +283,7 @@ __global__ void __launch_bounds__(kWave* NW) head_kernel(Step s) {
 #pragma unroll
     for (int j = 0; j < kZ4 / 4; ++j) zs[wv][4 * j + 2 * (g & 1) + (g >> 1)] = q[j];
   }
-  __builtin_amdgcn_wave_barrier();
+  wave_sync();
   // lane r: softmax of row r (a wavefront's LDS accesses complete in order)
   const float cscale = ((float)(-s.N) / (float)s.n) / s.temperature;
   if (lane < R) {
@@ -315,7 +315,7 @@ __global__ void __launch_bounds__(kWave* NW) head_kernel(Step s) {
     }
   }
   if (s.full) return;
-  __builtin_amdgcn_wave_barrier();
+  wave_sync();
   float dl[kZ];
 #pragma unroll
   for (int i = 0; i < kZ; ++i) dl[i] = zs[wv][i];

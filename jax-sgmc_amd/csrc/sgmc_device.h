@@ -417,6 +417,15 @@ __device__ __forceinline__ void lds_sync() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
+// Hands LDS data from lane to lane of one wavefront: the stores before it are visible to the
+// wavefront's loads after it. A wavefront's LDS accesses complete in order, so this costs no
+// instruction; the fences keep the compiler from moving accesses across.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // LDS_SYNC: barriers that leave global loads in flight (lds_sync) instead of
 // __syncthreads; for blocks that share only LDS between the two barriers.
 template <int NT, bool LDS_SYNC = false>
