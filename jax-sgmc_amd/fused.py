@@ -84,19 +84,46 @@ def default_blocks(n, D, loops, cus):
     blocks per unit where that still leaves a chain at most eight records: 64 chains of
     D = 100, n = 2048 take 25.8 us at 256 blocks and 20.1 at 512; 8 chains of D = 256,
     n = 2048 take 15.2 and 17.8 (64 records to sum per chain).
+  - Longer rows round the share down: a few blocks past one per unit take nearly two rounds
+    (55 chains of D = 1000, n = 4096: 184 us in 5 blocks each, 275 in all, 140 in 4; D = 512:
+    91 and 76).
+  - A share below four has no such even split nearby. It takes the first count up to eight
+    that fills its last round of blocks to 88%, with blocks short enough for the table: a row
+    costs a wavefront's latency of about 65 ns where a whole wavefront reads it (D > 128), so
+    rows may be as many as the table's bytes take that long to stream at 6.5 TB/s, and 1024
+    in any case. n = 4096, D = 300: 171 chains 258 us in one block each, 150 in four; 230
+    chains 259 and 187 in two; 300 chains 344 and 243 in four (64 KiB of rows or 1/2048 of
+    the table per block: 162, 210 and 263).
   """
   n, D = np.asarray(n, np.int64), np.asarray(D, np.int64)
   rows_bytes = n * 4 * ((D + 3) // 4 * 4)
-  share = cus * rows_bytes / max(1, int(rows_bytes.sum()))
-  share = np.where(D <= 256, np.maximum(share, np.minimum(8.0, 2.0 * share)), share)
+  total = max(1, int(rows_bytes.sum()))
   out = []
-  for nc, d, b, s in zip(n, D, rows_bytes, share):
-    least = -(-int(nc) // LDS_ROWS)
-    nb = min(int(round(float(s))), -(-int(nc) // _min_block_rows(int(d))))
+  for nc, d, b in zip(n.tolist(), D.tolist(), rows_bytes.tolist()):
+    least = -(-nc // LDS_ROWS)
+    per_unit = cus * b / total
+    share = max(per_unit, min(8.0, 2.0 * per_unit)) if d <= 256 else per_unit
+    if share < 4.0:
+      nb = _few_blocks(nc, d, per_unit, max(1, least, int(share)), total)
+    else:
+      nb = int(round(share)) if d <= 256 else int(share)
+    nb = min(nb, -(-nc // _min_block_rows(d)))
     if b < (96 if loops else 40) * 1024:
       nb = 1
     out.append(max(1, least, nb))
   return out
+
+
+def _few_blocks(n, D, per_unit, first, total):
+  """The split of a chain whose share of a block per unit is ``per_unit`` (default_blocks),
+  from ``first`` blocks on; ``total``: bytes of the table's minibatches."""
+  lanes = 4 if D <= 16 else 8 if D <= 32 else 16 if D <= 64 else 32 if D <= 128 else 64
+  rows = max(1024, total / (65e-9 * 6.5e12 * lanes / 64))
+  for nb in range(first, 9):
+    rounds = nb / per_unit
+    if rounds / math.ceil(rounds) >= 0.88 and n <= nb * rows:
+      return nb
+  return first
 
 
 class FusedGLM:
