@@ -66,8 +66,9 @@ def _min_block_rows(D):
 def default_blocks(n, D, loops, cus):
   """Grid blocks of every chain of a table when no bytes-per-block target is given.
 
-  n, D: minibatch sizes and row lengths of the chains; loops: whether the table's sampler
-  can run iterations in one launch (one block per chain); cus: compute units.
+  n, D: minibatch sizes and row lengths of the chains; loops: whether the table can run
+  iterations in one launch (one block per chain); cus: compute units. A table whose chains
+  do not all come out with one block runs no loop launches: see table_blocks.
 
   - A chain whose minibatch is under 96 KiB gets one block where iterations can run in a
     loop launch: D = 32, n = 512 takes 8.2 us per iteration there and 8.9 as launches of
@@ -112,6 +113,14 @@ def default_blocks(n, D, loops, cus):
       nb = 1
     out.append(max(1, least, nb))
   return out
+
+
+def table_blocks(n, D, loops, cus):
+  """default_blocks with the line of loop launches (96 KiB) only where the table will run
+  them: with ``loops`` and one block for each of its chains. One multi-block chain takes the
+  others to launches, whose line is 40 KiB."""
+  blocks = default_blocks(n, D, loops, cus)
+  return blocks if not loops or max(blocks) == 1 else default_blocks(n, D, False, cus)
 
 
 def _few_blocks(n, D, per_unit, first, total):
@@ -263,8 +272,8 @@ class FusedGLM:
 
   def _build_table(self):
     if self._blocks_by_rule:
-      nbs = default_blocks(self.n, self.D, self.mode in _LOOPS,
-                           torch.cuda.get_device_properties(self.device).multi_processor_count)
+      nbs = table_blocks(self.n, self.D, self._may_loop(),
+                         torch.cuda.get_device_properties(self.device).multi_processor_count)
     else:
       nbs = [blocks_for(int(n), int(d), self.target_bytes) for n, d in zip(self.n, self.D)]
     self.nblocks_chain = np.array(nbs)
@@ -347,9 +356,11 @@ class FusedGLM:
     """Chains of one block each, no Metropolis-Hastings test, and no exchange or one
     that runs only at its test iterations: many iterations can run in one launch
     (``sgmc_glm_fused_loop``), cut at the exchange's test iterations."""
-    return (bool(np.all(self.nblocks_chain == 1)) and self.mh is None and
-            (self.exchange is None or self.exchange.sparse) and
-            self.mode in _LOOPS)
+    return bool(np.all(self.nblocks_chain == 1)) and self._may_loop()
+
+  def _may_loop(self):
+    return (self.mode in _LOOPS and self.mh is None and
+            (self.exchange is None or self.exchange.sparse))
 
   def _launch_loop(self, iterations):
     _lib.call("sgmc_glm_fused_loop", _lib.ptr(self.table), self.C, self.uniform_dclass,
@@ -930,6 +941,8 @@ class ReplicaExchange:
     self.pairs = list(pairs)
     self.sparse = not any(save)
     engine.exchange = self
+    if not self.sparse and engine._blocks_by_rule:
+      engine._build_table()  # no loop launches any more: its chains may want more blocks
     engine._graph = None
 
   def needs_launch(self, done):

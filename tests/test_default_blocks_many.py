@@ -31,3 +31,12 @@ def test_measured_splits(D, C, n, least, most):
   """Counts of which the neighbours measured slower than the split before (blocks of 64 KiB or
   1/2048 of the table)."""
   assert least <= fused.default_blocks([n] * C, [D] * C, True, CUS)[0] <= most
+
+
+@pytest.mark.parametrize("n,D,loops,want", [
+    ([128], [100], True, [1]),                # 51 KiB alone: a loop launch
+    ([128], [100], False, [4]),               # the same without one
+    ([128, 4096], [100, 512], True, [3, 128]),  # beside a chain of several blocks
+    ([128, 128, 64], [100, 100, 30], True, [1, 1, 1])])
+def test_the_line_of_loop_launches_needs_them(n, D, loops, want):
+  assert fused.table_blocks(n, D, loops, CUS) == want

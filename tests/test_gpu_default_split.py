@@ -1,0 +1,45 @@
+"""The default split of chain tables (GPU): a saving exchange, which rules out loop launches,
+gives its chains the split of launches."""
+import numpy as np
+import pytest
+import torch
+
+from jax_sgmc_amd import fused
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _data(N, D):
+  g = torch.Generator(device=DEV).manual_seed(N + D)
+  X = torch.zeros((N, (D + 3) // 4 * 4), device=DEV)
+  X[:, :D] = torch.randn((N, D), generator=g, device=DEV) / D ** 0.5
+  return X, (torch.rand(N, generator=g, device=DEV) < 0.5).float()
+
+
+def _chain(X, y, D, n, c):
+  return dict(X=X, y=y, D=D, n=n, theta0=np.full(D, 0.01 * c, np.float32), key=(1, c),
+              dkey=(2, c))
+
+
+def test_saving_exchange_takes_the_split_of_launches():
+  print("default split under a saving exchange", flush=True)
+  X, y = _data(2000, 100)
+  kw = dict(save_slots=np.arange(6), n_slots=6)
+
+  def pair(save, target):
+    eng = fused.FusedGLM([_chain(X, y, 100, 128, c) for c in range(2)], "logistic", "sgld",
+                         np.full(6, 1e-4, np.float32), target_bytes=target, **kw)
+    ex = fused.ReplicaExchange(eng, [(0, 1)], [(1.0, 2.0)], keys=[(3, 4)], swap_every=2,
+                               save=[save])
+    return eng, ex
+  assert pair(False, None)[0].nblocks_chain.tolist() == [1, 1]  # loop launches between tests
+  eng, ex = pair(True, None)
+  assert eng.nblocks_chain.tolist() == [4, 4]
+  want, wex = pair(True, 128 * 400 / 4)
+  assert want.nblocks_chain.tolist() == [4, 4]
+  for e in (eng, want):
+    e.run(6)
+  torch.cuda.synchronize()
+  assert torch.equal(eng.theta_flat, want.theta_flat)
+  assert torch.equal(ex.sample_trace(0), wex.sample_trace(0))
