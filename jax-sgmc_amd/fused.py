@@ -204,8 +204,8 @@ class FusedGLM:
     dcl = {_lib.query("sgmc_glm_dclass", d) for d in Ds}
     self.uniform_dclass = dcl.pop() if len(dcl) == 1 else -1
     total_bytes = sum(int(c["n"]) * 4 * _align4(int(c["D"])) for c in chains)
-    self._target_bytes = target_bytes or max(64 * 1024, total_bytes // 2048)
-    self._blocks_by_rule = not target_bytes  # until a target is set
+    self._default_target = max(64 * 1024, total_bytes // 2048)
+    self.target_bytes = target_bytes or None
     self.keep_lik = bool(keep_lik)
     self.exchange = None
     self.mh = None
@@ -262,13 +262,13 @@ class FusedGLM:
   @property
   def target_bytes(self):
     """Bytes of rows per block; setting it replaces the default split at the next
-    _build_table."""
+    _build_table, setting None brings that back."""
     return self._target_bytes
 
   @target_bytes.setter
   def target_bytes(self, value):
-    self._target_bytes = value
-    self._blocks_by_rule = False
+    self._blocks_by_rule = value is None
+    self._target_bytes = self._default_target if value is None else value
 
   def _build_table(self):
     if self._blocks_by_rule:
@@ -513,32 +513,39 @@ class FusedGLM:
 
   # ------------------------------------------------------------ autotuner ----
   def autotune(self, candidates=None, reps=3):
-    """Picks the bytes-per-block target with the shortest launch time; restores the
-    chain state afterwards."""
+    """Picks the bytes-per-block target with the shortest time, ``reps`` iterations run as
+    the table would run them; restores the chain state afterwards. Without ``candidates`` the
+    default split is the first (None in ``tuned``) and stays unless a target is faster by
+    1%."""
     if candidates is None:
-      base = self.target_bytes
-      candidates = sorted({max(16 * 1024, int(base * f)) for f in (0.25, 0.5, 1, 2, 4, 8, 16)})
+      candidates = _target_candidates([self])
     snap = self._snapshot()
-    best = None
-    for tb in candidates:
-      self.target_bytes = tb
+
+    def timed(targets):
+      self.target_bytes = targets[0]
       self._build_table()
       self._launch_steps()
       torch.cuda.synchronize()
       t0 = time.perf_counter()
-      for _ in range(reps):
-        self._launch_steps()
+      self._launch_iterations(reps)
       torch.cuda.synchronize()
-      dt = (time.perf_counter() - t0) / reps
-      if best is None or dt < best[0]:
-        best = (dt, tb)
-    self.target_bytes = best[1]
+      return (time.perf_counter() - t0) / reps
+    dt, (self.target_bytes,) = _best_targets(1, candidates, timed)
+    tb = None if self._blocks_by_rule else self.target_bytes
     self._build_table()
     self._restore(snap)
     self._graph = None
-    self.tuned = {"target_bytes": best[1], "seconds_per_iteration": best[0],
-                  "candidates": candidates}
+    self.tuned = {"target_bytes": tb, "seconds_per_iteration": dt, "candidates": candidates}
     return self.tuned
+
+  def _launch_iterations(self, iterations):
+    """Evaluations of ``iterations`` iterations as run() launches them, without exchanges
+    and tests."""
+    if self.loop_capable() and self.prefer_loop is not False:
+      self._launch_loop(iterations)
+    else:
+      for _ in range(iterations):
+        self._launch_steps()
 
   def _snapshot(self):
     t = {k: getattr(self, k).clone() for k in ("theta_flat", "keys", "dkeys", "iter", "U", "var")}
@@ -553,6 +560,35 @@ class FusedGLM:
       if v is not None:
         getattr(self, k).copy_(v)
     torch.cuda.synchronize()
+
+
+def _target_candidates(engines):
+  """The autotuners' bytes-per-block targets: the default split (None) first where the
+  tables have it, then multiples of the largest table's target."""
+  base = max(e.target_bytes for e in engines)
+  sizes = sorted({max(16 * 1024, int(base * f)) for f in (0.25, 0.5, 1, 2, 4, 8, 16)})
+  return ([None] if any(e._blocks_by_rule for e in engines) else []) + sizes
+
+
+def _best_targets(tables, candidates, timed):
+  """(time, [target of each table]) with the shortest ``timed(targets)``: first one target
+  common to all tables, then each table's own, one table at a time. A target takes the place
+  of the default split (None) only where it is faster by 1%."""
+  best = None
+
+  def offer(targets, defaults):
+    nonlocal best
+    dt = timed(targets)
+    if best is None or dt < best[0] * (0.99 if defaults else 1.0):
+      best = (dt, targets)
+
+  for tb in candidates:
+    offer([tb] * tables, best is not None and best[1][0] is None)
+  for j in range(tables) if tables > 1 else []:
+    for tb in candidates:
+      if tb != best[1][j]:
+        offer([*best[1][:j], tb, *best[1][j + 1:]], best[1][j] is None)
+  return best
 
 
 # iterations issued by one sgmc_glm_fused_run call
@@ -767,16 +803,16 @@ class TableGroup:
     default all): first one target common to them, then each table's own, one table at
     a time. Each candidate is timed as a HIP graph in which every table of the group
     runs ``reps`` iterations' evaluations back to back on its stream (loop-capable
-    tables not being tuned in one loop launch, as they run), with HIP events around a
+    tables in one loop launch, as they run), with HIP events around a
     replay after a warm-up replay. Exchanges and tests are not launched; the chain
-    states are restored afterwards."""
+    states are restored afterwards. Without ``candidates`` the default split is the first
+    (None in ``tuned``) and stays unless a target is faster by 1%."""
     tables = list(range(len(self.engines))) if tables is None else list(tables)
     if not tables:
       return None
     eng = [self.engines[i] for i in tables]
     if candidates is None:
-      base = max(e.target_bytes for e in eng)
-      candidates = sorted({max(16 * 1024, int(base * f)) for f in (0.25, 0.5, 1, 2, 4, 8, 16)})
+      candidates = _target_candidates(eng)
     snaps = [e._snapshot() for e in self.engines]
     e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
     built = {}
@@ -785,19 +821,15 @@ class TableGroup:
       cur = torch.cuda.current_stream()
       for s in self.streams:
         s.wait_stream(cur)
-      for i, (e, s) in enumerate(zip(self.engines, self._table_streams())):
+      for e, s in zip(self.engines, self._table_streams()):
         with torch.cuda.stream(s):
-          if i not in tables and e.loop_capable():
-            e._launch_loop(reps)
-          else:
-            for _ in range(reps):
-              e._launch_steps()
+          e._launch_iterations(reps)
       for s in self.streams:
         cur.wait_stream(s)
 
     def timed(targets):
       for e, tb in zip(eng, targets):
-        if built.get(id(e)) != tb:
+        if built.get(id(e), 0) != tb:
           e.target_bytes = tb
           e._build_table()
           built[id(e)] = tb
@@ -816,20 +848,7 @@ class TableGroup:
       del g
       return e0.elapsed_time(e1) / 1e3 / reps
 
-    best = None
-    for tb in candidates:
-      dt = timed([tb] * len(eng))
-      if best is None or dt < best[0]:
-        best = (dt, [tb] * len(eng))
-    for j in range(len(eng)) if len(eng) > 1 else []:
-      for tb in candidates:
-        if tb == best[1][j]:
-          continue
-        trial = list(best[1])
-        trial[j] = tb
-        dt = timed(trial)
-        if dt < best[0]:
-          best = (dt, trial)
+    best = _best_targets(len(eng), candidates, timed)
     for e, tb in zip(eng, best[1]):
       e.target_bytes = tb
       e._build_table()

@@ -43,3 +43,25 @@ def test_saving_exchange_takes_the_split_of_launches():
   torch.cuda.synchronize()
   assert torch.equal(eng.theta_flat, want.theta_flat)
   assert torch.equal(ex.sample_trace(0), wex.sample_trace(0))
+
+
+@pytest.mark.parametrize("group", [False, True])
+def test_tuners_time_the_default_split(group):
+  print("tuners and the default split, group:", group, flush=True)
+  X, y = _data(5000, 100)
+  chains = [_chain(X, y, 100, 1000, c) for c in range(16)]
+  args = ("logistic", "sgld_rms", np.full(64, 1e-4, np.float32))
+  eng = (fused.TableGroup.split(chains, 2, *args) if group else fused.FusedGLM(chains, *args))
+  tables = eng.engines if group else [eng]
+  split = [e.nblocks_chain.tolist() for e in tables]
+  eng.run(3)
+  theta = [e.theta_flat.clone() for e in tables]
+  tuned = eng.autotune(reps=5)
+  assert tuned["candidates"][0] is None
+  chosen = tuned["target_bytes"] if group else [tuned["target_bytes"]]
+  for e, tb, nb, th in zip(tables, chosen, split, theta):
+    assert torch.equal(e.theta_flat, th)
+    if tb is None:
+      assert e.nblocks_chain.tolist() == nb
+    else:
+      assert e.nblocks_chain.tolist() == [fused.blocks_for(1000, 100, tb)] * e.C
