@@ -655,12 +655,11 @@ def mlp_posterior(torch, M, R, X, labels, th0, keys, dkeys, dims, n, prec, integ
 
 
 def tile_label(names, key):
-  """'G1 k128 s2' for a (slot, code) timing, 'G4+G5 k32 k128' for a joint one."""
+  """'G1 s2' for the timing of a (slot, code), 'chosen' for that of the final plan."""
   if len(key) == 2:
     i, c = key
-    return f"{names[i].split()[0]} k{c >> 4} s{c & 15}"
-  _, c4, c5 = key
-  return f"G4+G5 k{c4 >> 4} k{c5 >> 4}"
+    return f"{names[i].split()[0]} s{c & 15}"
+  return "chosen"
 
 
 def tune_tiles(eng, args):
@@ -677,15 +676,14 @@ def tune_tiles(eng, args):
   elif args.no_autotune:
     plan, how = eng.gemm_plan(), {"source": "built-in"}
   else:
-    log("autotune: GEMM k-tile depth and split-K on the live problem")
+    log("autotune: split-K of the forward GEMMs on the live problem")
     plan = eng.autotune()
     b, t = eng.tune_gain
     how = {"source": "autotune", "unit_ms_builtin": b, "unit_ms_tuned": t,
            "unit_ms": {tile_label(names, key): round(ms, 5)
                        for key, ms in sorted(eng.tune_ms.items())}}
-  tiles = {nm: {"BM": 64, "BN": 128, "BK": k, "split_k": s} for nm, (k, s) in zip(names, plan)}
-  # gW2 runs in gW1's launch when both take the same k-tile
-  return dict(how, tiles=tiles, gw1_gw2_one_launch=plan[3] == plan[4])
+  tiles = {nm: {"split_k": sp} for nm, (_, sp) in zip(names, plan)}
+  return dict(how, tiles=tiles)
 
 
 def run_mlp(args):

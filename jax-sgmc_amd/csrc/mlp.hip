@@ -930,7 +930,9 @@ int make_step(const sgmc_mlp_state* st, int update, Layout& L, Step& s) {
   s.fp32 = q.precision == 2 ? 1 : 0;
   const int trc = check_tune(q.D_in, q.H1, q.H2, q.n, q.precision, q.tune);
   if (trc != SGMC_OK) return trc;
-  plan_gemms(q.D_in, q.H1, q.H2, q.n, q.C, q.precision, update, q.tune, s.plan);
+  int plan[kSlots];
+  plan_gemms(q.D_in, q.H1, q.H2, q.n, q.C, q.precision, update, q.tune, plan);
+  for (int i = SLOT_G1; i <= SLOT_G3; ++i) s.split[i] = plan[i] & 15;
   s.q = q.q;
   s.shadow8 = q.shadow8;
   if (s.fp8)
@@ -990,10 +992,10 @@ void launch_forward(const Step& s, const sgmc_mlp_state& q, hipStream_t st_) {
   const void* W2 = gemm_weight(s, q, 1);
   Gemm g1{s.Xb, q.D_in, (int64_t)n * q.D_in, W1, q.H1, q.P, n, q.H1, q.D_in,
           s.h1, q.H1, (int64_t)n * q.H1, q.theta + s.off[3], q.P, nullptr, 0, 0, 0, 0};
-  launch_act_gemm(with_q(g1, Q_X, Q_W1, Q_H1), s, st_, s.plan[SLOT_G1] & 15);
+  launch_act_gemm(with_q(g1, Q_X, Q_W1, Q_H1), s, st_, s.split[SLOT_G1]);
   Gemm g2{s.h1, q.H1, (int64_t)n * q.H1, W2, q.H2, q.P, n, q.H2, q.H1,
           s.h2, q.H2, (int64_t)n * q.H2, q.theta + s.off[4], q.P, nullptr, 0, 0, 0, 0};
-  launch_act_gemm(with_q(g2, Q_H1, Q_W2, -1), s, st_, s.plan[SLOT_G2] & 15);
+  launch_act_gemm(with_q(g2, Q_H1, Q_W2, -1), s, st_, s.split[SLOT_G2]);
   launch_head(s, st_);
 }
 
@@ -1027,7 +1029,7 @@ int sgmc_mlp_step(const sgmc_mlp_state* st, int update, void* stream) {
   // dA1 = (dA2 W2^T) * (H1 > 0): B[k=b][n=a] = W2[a][b], k-contiguous rows of W2.
   Gemm g3{s.da2, q.H2, (int64_t)n * q.H2, W2, q.H2, q.P, n, q.H1, q.H2,
           s.da1, q.H1, (int64_t)n * q.H1, nullptr, 0, s.h1, q.H1, (int64_t)n * q.H1, 0, 0};
-  launch_act_gemm(with_q(g3, Q_DA2, Q_W2, Q_DA1), s, st_, s.plan[SLOT_G3] & 15);
+  launch_act_gemm(with_q(g3, Q_DA2, Q_W2, Q_DA1), s, st_, s.split[SLOT_G3]);
   // gW2 = H1^T dA2: A[m=a][k=i] = H1[i][a] (m-contiguous), B[k=i][n=b] = dA2[i][b].
   Gemm g4{s.h1, q.H1, (int64_t)n * q.H1, s.da2, q.H2, (int64_t)n * q.H2, q.H1, q.H2, n,
           nullptr, 0, 0, nullptr, 0, nullptr, 0, 0, 1, 0};

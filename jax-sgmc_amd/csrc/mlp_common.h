@@ -124,7 +124,7 @@ struct Step {
   // fp8 GEMM operands (Xb, h1, da2, da1 and the W1 / W2 shadows in e4m3)
   int fp8;
   int fp32;                // float32 activations and GEMM operands (weights from theta)
-  int plan[5];             // per GEMM (G1..G5): 16 k-tile + split-K factor
+  int split[3];            // split-K factors of G1, G2, G3
   float* q;                // [C][kQWords]
   uint8_t* shadow8;        // [C][P] (W1 and W2 leaves)
 };

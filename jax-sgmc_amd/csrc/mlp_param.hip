@@ -48,9 +48,11 @@ __device__ __forceinline__ void st4(f32x4 v, __amdgpu_buffer_rsrc_t r, uint32_t 
 
 typedef uint32_t u32_2 __attribute__((aligned(2)));  // e4m3 copies of odd chains
 
+constexpr int BW = 32;  // 64 x 64 tiles: 134 us for 124 (pSGLD), 316 for 295 (e4m3 OBA)
+
 // Block `lin` of a GEMM: 2 BW rows of the leaf (BW and, half the leaf further, BW more) by
 // TN = 4096 / BW columns, chain c. Four wavefronts of 64 x 32 each.
-template <int PREC, int BW, int EPI, int UM>
+template <int PREC, int EPI, int UM>
 __device__ __forceinline__ void param_tile(const Gemm& g, const Step& s, uint32_t lin,
                                            uint32_t gx, uint32_t gy, uint8_t* lds, float* red) {
   constexpr bool F8 = PREC == P_FP8;
@@ -230,7 +232,7 @@ __device__ __forceinline__ void param_tile(const Gemm& g, const Step& s, uint32_
 // column sums (colx per strip), which need the same activations and none of the parameters:
 // latency-bound on their own (20 us in e4m3, 8 in bf16, 6 in float32), here they run beside the
 // update (16 chains of 3072-512-512 bf16 121 + 8 -> 125 us, 4 chains in float32 47 + 6 -> 47).
-template <int PREC, int BW, int EPI, int UM>
+template <int PREC, int EPI, int UM>
 __global__ void __launch_bounds__(GT, kWavesPerSimd)
     param_kernel(Gemm ga, Gemm gb, Step s, uint32_t gxa, uint32_t gya, uint32_t gxb, uint32_t gyb,
                  uint32_t ncol, uint32_t colx) {
@@ -248,12 +250,12 @@ __global__ void __launch_bounds__(GT, kWavesPerSimd)
   const bool rev = s.mode == MLP_SGLD ? (cur_iter(s) & 1) != 0 : s.mode == MLP_OBABO_BO;
   const uint32_t lin = rev ? gridDim.x - 1 - blockIdx.x : blockIdx.x - ncol;
   if (lin < na)
-    param_tile<PREC, BW, EPI, UM>(ga, s, lin, gxa, gya, lds, red);
+    param_tile<PREC, EPI, UM>(ga, s, lin, gxa, gya, lds, red);
   else
-    param_tile<PREC, BW, EPI, UM>(gb, s, lin - na, gxb, gyb, lds, red);
+    param_tile<PREC, EPI, UM>(gb, s, lin - na, gxb, gyb, lds, red);
 }
 
-template <int PREC, int BW, int EPI, int UM>
+template <int PREC, int EPI, int UM>
 void launch(const Gemm& ga, const Gemm& gb, const Step& s, hipStream_t st) {
   constexpr int W = 2 * BW, TN = 4096 / BW;
   const uint32_t gxa = (uint32_t)(ga.M / W), gya = (uint32_t)(ga.N / TN);
@@ -261,7 +263,7 @@ void launch(const Gemm& ga, const Gemm& gb, const Step& s, hipStream_t st) {
   // the column sums' blocks first, padded to whole rounds over the XCDs
   const uint32_t colx = (uint32_t)colsum_blocks(s);
   const uint32_t ncol = (colx * (uint32_t)(s.n / kStrip) * (uint32_t)s.C + kXcds - 1) / kXcds * kXcds;
-  hipLaunchKernelGGL((param_kernel<PREC, BW, EPI, UM>),
+  hipLaunchKernelGGL((param_kernel<PREC, EPI, UM>),
                      dim3(ncol + (gxa * gya + gxb * gyb) * (uint32_t)s.C), dim3(GT), 0, st, ga, gb,
                      s, gxa, gya, gxb, gyb, ncol, colx);
 }
@@ -269,12 +271,11 @@ void launch(const Gemm& ga, const Gemm& gb, const Step& s, hipStream_t st) {
 // the update rule compiled in: rms_prop SGLD and the two OBABO halves; plain SGLD at run time
 template <int PREC>
 void by_rule(const Gemm& ga, const Gemm& gb, const Step& s, hipStream_t st) {
-  constexpr int BW = 32;  // 64 x 64 tiles: 134 us for 124 (pSGLD), 316 for 295 (e4m3 OBA)
-  if (!s.update) launch<PREC, BW, EPI_GRAD, UM_ANY>(ga, gb, s, st);
-  else if (s.mode == MLP_OBABO_BA) launch<PREC, BW, EPI_UPDATE, UM_OBA>(ga, gb, s, st);
-  else if (s.mode == MLP_OBABO_BO) launch<PREC, BW, EPI_UPDATE, UM_OBO>(ga, gb, s, st);
-  else if (s.rms) launch<PREC, BW, EPI_UPDATE, UM_RMS>(ga, gb, s, st);
-  else launch<PREC, BW, EPI_UPDATE, UM_ANY>(ga, gb, s, st);
+  if (!s.update) launch<PREC, EPI_GRAD, UM_ANY>(ga, gb, s, st);
+  else if (s.mode == MLP_OBABO_BA) launch<PREC, EPI_UPDATE, UM_OBA>(ga, gb, s, st);
+  else if (s.mode == MLP_OBABO_BO) launch<PREC, EPI_UPDATE, UM_OBO>(ga, gb, s, st);
+  else if (s.rms) launch<PREC, EPI_UPDATE, UM_RMS>(ga, gb, s, st);
+  else launch<PREC, EPI_UPDATE, UM_ANY>(ga, gb, s, st);
 }
 
 }  // namespace

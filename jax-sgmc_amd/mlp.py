@@ -76,8 +76,8 @@ class FusedMLP:
   "bf16" on bf16 operands and a bf16 shadow of the parameters; "fp8" on e4m3 operands
   with per-tensor delayed scaling. State, noise and updates are float32 in all three.
 
-  ``tune`` (five ints, see sgmc_mlp_state.tune) overrides the k-tile depth and split-K
-  factor of each GEMM; autotune() chooses them by timing the live problem."""
+  ``tune`` (five ints, see sgmc_mlp_state.tune) overrides the split-K factor of each forward
+  GEMM; autotune() chooses them by timing the live problem."""
 
   def __init__(self, X, labels, dims, n, theta0, eps_table, keys=None, dkeys=None, rms=False,
                alpha=0.9, lmbd=1e-5, prior_scale=1.0, has_prior=True, temperature=1.0,
@@ -246,12 +246,17 @@ class FusedMLP:
     return [(v >> 4, v & 15) for v in out]
 
   def tile_candidates(self, slot):
-    """Codes 16 k + s that sgmc_mlp_step accepts for GEMM `slot` at these shapes."""
+    """One code 16 k + s that sgmc_mlp_step accepts for GEMM `slot` at these shapes per
+    split-K factor s (the k-tile only takes part in which splits fit: the plan's, else the
+    first that does)."""
     D_in, H1, H2 = self.dims
     K = (D_in, H1, H2, self.n, self.n)[slot]
-    depths = {"fp32": (32,), "fp8": (64, 128), "bf16": (32, 128)}[self.precision]
+    depths = [self.gemm_plan()[slot][0]]
+    depths += [k for k in {"fp32": (32,), "fp8": (64, 128), "bf16": (32, 128)}[self.precision]
+               if k not in depths]
     splits = (1, 2, 3, 4) if slot < 3 else (1,)
-    return [k * 16 + s for k in depths for s in splits if K % (k * s) == 0]
+    fits = [[k * 16 + s for k in depths if K % (k * s) == 0] for s in splits]
+    return [codes[0] for codes in fits if codes]
 
   def _mutable(self):
     names = ("theta", "v", "shadow", "shadow8", "q", "keys", "dkeys", "U", "iter", "counters",
@@ -260,18 +265,17 @@ class FusedMLP:
     return [t for t in (getattr(self, n) for n in names) if t is not None]
 
   def autotune(self, reps=20, min_gain=0.01):
-    """Chooses the k-tile depth and split-K factor of each GEMM by timing the live
+    """Chooses the split-K factor of each forward GEMM by timing the live
     problem (HIP events on the launch stream around `reps` back-to-back units after one
     warm-up unit): whole iterations for SGLD, one OBABO step (two evaluations, the unit
-    OBABO and SGGMC iterations repeat) otherwise. The forward GEMMs one at a time, then the
-    two parameter GEMMs jointly (they share a launch), starting from the
-    built-in choice; a candidate replaces the current one only if it is faster by more
+    OBABO and SGGMC iterations repeat) otherwise. The forward GEMMs one at a time, starting
+    from the built-in choice (the parameter GEMMs have no other); a candidate replaces the current one only if it is faster by more
     than `min_gain`. Each timing starts from a snapshot of the engine's state (the
     iteration counter runs at most reps + 1 past it; the schedule tables clamp it),
     which is restored at the end, so the chains continue where they were. Sets
-    self.tune (and self.tune_ms: the time per unit of every plan tried, keyed (slot, code)
-    and (3, gW2 code, gW1 code), self.tune_gain:
-    (built-in ms, tuned ms)) and returns gemm_plan()."""
+    self.tune (and self.tune_ms: the time per unit of every plan tried, keyed (slot, code),
+    and of the final one as (3, gW2 code, gW1 code), self.tune_gain: (built-in ms, tuned ms))
+    and returns gemm_plan()."""
     unit = self.iteration if self.integrator == "sgld" else self.obabo_step
     tensors = self._mutable()
     snap = [t.clone() for t in tensors]
@@ -308,20 +312,7 @@ class FusedMLP:
         if t < best * (1.0 - min_gain):
           best, best_code = t, code
       self.tune[slot] = best_code
-    # the parameter GEMMs jointly: gW2 runs in gW1's launch,
-    # so they are timed together (tune_ms[(3, c4, c5)])
-    best_pair = (self.tune[3], self.tune[4])
-    self.tune_ms[(3,) + best_pair] = best
-    for c4 in self.tile_candidates(3):
-      for c5 in self.tile_candidates(4):
-        if (c4, c5) == best_pair:
-          continue
-        self.tune[3], self.tune[4] = c4, c5
-        t = timed()
-        self.tune_ms[(3, c4, c5)] = t
-        if t < best * (1.0 - min_gain):
-          best, best_pair = t, (c4, c5)
-    self.tune[3], self.tune[4] = best_pair
+    self.tune_ms[(3, self.tune[3], self.tune[4])] = best
     self.tune_gain = (builtin, best)
     restore()
     torch.cuda.synchronize()
