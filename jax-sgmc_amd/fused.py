@@ -362,14 +362,6 @@ class FusedGLM:
     return (self.mode in _LOOPS and self.mh is None and
             (self.exchange is None or self.exchange.sparse))
 
-  def _launch_loop(self, iterations):
-    _lib.call("sgmc_glm_fused_loop", _lib.ptr(self.table), self.C, self.uniform_dclass,
-              self.family, self.sigma, self.has_prior, self.prior_scale, self.pot_temperature,
-              self.mode, self.steps, self.friction, self.alpha, self.lmbd,
-              _lib.ptr(self.inv_mass), _lib.ptr(self.sqrt_mass), _lib.ptr(self.eps_table),
-              self.table_len, _lib.ptr(self.save_slot), _lib.ptr(self.iter),
-              _lib.ptr(self.done), int(iterations), _lib.stream())
-
   def _plan(self, iterations, loop):
     """Launch sequence of ``iterations`` iterations starting after host_iter: ("it",)
     one iteration's evaluations, ("loop", k) k iterations in one loop launch, ("swap",)
@@ -524,7 +516,7 @@ class FusedGLM:
     def timed(targets):
       self.target_bytes = targets[0]
       self._build_table()
-      self._launch_steps()
+      self._launch_iterations(1)
       torch.cuda.synchronize()
       t0 = time.perf_counter()
       self._launch_iterations(reps)
@@ -538,14 +530,17 @@ class FusedGLM:
     self.tuned = {"target_bytes": tb, "seconds_per_iteration": dt, "candidates": candidates}
     return self.tuned
 
-  def _launch_iterations(self, iterations):
-    """Evaluations of ``iterations`` iterations as run() launches them, without exchanges
-    and tests."""
+  def _bare_plan(self, iterations):
+    """The launches of ``iterations`` iterations as run() plans them, without exchanges and
+    tests."""
     if self.loop_capable() and self.prefer_loop is not False:
-      self._launch_loop(iterations)
-    else:
-      for _ in range(iterations):
-        self._launch_steps()
+      return [("loop", iterations)]
+    return [("it",)] * iterations
+
+  def _launch_iterations(self, iterations):
+    start = self.host_iter
+    self._execute(self._bare_plan(iterations))
+    self.host_iter = start
 
   def _snapshot(self):
     t = {k: getattr(self, k).clone() for k in ("theta_flat", "keys", "dkeys", "iter", "U", "var")}
@@ -756,11 +751,6 @@ class TableGroup:
     for s in self.streams:
       cur.wait_stream(s)
 
-  def _side_stream(self):
-    if getattr(self, "_side", None) is None:
-      self._side = torch.cuda.Stream(device=self.engines[0].device)
-    return self._side
-
   def _table_streams(self):
     return [self.streams[i] for i in self.stream_of]
 
@@ -801,11 +791,10 @@ class TableGroup:
   def autotune(self, candidates=None, reps=50, tables=None):
     """Chooses the bytes-per-block target of the tables listed in ``tables`` (indices;
     default all): first one target common to them, then each table's own, one table at
-    a time. Each candidate is timed as a HIP graph in which every table of the group
-    runs ``reps`` iterations' evaluations back to back on its stream (loop-capable
-    tables in one loop launch, as they run), with HIP events around a
-    replay after a warm-up replay. Exchanges and tests are not launched; the chain
-    states are restored afterwards. Without ``candidates`` the default split is the first
+    a time. For each candidate every table of the group runs ``reps`` iterations'
+    evaluations on its stream as run() launches them (loop-capable tables in one loop
+    launch), between HIP events, after a warm-up of the same. Exchanges and tests are not
+    launched; the chain states are restored afterwards. Without ``candidates`` the default split is the first
     (None in ``tuned``) and stays unless a target is faster by 1%."""
     tables = list(range(len(self.engines))) if tables is None else list(tables)
     if not tables:
@@ -816,36 +805,20 @@ class TableGroup:
     snaps = [e._snapshot() for e in self.engines]
     e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
     built = {}
-
-    def block():
-      cur = torch.cuda.current_stream()
-      for s in self.streams:
-        s.wait_stream(cur)
-      for e, s in zip(self.engines, self._table_streams()):
-        with torch.cuda.stream(s):
-          e._launch_iterations(reps)
-      for s in self.streams:
-        cur.wait_stream(s)
+    start = [e.host_iter for e in self.engines]
 
     def timed(targets):
+      torch.cuda.synchronize()  # nothing runs on the tables that are replaced
       for e, tb in zip(eng, targets):
         if built.get(id(e), 0) != tb:
           e.target_bytes = tb
           e._build_table()
           built[id(e)] = tb
-      g = torch.cuda.CUDAGraph()
-      side = self._side_stream()
-      side.wait_stream(torch.cuda.current_stream())
-      with _lib.capture_guard(), torch.cuda.stream(side):
-        with torch.cuda.graph(g, stream=side):
-          block()
-      torch.cuda.current_stream().wait_stream(side)
-      g.replay()
+      self._run_plans(lambda e: e._bare_plan(reps))
       e0.record()
-      g.replay()
+      self._run_plans(lambda e: e._bare_plan(reps))
       e1.record()
       e1.synchronize()
-      del g
       return e0.elapsed_time(e1) / 1e3 / reps
 
     best = _best_targets(len(eng), candidates, timed)
@@ -853,8 +826,9 @@ class TableGroup:
       e.target_bytes = tb
       e._build_table()
       e._graph = None
-    for e, snap in zip(self.engines, snaps):
+    for e, snap, k in zip(self.engines, snaps, start):
       e._restore(snap)
+      e.host_iter = k
     self._graphs = None
     self.tuned = {"target_bytes": best[1], "seconds_per_iteration": best[0],
                   "candidates": list(candidates), "tables": tables}

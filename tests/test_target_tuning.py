@@ -20,6 +20,7 @@ class Clock:
     e.target_bytes = None if by_rule else 64 << 10
     e.loop_capable = lambda: False
     e._build_table, e._launch_steps = self.build, self.launch
+    e._launch_iterations = lambda k: [self.launch() for _ in range(k)]
     e._snapshot, e._restore = dict, lambda s: None
     self.engine = e
 
