@@ -23,8 +23,9 @@ prior, the data loader is device-resident, and the integrator is SGLD (with or
 without rms_prop), SGHMC or OBABO with unit mass and scalar friction, all chains run
 together in the fused multi-chain kernel (``fused.FusedGLM``); AMAGOLD and SGGMC do
 too when the full potential is the same family, followed by one full-data pass for
-all chains and the Metropolis-Hastings kernel. The result is the same chain by chain.
-Otherwise the chains run one after another through the modular kernels (solver.mcmc
+all chains and the Metropolis-Hastings kernel. A chain draws the same minibatches and noise
+however many run beside it; its float32 sums are split by the number of chains, so runs of
+different numbers of chains agree within rounding. Otherwise the chains run one after another through the modular kernels (solver.mcmc
 with strategy 'map', as in the reference).
 """
 from functools import partial
@@ -133,7 +134,7 @@ def _run_fused(potential_fn, data_loader, batch_size, init_samples, iterations, 
   multi = any(FU.blocks_for(int(c["n"]), int(c["D"]), tb) > 1 for c in chains)
   if len(chains) >= _TABLE_SPLIT_CHAINS and multi:
     # many multi-block chains: two tables on two streams, so that one table's launch
-    # tail overlaps the other's row gather (same results chain by chain)
+    # tail overlaps the other's row gather (each table splits its own chains into blocks)
     eng = FU.TableGroup.split(chains, 2, lik.family, mode, eps, **kw)
   else:
     eng = FU.FusedGLM(chains, lik.family, mode, eps, **kw)

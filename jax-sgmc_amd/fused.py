@@ -10,10 +10,13 @@ on the device, so a captured HIP graph of one or more iterations replays without
 host input.
 
 Chains may differ in dataset, N, D (<= 1024), minibatch size and temperature
-(tempering ladders); they share the family, the prior and the integrator. Per-chain
-results equal the same chain run alone (chains are independent; every chain owns
-its keys and its reduction order is fixed by its own block count). TableGroup runs
-several tables side by side on their own streams; ReplicaExchange, AmagoldMH and
+(tempering ladders); they share the family, the prior and the integrator. Chains are
+independent: every chain owns its keys, and its reduction order is fixed by its own block
+count. With equal block counts (a ``target_bytes``, which splits every chain by itself) a
+chain gives the same bits alone and in any table. The default split shares one block per
+compute unit among the chains of a table, so with it a chain alone, in another table or on
+a card with another number of units may sum its rows in another order and agrees within
+float32 rounding. TableGroup runs several tables side by side on their own streams; ReplicaExchange, AmagoldMH and
 SggmcMH attach a swap or Metropolis-Hastings step to a table.
 """
 import ctypes
@@ -44,7 +47,7 @@ def _align4(x):
   return (x + 3) // 4 * 4
 
 
-# Rows per block whose likelihoods a fused block stages in LDS (kLdsRows in glm.hip).
+# Rows per block whose likelihoods a fused block stages in LDS (kLdsRows in glm_rows.h).
 LDS_ROWS = 4096
 
 

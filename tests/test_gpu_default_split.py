@@ -69,3 +69,36 @@ def test_tuners_time_the_default_split(group):
       assert e.nblocks_chain.tolist() == nb
     else:
       assert e.nblocks_chain.tolist() == [fused.blocks_for(1000, 100, tb)] * e.C
+
+
+@pytest.mark.parametrize("D,n", [(100, 1000), (24, 600)])
+def test_chain_alone_and_in_tables(D, n):
+  """One SGLD step of chain 0 alone, among 16 and among the 8 of a group's table. Two orders
+  of a float32 sum of n terms differ by at most 2 n 2^-24 sum |terms|; |dlik/dz| <= 1, so
+  a column's terms add up to at most sum |x|, and the step scales the sum by eps N / n."""
+  print("default split, chain alone and in tables", D, n, flush=True)
+  N, eps = 3000, 1e-5
+  X, y = _data(N, D)
+  chains = [_chain(X, y, D, n, c) for c in range(16)]
+  args = ("logistic", "sgld", np.full(4, eps, np.float32))
+
+  def step(eng, table):
+    eng.run(1)
+    torch.cuda.synchronize()
+    return table.theta(0).clone(), table.nblocks_chain[0], table.U[0].item()
+  alone = fused.FusedGLM(chains[:1], *args)
+  single = fused.FusedGLM(chains, *args)
+  halves = fused.TableGroup.split(chains, 2, *args)
+  got = [step(alone, alone), step(single, single), step(halves, halves.engines[0])]
+  terms = n * X[:, :D].abs().max(0).values  # of any minibatch
+  tol = eps * N / n * 2 * n * 2.0 ** -24 * terms + 2.0 ** -23 * got[0][0].abs()
+  for th, nb, U in got[1:]:
+    assert ((th - got[0][0]).abs() <= tol).all()
+    assert abs(U - got[0][2]) <= 2 * n * 2.0 ** -24 * abs(got[0][2])
+  if D == 100:
+    assert len({nb for _, nb, _ in got}) > 1  # or this compares one split with itself
+  target = n * 400
+  same = [step(e, t)[0] for e, t in
+          [(e, e) for e in (fused.FusedGLM(chains[:1], *args, target_bytes=target / 4),
+                            fused.FusedGLM(chains, *args, target_bytes=target / 4))]]
+  assert torch.equal(same[0], same[1])
