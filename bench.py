@@ -469,7 +469,6 @@ def run_ladder(args):
   big = [i for i, e in enumerate(grp.engines) if not e.loop_capable()]
   tuned = grp.autotune(tables=big)
   log(f"autotune: {tuned}")
-  assert all(e.loop_capable() == (d <= 64) for e, d in zip(grp.engines, dims))
   grp.capture(G)
   grp.run(max(1, W // G) * G, G)
   torch.cuda.synchronize()

@@ -27,6 +27,8 @@ class Clock:
   def build(self):
     e = self.engine
     self.built = "default" if e._blocks_by_rule else e.target_bytes
+    # 1 MiB in blocks; a default split that no target gives
+    e.nblocks_chain = [13 if e._blocks_by_rule else (1 << 20) // e.target_bytes]
 
   def launch(self):
     self.now += self.cost(self.built)
@@ -47,11 +49,47 @@ def test_table_keeps_its_default_split(monkeypatch, default, best, kept):
   assert c.built in (16 << 10, 32 << 10)
 
 
+class Table:
+  nblocks_chain = ()
+
+
+def best_of(cost, candidates, tables, splits=None):
+  """_best_targets over simulated costs; the split of a target is itself unless given."""
+  engines = [Table() for _ in range(tables)]
+  now = []
+
+  def build(targets):
+    now[:] = targets
+    for e, tb in zip(engines, targets):
+      e.nblocks_chain = [(splits or {}).get(tb, 0 if tb is None else tb)]
+  return fused._best_targets(engines, candidates, build, lambda: cost[tuple(now)])
+
+
 def test_tables_of_a_group_choose_one_by_one():
   cost = {(None, None): 10.0, (1, 1): 9.95, (2, 2): 12.0, (None, 1): 9.8, (None, 2): 11.0,
           (1, None): 12.0, (2, None): 13.0, (2, 1): 13.0}
-  assert fused._best_targets(2, [None, 1, 2], lambda t: cost[tuple(t)]) == (9.8, [None, 1])
-  assert fused._best_targets(1, [2, 1], lambda t: {1: 1.0, 2: 1.001}[t[0]]) == (1.0, [1])
+  assert best_of(cost, [None, 1, 2], 2) == (9.8, [None, 1])
+  assert best_of({(2,): 1.001, (1,): 1.0}, [2, 1], 1) == (1.0, [1])
+
+
+def test_a_target_with_the_default_split_is_not_timed_again():
+  cost = {(None,): 10.0, (1,): 9.0, (2,): 11.0}
+  assert best_of(cost, [None, 1, 2], 1, {None: 4, 1: 4, 2: 8}) == (10.0, [None])
+
+
+def test_a_slow_first_timing_does_not_cost_the_default_split():
+  """The clocks settle while the default split is timed: it is timed again against the best
+  target."""
+  e, now, count = Table(), [], [0]
+
+  def build(targets):
+    now[:] = targets
+    e.nblocks_chain = [0 if targets[0] is None else targets[0]]
+
+  def timed():
+    count[0] += 1
+    return (10.0 if now[0] is None else 10.1) * (1.2 if count[0] <= 4 else 1.0)
+  assert fused._best_targets([e], [None, 1, 2], build, timed) == (10.0, [None])
 
 
 def test_candidates():
