@@ -11,7 +11,7 @@
 // Threefry block, integrator.py:119-135), its state moves in 16-byte accesses that cover
 // whole lines, and the first of them are in flight before the product is begun.
 // Against a lane per parameter pair, 4-byte accesses and operands transposed in registers:
-// that step's update 163 -> 121 us (694 MB of traffic with the operands, 5.7 TB/s); 16
+// that step's update 163 -> 121 us (611 MB beyond the L2 with the operands, 5.0 TB/s); 16
 // chains of 3072-1024-1024 in e4m3, n = 512: OBA half 378 -> 279 us, BO half 252 -> 204 us,
 // gradient 210 -> 161 us; float32 gradient of 4 chains of 3072-512-512 55 -> 47 us.
 #include "mlp_colsum.h"
