@@ -270,10 +270,12 @@ __device__ __forceinline__ void process_group(RowGroup<LPR, CPL>& g, int row0, i
 // the row ids of the next 64-row chunk are drawn before the current chunk is done. mid()
 // runs (on every wavefront, also one without rows) when the first loads are in flight: it
 // sets th, and whatever else does not depend on the rows is hidden behind them.
-// The float32 sums are kept in two levels, chunks of 64 rows and their sum: a wavefront of a
-// long block adds hundreds of rows per lane (256 at 64 chains of n = 4096), and one running
-// sum over them rounds more than the many short blocks of a finer split did (SGHMC of 64
-// chains against 64 bits: @ERR@).
+// Where a lane adds every row (D > 128), the float32 sums are kept in two levels, chunks of 64
+// rows and their sum: a wavefront of a long block has hundreds of rows (256 at 64 chains of
+// n = 4096), and one running sum over them rounds more than the many short blocks of a finer
+// split did. Errors of SGHMC of 64 chains, n = 4096, against 64 bits, one sum and two levels:
+// D = 200 2.6e-7 2.5e-7, D = 512 2.9e-7 2.6e-7, D = 900 2.5e-7 2.4e-7, at the same times within
+// 0.5%; D = 60 and 100, several rows per load, 3.9e-7 and 5.0e-7 either way (and 1% slower).
 template <int LPR, int CPL, class Mid>
 __device__ __forceinline__ void accumulate_rows(gcfloat* __restrict__ X, int64_t ldx,
                                                 gcfloat* __restrict__ y, int D4,
@@ -283,6 +285,7 @@ __device__ __forceinline__ void accumulate_rows(gcfloat* __restrict__ X, int64_t
                                                 float* lds_lik, int lds_row0, Mid mid) {
   constexpr int RPW = kWave / LPR;
   constexpr int G = RPW * RowGroup<LPR, CPL>::U;  // rows per group; divides 64
+  constexpr bool kTwo = RPW == 1;  // sums in two levels
   static_assert(kWave % G == 0, "row groups must tile a 64-row chunk");
   if (r0 >= r1) {
     mid();
@@ -320,7 +323,7 @@ __device__ __forceinline__ void accumulate_rows(gcfloat* __restrict__ X, int64_t
     process_group<LPR, CPL>(ga, cb + gl, D4, th, L, acc, lik_acc, lds_lik, lds_row0);
     if (!more) break;
     if (next) {
-      fold();
+      if (kTwo) fold();
       cb += kWave;
       nl = 0;
       rid = rid_n;
@@ -334,7 +337,7 @@ __device__ __forceinline__ void accumulate_rows(gcfloat* __restrict__ X, int64_t
     process_group<LPR, CPL>(gb, cb + gl, D4, th, L, acc, lik_acc, lds_lik, lds_row0);
     if (!more) break;
     if (next) {
-      fold();
+      if (kTwo) fold();
       cb += kWave;
       nl = 0;
       rid = rid_n;
@@ -342,7 +345,7 @@ __device__ __forceinline__ void accumulate_rows(gcfloat* __restrict__ X, int64_t
     }
     gl = nl;
   }
-  if (r1 - r0 > kWave) {
+  if (kTwo && r1 - r0 > kWave) {
     fold();
 #pragma unroll
     for (int k = 0; k < CPL; ++k) acc[k] = tot[k];

@@ -1,8 +1,8 @@
 """Rounding of the float32 sums over the rows of one long block (GPU): 4096 equal terms
 t = 1 + 2^-15 - 2^-23, which a running sum rounds down at every addition once it is past 512
-(2e-5 relative after a wavefront's 1024). Sums of 64 rows, added up, stay within
-(64 + 16 + 4 + 8) 2^-24 = 5.5e-6: at most 64 additions of a lane in a chunk, 16 chunks of a
-wavefront, 4 wavefronts, the scaling."""
+(2e-5 relative after a wavefront's 1024; a lane that shares them with others, at D <= 128, adds
+at most 512). Sums of 64 rows, added up, stay within (64 + 16 + 4 + 8) 2^-24 = 5.5e-6: at most
+64 additions of a lane in a chunk, 16 chunks of a wavefront, 4 wavefronts, the scaling."""
 import pytest
 import torch
 
