@@ -14,7 +14,6 @@
 
 #include <algorithm>
 #include <mutex>
-#include <vector>
 
 #include "glm_fused.h"
 
@@ -476,6 +475,61 @@ void launch_loop_mode(const sgmc_glm_run& r, int iterations, FusedArgs a) {
   }
 }
 
+// Tables whose launches one call takes in turn.
+constexpr int kTogether = 64;
+
+// Issues the operations of up to kTogether checked tables, one launch per table and turn.
+int issue_runs(const sgmc_glm_run* runs, int nruns) {
+  struct Cursor {
+    int op = 0;
+    int64_t at = 0;  // launches of the operation issued so far
+  };
+  Cursor cur[kTogether];
+  for (bool any = true; any;) {
+    any = false;
+    for (int k = 0; k < nruns; ++k) {
+      const sgmc_glm_run& r = runs[k];
+      Cursor& c = cur[k];
+      while (c.op < r.nops) {
+        const int count = r.ops[2 * c.op + 1];
+        const int64_t total = r.ops[2 * c.op] == SGMC_OP_ITERATIONS
+                                  ? (int64_t)count * launches_of(r)
+                                  : r.ops[2 * c.op] == SGMC_OP_LOOP ? (count > 0) : count;
+        if (c.at < total) break;
+        ++c.op;
+        c.at = 0;
+      }
+      if (c.op == r.nops) continue;
+      any = true;
+      int rc;
+      switch (r.ops[2 * c.op]) {
+        case SGMC_OP_ITERATIONS: {
+          FusedArgs a = run_args(r);
+          a.step = (int)(c.at % launches_of(r));
+          launch_step(r, a);
+          rc = check_launch("sgmc_glm_fused_run");
+          break;
+        }
+        case SGMC_OP_LOOP: {
+          FusedArgs a = run_args(r);
+          a.blocks_per_chain = 1;
+          a.block_chain = nullptr;
+          a.advance = -1;
+          launch_loop_mode(r, r.ops[2 * c.op + 1], a);
+          rc = check_launch("sgmc_glm_fused_run");
+          break;
+        }
+        default:
+          rc = sgmc_resgld_swap(r.chains, r.nchains, r.pairs, r.npairs, r.F, r.swap_every,
+                                r.save_slot, r.table_len, r.iter, r.stream);
+      }
+      if (rc != SGMC_OK) return rc;
+      ++c.at;
+    }
+  }
+  return SGMC_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -718,53 +772,10 @@ int sgmc_glm_fused_run(const sgmc_glm_run* runs, int nruns) {
                    SGMC_E_ARG, "sgmc_glm_fused_run: a swap launch without pairs");
     }
   }
-  // one launch per table and turn
-  struct Cursor {
-    int op = 0;
-    int64_t at = 0;  // launches of the operation issued so far
-  };
-  std::vector<Cursor> cur(nruns);
-  for (bool any = true; any;) {
-    any = false;
-    for (int k = 0; k < nruns; ++k) {
-      const sgmc_glm_run& r = runs[k];
-      Cursor& c = cur[k];
-      while (c.op < r.nops) {
-        const int count = r.ops[2 * c.op + 1];
-        const int64_t total = r.ops[2 * c.op] == SGMC_OP_ITERATIONS
-                                  ? (int64_t)count * launches_of(r)
-                                  : r.ops[2 * c.op] == SGMC_OP_LOOP ? (count > 0) : count;
-        if (c.at < total) break;
-        ++c.op;
-        c.at = 0;
-      }
-      if (c.op == r.nops) continue;
-      any = true;
-      int rc;
-      switch (r.ops[2 * c.op]) {
-        case SGMC_OP_ITERATIONS: {
-          FusedArgs a = run_args(r);
-          a.step = (int)(c.at % launches_of(r));
-          launch_step(r, a);
-          rc = check_launch("sgmc_glm_fused_run");
-          break;
-        }
-        case SGMC_OP_LOOP: {
-          FusedArgs a = run_args(r);
-          a.blocks_per_chain = 1;
-          a.block_chain = nullptr;
-          a.advance = -1;
-          launch_loop_mode(r, r.ops[2 * c.op + 1], a);
-          rc = check_launch("sgmc_glm_fused_run");
-          break;
-        }
-        default:
-          rc = sgmc_resgld_swap(r.chains, r.nchains, r.pairs, r.npairs, r.F, r.swap_every,
-                                r.save_slot, r.table_len, r.iter, r.stream);
-      }
-      if (rc != SGMC_OK) return rc;
-      ++c.at;
-    }
+  // (the entry points allocate nothing: more tables go in groups of kTogether)
+  for (int k = 0; k < nruns; k += kTogether) {
+    const int rc = issue_runs(runs + k, std::min(kTogether, nruns - k));
+    if (rc != SGMC_OK) return rc;
   }
   return SGMC_OK;
 }
